@@ -35,9 +35,6 @@ int kodama_hip_knn_graph(const float* x, int32_t n, int32_t p, int32_t k, int32_
     require(kk <= (p <= 128 ? kMaxScanK : kMaxK),
             "graph neighbours above 128 (above 64 beyond 128 feature columns) are not supported by the HIP kNN kernel.");
     require(p <= kMaxDims, "the HIP kNN kernel supports 1..256 feature columns.");
-    // Cosine rows are normalised as the reference's exact search expects
-    // (native_knn.cpp:1005-1035).
-    const std::vector<float> xs = prepare_rows(x, n, p, metric, 1);
     select_device(device);
     Stream st(device);
     const hipStream_t s = st.get();
@@ -47,10 +44,13 @@ int kodama_hip_knn_graph(const float* x, int32_t n, int32_t p, int32_t k, int32_
     DeviceBuffer<float> d_dist(static_cast<size_t>(n) * kk);
     std::vector<int> ex(static_cast<size_t>(n));
     std::iota(ex.begin(), ex.end(), 0);
-    d_x.upload(xs.data(), d_x.size(), s);
+    d_x.upload(x, d_x.size(), s);
     d_ex.upload(ex.data(), ex.size(), s);
+    // Cosine rows are normalised as the reference's exact search expects
+    // (native_knn.cpp:1005-1035).
+    if (metric == KODAMA_HIP_COSINE) check(launch_normalize_rows(d_x.get(), n, p, s), "normalize_rows launch");
     device_exact_knn(d_x.get(), n, d_x.get(), n, p, kk, metric, d_ex.get(), d_idx.get(), d_dist.get(),
-                     max_row_norm2(xs.data(), n, p), s, &last_knn_fallbacks());
+                     s, &last_knn_fallbacks());
     check(launch_graph_publish(d_idx.get(), d_dist.get(), d_idx.size(), metric, s), "graph_publish launch");
     d_idx.download(indices_one_based, d_idx.size(), s);
     d_dist.download(distances, d_dist.size(), s);
@@ -136,7 +136,6 @@ int kodama_hip_graph_build(const float* x, int32_t n, int32_t p, int32_t k, int3
     require(kk <= (p <= 128 ? kMaxScanK : kMaxK),
             "graph neighbours above 128 (above 64 beyond 128 feature columns) are not supported by the HIP kNN kernel.");
     require(p <= kMaxDims, "the HIP kNN kernel supports 1..256 feature columns.");
-    const std::vector<float> xs = prepare_rows(x, n, p, metric, 1);
     select_device(device);
     std::unique_ptr<kodama_hip_graph> g(new kodama_hip_graph);
     g->device = device;
@@ -150,10 +149,13 @@ int kodama_hip_graph_build(const float* x, int32_t n, int32_t p, int32_t k, int3
     DeviceBuffer<int> d_ex(static_cast<size_t>(n));
     std::vector<int> ex(static_cast<size_t>(n));
     std::iota(ex.begin(), ex.end(), 0);
-    d_x.upload(xs.data(), d_x.size(), s);
+    d_x.upload(x, d_x.size(), s);
     d_ex.upload(ex.data(), ex.size(), s);
+    // Cosine rows are normalised as the reference's exact search expects
+    // (native_knn.cpp:1005-1035).
+    if (metric == KODAMA_HIP_COSINE) check(launch_normalize_rows(d_x.get(), n, p, s), "normalize_rows launch");
     device_exact_knn(d_x.get(), n, d_x.get(), n, p, kk, metric, d_ex.get(), g->idx.get(), g->dist.get(),
-                     max_row_norm2(xs.data(), n, p), s, &last_knn_fallbacks());
+                     s, &last_knn_fallbacks());
     check(launch_graph_publish(g->idx.get(), g->dist.get(), g->idx.size(), metric, s), "graph_publish launch");
     st.sync();
     *out = g.release();

@@ -192,8 +192,8 @@ int kodama_hip_exact_knn_search(const float* train, int32_t train_rows, const fl
     d_query.upload(query, d_query.size(), s);
     if (query_train_indices) d_ex.upload(query_train_indices, d_ex.size(), s);
     device_exact_knn(d_train.get(), train_rows, d_query.get(), query_rows, dimensions, k, metric,
-                     query_train_indices ? d_ex.get() : nullptr, d_idx.get(), d_dist.get(),
-                     max_row_norm2(train, train_rows, dimensions), s, &last_knn_fallbacks());
+                     query_train_indices ? d_ex.get() : nullptr, d_idx.get(), d_dist.get(), s,
+                     &last_knn_fallbacks());
     d_idx.download(out_indices, d_idx.size(), s);
     d_dist.download(out_distances, d_dist.size(), s);
     st.sync();

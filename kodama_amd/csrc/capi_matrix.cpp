@@ -236,15 +236,19 @@ void matrix_impl(const float* x, int32_t n, int32_t p, const kodama_hip_matrix_o
   } else if (build_graph) {
     d_gidx.resize(edges);
     d_gdist.resize(edges);
-    const std::vector<float> xs = prepare_rows(x, n, p, o.metric, 1);
-    DeviceBuffer<float> d_xs(xs.size());
+    DeviceBuffer<float> d_norm;  // cosine: the rows as native_knn.cpp:1005-1035 prepares them
     DeviceBuffer<int> d_self(static_cast<size_t>(n));
     IVec self(static_cast<size_t>(n));
     std::iota(self.begin(), self.end(), 0);
-    d_xs.upload(xs.data(), xs.size(), s);
+    if (o.metric == KODAMA_HIP_COSINE) {
+      d_norm.resize(d_x.size());
+      check(hipMemcpyAsync(d_norm.get(), d_x.get(), d_x.size() * sizeof(float), hipMemcpyDeviceToDevice, s), "copy");
+      check(launch_normalize_rows(d_norm.get(), n, p, s), "normalize_rows launch");
+    }
+    const float* d_xs = o.metric == KODAMA_HIP_COSINE ? d_norm.get() : d_x.get();
     d_self.upload(self.data(), self.size(), s);
-    device_exact_knn(d_xs.get(), n, d_xs.get(), n, p, z.neighbors, o.metric, d_self.get(), d_gidx.get(),
-                     d_gdist.get(), max_row_norm2(xs.data(), n, p), s, &last_knn_fallbacks());
+    device_exact_knn(d_xs, n, d_xs, n, p, z.neighbors, o.metric, d_self.get(), d_gidx.get(), d_gdist.get(), s,
+                     &last_knn_fallbacks());
   }
   check(hipStreamSynchronize(s), "graph sync");
   t[1] = seconds_since(clock);

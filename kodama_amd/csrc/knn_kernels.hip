@@ -24,6 +24,7 @@
 #include <climits>
 #include <cstdint>
 
+#include "knn_mfma.h"
 #include "launch.h"
 
 namespace kodama_hip {
@@ -497,7 +498,26 @@ __global__ void __launch_bounds__(kBlock) knn_merge_slices_kernel(const int* __r
   }
 }
 
+// One thread per row: the float sum of squares in column order, without
+// contraction, so the scale is the host's bit for bit.
+__global__ void normalize_rows_kernel(float* __restrict__ x, int rows, int p) {
+#pragma clang fp contract(off)
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= rows) return;
+  float* row = x + static_cast<size_t>(r) * p;
+  float ss = 0.0f;
+  for (int j = 0; j < p; ++j) ss += row[j] * row[j];
+  const float scale = ss > 0.0f && isfinite(ss) ? 1.0f / sqrtf(ss) : 1.0f;
+  for (int j = 0; j < p; ++j) row[j] *= scale;
+}
+
 // ---- host launchers --------------------------------------------------------
+
+hipError_t launch_normalize_rows(float* x, int rows, int p, hipStream_t s) {
+  if (rows == 0) return hipSuccess;
+  hipLaunchKernelGGL(normalize_rows_kernel, dim3((rows + 63) / 64), dim3(64), 0, s, x, rows, p);
+  return hipGetLastError();
+}
 
 // MODES = 1: query vs train only; 2: both modes.
 template <int PMAX, int KMAX, int MODES = 2>

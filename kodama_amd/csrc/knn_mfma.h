@@ -11,7 +11,6 @@ namespace kodama_hip {
 constexpr int kMfmaMaxK = 128;        // k served by the MFMA path
 // Candidates kept per (query, lane column): 16 x this per query.
 inline int mfma_list_len(int k) { return k <= 32 ? 8 : 16; }
-constexpr int kMfmaMinTrain = 4096;   // smaller train sets use the register scan
 constexpr float kMfmaErrorScale = 8e-5f;  // E = scale * (|q|^2 + max |t|^2)
 
 struct KnnMfmaParams {
@@ -68,7 +67,6 @@ inline int mfma_list(const KnnMfmaParams& p) { return p.list != 0 ? p.list : mfm
 
 hipError_t launch_split_rows(const float* x, int rows, int p, unsigned short* hi, unsigned short* lo, float* norm2,
                              hipStream_t s);
-hipError_t launch_knn_mfma(const KnnMfmaParams& prm, bool euclid, hipStream_t s);
 hipError_t launch_knn_mfma_tables(const KnnMfmaParams& prm, bool euclid, int runs, int max_rows, hipStream_t s);
 hipError_t launch_publish_tables(const int* idx, const float* dist, const int* flags, const int* run_offsets,
                                  int runs, const int* pad_offsets, int pad_total, int rows, int k, int* out_index,
@@ -83,15 +81,17 @@ hipError_t launch_scatter_results(const int* src_idx, const float* src_dist, con
 
 // Exact kNN of device-resident rows (internal distances, (distance, index)
 // order, -1 / +inf beyond the available rows), bit-identical to the register
-// scan: the MFMA path when dims <= 64, k <= 128 and train_rows >= 4096,
-// otherwise the register scan. Queries the 8-entry lists (k <= 32) cannot
-// certify take, when there are 4096 or more, a second MFMA pass with 16-entry
-// lists; the rest (those it flags again, fewer, or of 16-entry lists) take
-// the register scan. `train_norm2_max`
-// bounds the squared norms of the train rows (prepared rows for cosine).
+// scan: FP16 matrix-core candidates with the exact rerank (knn_stream.h) when
+// k <= 128 and train_rows >= 4096 (beyond 64 dimensions also query_rows >=
+// 1024), otherwise the register scan. Queries the first pass cannot certify
+// take a second one with three operand parts and 256 candidates, and what that
+// leaves the scan; *mfma_fallbacks counts those (-1: the scan ran alone).
 void device_exact_knn(const float* d_train, int train_rows, const float* d_query, int query_rows, int dims, int k,
-                      int metric, const int* d_exclude, int* d_idx, float* d_dist, float train_norm2_max,
-                      hipStream_t s, int* mfma_fallbacks = nullptr);
+                      int metric, const int* d_exclude, int* d_idx, float* d_dist, hipStream_t s,
+                      int* mfma_fallbacks = nullptr);
+// Cosine rows as native_knn.cpp:1005-1035 prepares them (prepare_rows, variant
+// 1): the row times 1 / sqrt of its float sum of squares in column order.
+hipError_t launch_normalize_rows(float* x, int rows, int p, hipStream_t s);
 
 // Per-fold kNN tables of a batch of runs (precompute_knn_cv_cuda,
 // core.cpp:694-782, for all runs at once) into the transposed padded vote

@@ -622,21 +622,16 @@ hipError_t launch_split_rows(const float* x, int rows, int p, unsigned short* hi
 }
 
 template <int LIST, int WAVES, int PACK>
-static void launch_mfma_schedule(const KnnMfmaParams& prm, bool euclid, bool tables, dim3 grid, hipStream_t s) {
+static void launch_mfma_schedule(const KnnMfmaParams& prm, bool euclid, dim3 grid, hipStream_t s) {
   const dim3 block(WAVES * 64);
-  if (tables) {
-    if (euclid) hipLaunchKernelGGL((knn_mfma_candidates_kernel<true, true, LIST, WAVES, PACK>), grid, block, 0, s, prm);
-    else hipLaunchKernelGGL((knn_mfma_candidates_kernel<false, true, LIST, WAVES, PACK>), grid, block, 0, s, prm);
-  } else {
-    if (euclid) hipLaunchKernelGGL((knn_mfma_candidates_kernel<true, false, LIST, WAVES, PACK>), grid, block, 0, s, prm);
-    else hipLaunchKernelGGL((knn_mfma_candidates_kernel<false, false, LIST, WAVES, PACK>), grid, block, 0, s, prm);
-  }
+  if (euclid) hipLaunchKernelGGL((knn_mfma_candidates_kernel<true, true, LIST, WAVES, PACK>), grid, block, 0, s, prm);
+  else hipLaunchKernelGGL((knn_mfma_candidates_kernel<false, true, LIST, WAVES, PACK>), grid, block, 0, s, prm);
 }
 
 template <int LIST, int PACK>
-static void launch_mfma_packing(const KnnMfmaParams& prm, bool euclid, bool tables, dim3 grid, hipStream_t s) {
-  if (prm.waves == 4) launch_mfma_schedule<LIST, 4, PACK>(prm, euclid, tables, grid, s);
-  else launch_mfma_schedule<LIST, 8, PACK>(prm, euclid, tables, grid, s);
+static void launch_mfma_packing(const KnnMfmaParams& prm, bool euclid, dim3 grid, hipStream_t s) {
+  if (prm.waves == 4) launch_mfma_schedule<LIST, 4, PACK>(prm, euclid, grid, s);
+  else launch_mfma_schedule<LIST, 8, PACK>(prm, euclid, grid, s);
   const unsigned rblocks = static_cast<unsigned>((prm.query_rows + 3) / 4);
   if (euclid) hipLaunchKernelGGL((knn_rerank_kernel<true, LIST, PACK == 1>), dim3(rblocks), dim3(256), 0, s, prm);
   else hipLaunchKernelGGL((knn_rerank_kernel<false, LIST, PACK == 1>), dim3(rblocks), dim3(256), 0, s, prm);
@@ -652,44 +647,34 @@ int mfma_packed_lists() { return g_packed_lists.load(); }
 // past that, 8-entry lists are packed per segment of kMfmaSegmentBits index
 // bits (16 << kMfmaSegmentBits rows) and merged into (value, row) pairs.
 template <int LIST>
-static void launch_mfma_list(KnnMfmaParams prm, bool euclid, bool tables, int rows, int train_rows, hipStream_t s,
+static void launch_mfma_list(KnnMfmaParams prm, bool euclid, int rows, int train_rows, hipStream_t s,
                              unsigned runs) {
   const int qpb = prm.waves * 16;
   const dim3 grid(static_cast<unsigned>((rows + qpb - 1) / qpb), runs);
   const unsigned top = static_cast<unsigned>((train_rows + 15) / 16 - 1);  // largest column index
   int bits = 0;
   while (bits < 32 && (top >> bits) != 0u) ++bits;
-  prm.runs = tables ? static_cast<int>(runs) : 0;
+  prm.runs = static_cast<int>(runs);
   const bool packed = g_packed_lists.load() != 0;
   if (packed && bits <= kMfmaMaxIndexBits) {
     prm.index_bits = bits;
-    launch_mfma_packing<LIST, 1>(prm, euclid, tables, grid, s);
+    launch_mfma_packing<LIST, 1>(prm, euclid, grid, s);
     return;
   }
   if constexpr (LIST == 8) {
     if (packed) {
       prm.index_bits = kMfmaSegmentBits;
-      launch_mfma_packing<LIST, 2>(prm, euclid, tables, grid, s);
+      launch_mfma_packing<LIST, 2>(prm, euclid, grid, s);
       return;
     }
   }
   prm.index_bits = -1;
-  launch_mfma_packing<LIST, 0>(prm, euclid, tables, grid, s);
+  launch_mfma_packing<LIST, 0>(prm, euclid, grid, s);
 }
 
 static bool schedule_ok(const KnnMfmaParams& prm) {
   const int list = mfma_list(prm);
   return (prm.waves == 4 || prm.waves == 8) && (list == 16 || (list == 8 && prm.k <= 32));
-}
-
-hipError_t launch_knn_mfma(const KnnMfmaParams& prm, bool euclid, hipStream_t s) {
-  if (prm.query_rows == 0) return hipSuccess;
-  if (prm.dims < 1 || prm.dims > 64 || prm.k < 1 || prm.k > kMfmaMaxK || prm.train_rows < 1 || !schedule_ok(prm)) {
-    return hipErrorInvalidValue;
-  }
-  if (mfma_list(prm) == 8) launch_mfma_list<8>(prm, euclid, false, prm.query_rows, prm.train_rows, s, 1);
-  else launch_mfma_list<16>(prm, euclid, false, prm.query_rows, prm.train_rows, s, 1);
-  return hipGetLastError();
 }
 
 hipError_t launch_knn_mfma_tables(const KnnMfmaParams& prm, bool euclid, int runs, int max_rows, hipStream_t s) {
@@ -698,8 +683,8 @@ hipError_t launch_knn_mfma_tables(const KnnMfmaParams& prm, bool euclid, int run
       prm.folds == nullptr || prm.query_rows != prm.train_rows || max_rows < 1 || !schedule_ok(prm)) {
     return hipErrorInvalidValue;
   }
-  if (mfma_list(prm) == 8) launch_mfma_list<8>(prm, euclid, true, max_rows, max_rows, s, static_cast<unsigned>(runs));
-  else launch_mfma_list<16>(prm, euclid, true, max_rows, max_rows, s, static_cast<unsigned>(runs));
+  if (mfma_list(prm) == 8) launch_mfma_list<8>(prm, euclid, max_rows, max_rows, s, static_cast<unsigned>(runs));
+  else launch_mfma_list<16>(prm, euclid, max_rows, max_rows, s, static_cast<unsigned>(runs));
   return hipGetLastError();
 }
 

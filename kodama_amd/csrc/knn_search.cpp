@@ -1,6 +1,7 @@
-// Host driver of the exact kNN on the device: the split-BF16 MFMA candidates
-// with the exact rerank where they apply, the register scan otherwise and for
-// the queries the rerank flags.
+// Host driver of the exact kNN on the device: matrix-core candidates with the
+// exact rerank where they apply (FP16 stream for searches, split BF16 for the
+// per-fold tables), the register scan otherwise and for the queries the
+// rerank flags.
 #include <algorithm>
 #include <atomic>
 #include <chrono>
@@ -13,6 +14,7 @@
 #include "../../include/kodama_hip.h"
 #include "device.h"
 #include "knn_mfma.h"
+#include "knn_stream.h"
 #include "launch.h"
 
 namespace kodama_hip {
@@ -24,13 +26,16 @@ constexpr int kScanTargetBlocks = 512;   // two blocks per CU
 constexpr int kMaxSlices = 64;           // lists one merge wave combines
 constexpr int kSliceAlign = 64;          // LDS tile rows of the scan
 constexpr int kTableTargetBlocks = 2048; // sliced rescans of flagged table rows
-constexpr int kMfmaSecondPassMin = 4096; // flagged queries for a 16-entry MFMA pass before the scan
+constexpr int kStreamMinTrain = 4096;     // smaller train sets use the register scan
+constexpr int kStreamWideQueries = 1024;  // queries beyond 64 dimensions for the matrix cores
+constexpr int kStreamTargetBlocks = 2048; // eight workgroups per CU
+constexpr int kStreamSliceRows = 1024;    // train rows per slice at least
+constexpr size_t kStreamCandBytes = size_t(1) << 30;  // candidate buffers per launch
 
 }  // namespace
 
 void device_exact_knn(const float* d_train, int train_rows, const float* d_query, int query_rows, int dims, int k,
-                      int metric, const int* d_exclude, int* d_idx, float* d_dist, float train_norm2_max,
-                      hipStream_t s, int* mfma_fallbacks) {
+                      int metric, const int* d_exclude, int* d_idx, float* d_dist, hipStream_t s, int* mfma_fallbacks) {
   const bool euclid = metric == KODAMA_HIP_EUCLIDEAN;
   if (mfma_fallbacks) *mfma_fallbacks = -1;  // -1: the MFMA path was not used
   // Register scan. Few queries (one block per 256) would leave most CUs idle,
@@ -66,127 +71,144 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
           "knn_merge_slices launch");
     check(hipStreamSynchronize(s), "knn scan sync");  // the partial lists are freed on return
   };
-  if (dims > 64 || k > kMfmaMaxK || train_rows < kMfmaMinTrain || query_rows == 0) {
+  const int narrow = stream_steps(dims, 1, euclid);
+  if (k > kStreamMaxK || train_rows < kStreamMinTrain || query_rows == 0 || narrow > kStreamMaxSteps ||
+      (dims > 64 && query_rows < kStreamWideQueries)) {
     scan(d_query, query_rows, d_exclude, d_idx, d_dist);
     return;
   }
+  // Matrix-core candidates in one FP16 part (three where that is as wide) and
+  // the buffer the width of k needs; the queries it cannot certify take three
+  // parts and the larger buffer, and only what is left the scan.
   const bool same = d_query == d_train;
-  DeviceBuffer<unsigned short> t_hi(static_cast<size_t>(train_rows) * 64), t_lo(t_hi.size());
-  DeviceBuffer<float> t_n2(static_cast<size_t>(train_rows));
-  check(launch_split_rows(d_train, train_rows, dims, t_hi.get(), t_lo.get(), t_n2.get(), s), "split_rows launch");
-  DeviceBuffer<unsigned short> q_hi, q_lo;
-  DeviceBuffer<float> q_n2;
-  if (!same) {
-    q_hi.resize(static_cast<size_t>(query_rows) * 64);
-    q_lo.resize(q_hi.size());
-    q_n2.resize(static_cast<size_t>(query_rows));
-    check(launch_split_rows(d_query, query_rows, dims, q_hi.get(), q_lo.get(), q_n2.get(), s), "split_rows launch");
-  }
-  const size_t cand = static_cast<size_t>(query_rows) * 16 * mfma_list_len(k);
-  DeviceBuffer<float> c_val(cand);
-  DeviceBuffer<int> c_idx(cand), flags(static_cast<size_t>(query_rows));
-  KnnMfmaParams m;
-  m.train = d_train;
-  m.query = d_query;
-  m.train_hi = t_hi.get();
-  m.train_lo = t_lo.get();
-  m.query_hi = same ? t_hi.get() : q_hi.get();
-  m.query_lo = same ? t_lo.get() : q_lo.get();
-  m.train_norm2 = t_n2.get();
-  m.query_norm2 = same ? t_n2.get() : q_n2.get();
-  m.train_norm2_max = train_norm2_max;
-  m.train_rows = train_rows;
-  m.query_rows = query_rows;
-  m.dims = dims;
-  m.k = k;
-  m.exclude = d_exclude;
-  m.cand_value = c_val.get();
-  m.cand_index = c_idx.get();
-  m.flags = flags.get();
-  m.out_index = d_idx;
-  m.out_dist = d_dist;
-  m.waves = 4;  // two 4-wave blocks per CU overlap each other's staging barriers
-  check(launch_knn_mfma(m, euclid, s), "knn_mfma launch");
-  std::vector<int> h_flags(static_cast<size_t>(query_rows));
-  flags.download(h_flags.data(), h_flags.size(), s);
-  check(hipStreamSynchronize(s), "knn_mfma sync");
-  std::vector<int> redo;
-  for (int q = 0; q < query_rows; ++q) if (h_flags[q]) redo.push_back(q);
+  DeviceBuffer<float> t_n2(static_cast<size_t>(train_rows)), n2_max(2);
+  check(hipMemsetAsync(n2_max.get(), 0, 2 * sizeof(float), s), "memset");
+  check(launch_stream_norms(d_train, train_rows, dims, t_n2.get(), n2_max.get(), s), "stream_norms launch");
+  // One pass over `rows` queries; returns the flagged ones.
+  auto pass = [&](const float* q, int rows, const int* ex, int parts, int list, bool self, int* idx, float* dist) {
+    const int steps = stream_steps(dims, parts, euclid);
+    const int t_pad = (train_rows + kStreamBlockRows - 1) / kStreamBlockRows * kStreamBlockRows;
+    const int q_pad = (rows + kStreamBlockRows - 1) / kStreamBlockRows * kStreamBlockRows;
+    DeviceBuffer<unsigned char> t_op(stream_operand_bytes(static_cast<size_t>(t_pad), steps)),
+      q_op(stream_operand_bytes(static_cast<size_t>(q_pad), steps));
+    DeviceBuffer<float> q_n2;
+    if (!self) {
+      q_n2.resize(static_cast<size_t>(rows));
+      check(launch_stream_norms(q, rows, dims, q_n2.get(), n2_max.get() + 1, s), "stream_norms launch");
+    }
+    StreamOperandJob op;
+    op.x = d_train;
+    op.norm2 = t_n2.get();
+    op.norm2_max = n2_max.get();
+    op.rows = train_rows;
+    op.p = dims;
+    op.parts = parts;
+    op.euclid = euclid ? 1 : 0;
+    op.pad_rows = t_pad;
+    op.train_op = t_op.get();
+    op.query_op = self ? q_op.get() : nullptr;
+    check(launch_stream_operands(op, s), "stream_operands launch");
+    if (!self) {
+      op.x = q;
+      op.norm2 = q_n2.get();
+      op.rows = rows;
+      op.pad_rows = q_pad;
+      op.train_op = nullptr;
+      op.query_op = q_op.get();
+      check(launch_stream_operands(op, s), "stream_operands launch");
+    }
+    // Slices: about eight workgroups per CU in all, each scanning at least
+    // kStreamSliceRows rows, the candidate buffers within kStreamCandBytes.
+    const int per_block = 4 * stream_queries_per_wave(steps);
+    const int blocks = (rows + per_block - 1) / per_block;
+    const int most = std::min(kStreamMaxSlices, std::max(1, train_rows / kStreamSliceRows));
+    const int cap = stream_capacity(list);
+    const size_t row_bytes = static_cast<size_t>(cap) * sizeof(uint2);
+    int slices = std::min(most, (kStreamTargetBlocks + blocks - 1) / blocks);
+    slices = std::max(1, std::min(slices, static_cast<int>(kStreamCandBytes / (row_bytes * q_pad))));
+    const int max_slices =
+      std::min(kStreamMaxSlices, std::max(stream_min_max_slices(k), std::min(most, (kStreamTargetBlocks + blocks - 1) / blocks)));
+    // The maxima are read before the candidates are written: one buffer.
+    const size_t query_bytes = std::max(row_bytes * slices, static_cast<size_t>(max_slices) * 32 * sizeof(float));
+    const size_t fit = kStreamCandBytes / query_bytes;
+    const int batch = std::min(q_pad, static_cast<int>(std::max<size_t>(1, fit / kStreamBlockRows) * kStreamBlockRows));
+    DeviceBuffer<unsigned char> cand(static_cast<size_t>(batch) * query_bytes);
+    DeviceBuffer<float> threshold(static_cast<size_t>(batch));
+    DeviceBuffer<int> count(static_cast<size_t>(batch) * slices), flags(static_cast<size_t>(rows));
+    DeviceBuffer<float> bound(count.size());
+    KnnStreamParams m;
+    m.train = d_train;
+    m.train_op = t_op.get();
+    m.norm2_max = n2_max.get();
+    m.train_rows = train_rows;
+    m.dims = dims;
+    m.k = k;
+    m.parts = parts;
+    m.euclid = euclid ? 1 : 0;
+    m.slices = slices;
+    m.list = list;
+    m.sample_chunks = stream_sample_chunks(k);
+    m.max_slices = max_slices;
+    m.maxima = reinterpret_cast<float*>(cand.get());
+    m.threshold = threshold.get();
+    m.cand = reinterpret_cast<uint2*>(cand.get());
+    m.cand_count = count.get();
+    m.cand_bound = bound.get();
+    for (int q0 = 0; q0 < rows; q0 += batch) {
+      m.query = q + static_cast<size_t>(q0) * dims;
+      m.query_op = q_op.get() + stream_operand_bytes(static_cast<size_t>(q0), steps);
+      m.query_norm2 = (self ? t_n2.get() : q_n2.get()) + q0;
+      m.query_rows = std::min(batch, rows - q0);
+      m.exclude = ex ? ex + q0 : nullptr;
+      m.flags = flags.get() + q0;
+      m.out_index = idx + static_cast<size_t>(q0) * k;
+      m.out_dist = dist + static_cast<size_t>(q0) * k;
+      check(launch_knn_stream(m, s), "knn_stream launch");
+    }
+    std::vector<int> h_flags(static_cast<size_t>(rows)), redo;
+    flags.download(h_flags.data(), h_flags.size(), s);
+    check(hipStreamSynchronize(s), "knn_stream sync");
+    for (int i = 0; i < rows; ++i) if (h_flags[i]) redo.push_back(i);
+    return redo;
+  };
+  const int parts = stream_steps(dims, 3, euclid) == narrow ? 3 : 1;
+  const int list = k <= 32 ? 8 : 16;
+  const std::vector<int> redo = pass(d_query, query_rows, d_exclude, parts, list, same, d_idx, d_dist);
   if (mfma_fallbacks) *mfma_fallbacks = static_cast<int>(redo.size());
   if (redo.empty()) return;
-  const int nr = static_cast<int>(redo.size());
-  DeviceBuffer<int> d_rows(static_cast<size_t>(nr));
-  d_rows.upload(redo.data(), redo.size(), s);
-  DeviceBuffer<float> q_sub(static_cast<size_t>(nr) * dims), r_dist(static_cast<size_t>(nr) * k);
-  DeviceBuffer<int> r_idx(static_cast<size_t>(nr) * k), ex_sub;
-  check(launch_gather_rows(d_query, d_rows.get(), nr, dims, q_sub.get(), s), "gather_rows launch");
-  if (d_exclude) {
-    std::vector<int> h_ex(static_cast<size_t>(query_rows)), sub(redo.size());
-    // Exclusions of the flagged queries (host copy: the list is short).
-    check(hipMemcpyAsync(h_ex.data(), d_exclude, h_ex.size() * sizeof(int), hipMemcpyDeviceToHost, s), "download");
-    check(hipStreamSynchronize(s), "exclusion sync");
-    for (int i = 0; i < nr; ++i) sub[i] = h_ex[redo[i]];
-    ex_sub.resize(sub.size());
-    ex_sub.upload(sub.data(), sub.size(), s);
-  }
-  const int* d_ex_sub = d_exclude ? ex_sub.get() : nullptr;
-  if (mfma_list(m) == 8 && nr >= kMfmaSecondPassMin) {
-    // Second pass over the flagged queries with 16 candidates per lane column
-    // (most certify there); only queries flagged again take the scan. Its
-    // workgroups stream every train row, so it pays once the flagged queries
-    // would keep the sliced scan busy for longer.
-    DeviceBuffer<unsigned short> s_hi(static_cast<size_t>(nr) * 64), s_lo(s_hi.size());
-    DeviceBuffer<float> s_n2(static_cast<size_t>(nr));
-    check(launch_split_rows(q_sub.get(), nr, dims, s_hi.get(), s_lo.get(), s_n2.get(), s), "split_rows launch");
-    const size_t cand2 = static_cast<size_t>(nr) * 16 * 16;
-    DeviceBuffer<float> c2_val(cand2);
-    DeviceBuffer<int> c2_idx(cand2), flags2(static_cast<size_t>(nr));
-    KnnMfmaParams m2 = m;
-    m2.query = q_sub.get();
-    m2.query_hi = s_hi.get();
-    m2.query_lo = s_lo.get();
-    m2.query_norm2 = s_n2.get();
-    m2.query_rows = nr;
-    m2.exclude = d_ex_sub;
-    m2.cand_value = c2_val.get();
-    m2.cand_index = c2_idx.get();
-    m2.flags = flags2.get();
-    m2.out_index = r_idx.get();
-    m2.out_dist = r_dist.get();
-    m2.list = 16;
-    check(launch_knn_mfma(m2, euclid, s), "knn_mfma launch");
-    std::vector<int> h_flags2(static_cast<size_t>(nr));
-    flags2.download(h_flags2.data(), h_flags2.size(), s);
-    check(hipStreamSynchronize(s), "knn_mfma sync");
-    std::vector<int> redo2;
-    for (int i = 0; i < nr; ++i) if (h_flags2[i]) redo2.push_back(i);
-    if (mfma_fallbacks) *mfma_fallbacks = static_cast<int>(redo2.size());
-    if (!redo2.empty()) {
-      const int n2 = static_cast<int>(redo2.size());
-      DeviceBuffer<int> d_rows2(static_cast<size_t>(n2));
-      d_rows2.upload(redo2.data(), redo2.size(), s);
-      DeviceBuffer<float> q_sub2(static_cast<size_t>(n2) * dims), r2_dist(static_cast<size_t>(n2) * k);
-      DeviceBuffer<int> r2_idx(static_cast<size_t>(n2) * k), ex_sub2;
-      check(launch_gather_rows(q_sub.get(), d_rows2.get(), n2, dims, q_sub2.get(), s), "gather_rows launch");
-      if (d_exclude) {
-        std::vector<int> h_ex(static_cast<size_t>(query_rows)), sub2(redo2.size());
-        check(hipMemcpyAsync(h_ex.data(), d_exclude, h_ex.size() * sizeof(int), hipMemcpyDeviceToHost, s),
-              "download");
-        check(hipStreamSynchronize(s), "exclusion sync");
-        for (int i = 0; i < n2; ++i) sub2[i] = h_ex[redo[redo2[i]]];
-        ex_sub2.resize(sub2.size());
-        ex_sub2.upload(sub2.data(), sub2.size(), s);
-      }
-      scan(q_sub2.get(), n2, d_exclude ? ex_sub2.get() : nullptr, r2_idx.get(), r2_dist.get());
-      check(launch_scatter_results(r2_idx.get(), r2_dist.get(), d_rows2.get(), n2, k, r_idx.get(), r_dist.get(), s),
-            "scatter_results launch");
+  // Gathers the listed rows of a query set and runs `find` on them.
+  auto on_rows = [&](const std::vector<int>& list_rows, const float* q, int all, const int* ex, int* idx, float* dist,
+                     const std::function<void(const float*, int, const int*, int*, float*)>& find) {
+    const int nr = static_cast<int>(list_rows.size());
+    DeviceBuffer<int> d_rows(static_cast<size_t>(nr)), r_idx(static_cast<size_t>(nr) * k), ex_sub;
+    DeviceBuffer<float> q_sub(static_cast<size_t>(nr) * dims), r_dist(static_cast<size_t>(nr) * k);
+    std::vector<int> sub;
+    d_rows.upload(list_rows.data(), list_rows.size(), s);
+    check(launch_gather_rows(q, d_rows.get(), nr, dims, q_sub.get(), s), "gather_rows launch");
+    if (ex) {
+      std::vector<int> h_ex(static_cast<size_t>(all));
+      check(hipMemcpyAsync(h_ex.data(), ex, h_ex.size() * sizeof(int), hipMemcpyDeviceToHost, s), "download");
+      check(hipStreamSynchronize(s), "exclusion sync");
+      for (int i : list_rows) sub.push_back(h_ex[i]);
+      ex_sub.resize(sub.size());
+      ex_sub.upload(sub.data(), sub.size(), s);
     }
-  } else {
-    scan(q_sub.get(), nr, d_ex_sub, r_idx.get(), r_dist.get());
-  }
-  check(launch_scatter_results(r_idx.get(), r_dist.get(), d_rows.get(), nr, k, d_idx, d_dist, s),
-        "scatter_results launch");
-  check(hipStreamSynchronize(s), "fallback sync");
+    find(q_sub.get(), nr, ex ? ex_sub.get() : nullptr, r_idx.get(), r_dist.get());
+    check(launch_scatter_results(r_idx.get(), r_dist.get(), d_rows.get(), nr, k, idx, dist, s),
+          "scatter_results launch");
+    check(hipStreamSynchronize(s), "fallback sync");
+  };
+  const int wide = stream_steps(dims, 3, euclid) <= kStreamMaxSteps ? 3 : 1;
+  on_rows(redo, d_query, query_rows, d_exclude, d_idx, d_dist,
+          [&](const float* q, int rows, const int* ex, int* idx, float* dist) {
+            if (wide == parts && list == 16) {
+              scan(q, rows, ex, idx, dist);
+              return;
+            }
+            const std::vector<int> redo2 = pass(q, rows, ex, wide, 16, false, idx, dist);
+            if (mfma_fallbacks) *mfma_fallbacks = static_cast<int>(redo2.size());
+            if (!redo2.empty()) on_rows(redo2, q, rows, ex, idx, dist, scan);
+          });
 }
 
 namespace {

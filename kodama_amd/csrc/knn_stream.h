@@ -1,0 +1,92 @@
+// Exact kNN through FP16 matrix-core candidates with a running threshold
+// (knn_stream.hip): parameter blocks and launchers.
+#pragma once
+
+#include <hip/hip_runtime_api.h>
+
+#include <cstddef>
+
+namespace kodama_hip {
+
+constexpr int kStreamMaxSteps = 9;     // 32-deep MFMA steps per pair (operand width / 32)
+constexpr int kStreamMaxK = 128;       // neighbours served
+constexpr int kStreamBlockRows = 256;  // operand rows are padded to this multiple per set or run
+constexpr int kStreamMerge = 1024;     // candidates the rerank holds per query (all slices)
+constexpr int kStreamMaxSlices = 16;
+
+// Operand width of one pair: `parts` 1 (FP16 of the rows) or 3 (high and low
+// FP16 parts, hi.hi + hi.lo + lo.hi) of p columns and, for Euclidean
+// distances, the FP16 parts of -|t|^2 / 2.
+inline int stream_width(int p, int parts, bool euclid) { return parts * p + (euclid ? (parts == 1 ? 2 : 3) : 0); }
+inline int stream_steps(int p, int parts, bool euclid) { return (stream_width(p, parts, euclid) + 31) / 32; }
+// Candidates kept per query and slice (list 8, k <= 32: 128; list 16: 256).
+inline int stream_capacity(int list) { return 16 * list; }
+// Queries per wave of the candidates: four 16-query tiles, two where the
+// operands are wide.
+inline int stream_queries_per_wave(int steps) { return steps <= 4 ? 64 : 32; }
+// Slices of the maxima at least: 2.1 k class maxima place the k-th largest of
+// them at about the 1.4 k-th largest score.
+inline int stream_min_max_slices(int k) { return (21 * k / 10 + 31) / 32; }
+// Sampled chunks for the threshold, about 1000 k rows: scoring a row twice
+// costs as much as 1 / (1000 k) of an append per query, so past this many the
+// appends that a longer sample saves no longer pay for it.
+inline int stream_sample_chunks(int k) { return 16 * k; }
+
+struct KnnStreamParams {
+  const float* train = nullptr;     // [train rows x dims], for the exact re-score
+  const float* query = nullptr;
+  const void* train_op = nullptr;   // operand fragments (launch_stream_operands)
+  const void* query_op = nullptr;
+  const float* query_norm2 = nullptr;  // [query rows]
+  const float* norm2_max = nullptr;    // [2] largest squared norm of the train rows, of the queries
+  int train_rows = 0, query_rows = 0, dims = 0, k = 0;
+  int parts = 1, euclid = 0;
+  const int* exclude = nullptr;     // [query rows] train row to skip, may be null
+  // Per-fold tables of a batch of runs: operands in the padded layout (each
+  // run's rows start at a multiple of 256), results and rows concatenated.
+  const int* block_run = nullptr;   // run of each 256 padded rows
+  const int* run_offsets = nullptr;
+  const int* pad_offsets = nullptr;
+  const int* folds = nullptr;       // [rows], concatenated
+  int pad_rows = 0;
+  // Class maxima: sampled 64-row chunks (all rows when at least as many),
+  // dealt to max_slices workgroups per query block; 32 values per query and slice.
+  int sample_chunks = 1, max_slices = 1;
+  float* maxima = nullptr;          // [query rows (padded for tables)][max_slices][32]; may share cand
+  float* threshold = nullptr;       // [query rows]
+  int slices = 1;                   // the candidates' train rows are cut into this many ranges
+  int list = 8;                     // capacity / 16
+  uint2* cand = nullptr;            // [query rows (padded for tables)][slices][capacity] (score bits, row)
+  int* cand_count = nullptr;        // [query rows][slices], -1 = overflowed
+  float* cand_bound = nullptr;      // [query rows][slices] scores below it were dropped
+  int* flags = nullptr;             // [query rows] 1 = needs another path
+  int* out_index = nullptr;         // [query rows x k]
+  float* out_dist = nullptr;
+};
+
+// Squared norms [rows] and their maximum (into *norm2_max, which the caller
+// cleared to 0).
+hipError_t launch_stream_norms(const float* x, int rows, int p, float* norm2, float* norm2_max, hipStream_t s);
+// Rows -> operand fragments of `steps` x 32 columns, rows padded with zeros to
+// a multiple of 256; either output may be null. norm2_max [2] scales them.
+// For the padded table layout pass block_run / run_offsets / pad_offsets.
+struct StreamOperandJob {
+  const float* x = nullptr;
+  const float* norm2 = nullptr;
+  const float* norm2_max = nullptr;
+  int rows = 0, p = 0, parts = 1, euclid = 0;
+  int pad_rows = 0;                 // multiple of 256
+  const int* block_run = nullptr;   // tables: run of each 256 padded rows
+  const int* run_offsets = nullptr;
+  const int* pad_offsets = nullptr;
+  void* train_op = nullptr;
+  void* query_op = nullptr;
+};
+hipError_t launch_stream_operands(const StreamOperandJob& job, hipStream_t s);
+inline size_t stream_operand_bytes(size_t pad_rows, int steps) { return pad_rows * steps * 64; }
+
+// Candidates of every query, then the rerank (certified queries get their k
+// nearest, the others flags = 1).
+hipError_t launch_knn_stream(const KnnStreamParams& prm, hipStream_t s);
+
+}  // namespace kodama_hip

@@ -1,0 +1,845 @@
+// Exact kNN through FP16 matrix-core candidates with a running threshold, and
+// an exact FP32 rerank.
+//
+// Score of a (query, train row) pair: s = q.t - |t|^2 / 2 (Euclidean) or q.t
+// (inner product, cosine rows); the nearest rows have the largest scores. All
+// rows are scaled by one power of two that brings the largest norm to at most
+// 2^14, rounded to FP16 (parts = 1) or split into two FP16 parts (parts = 3:
+// hi.hi + hi.lo + lo.hi along K), and the norm term rides in spare K columns
+// (2^13 on the query side, the FP16 parts of -|t|^2 / 2^14 on the train
+// side), so one v_mfma_f32_16x16x32_f16 chain gives s for 16 x 16 pairs. Each
+// s differs from the exact distance's by at most E (pair_error below).
+//
+// Three kernels stream the train rows (a wave owns 16 NQ queries as B operands
+// in registers; train rows go through LDS 64 at a time in the fragment order
+// of the A operand, so staging and reads are linear; output lane l holds query
+// l % 16 against train rows 4 (l / 16) + r):
+//
+// knn_maxima_kernel, over all rows or a sample of about 1000 k: each lane
+// keeps the largest score of each of its 8 row classes (half a three-way
+// maximum per pair, no branch). A query has 32 classes per slice of the
+// sample, at least 2.1 k in all.
+// knn_threshold_kernel: T = the k-th largest of a query's class maxima (all of
+// distinct rows, so at least k rows reach T; it is about the 1.4 k-th largest
+// score), threshold T - 2E: the k-th best exact distance belongs to a
+// score >= T - E, so every row of the true k nearest scores >= T - 2E.
+// knn_candidates_kernel, over all rows: a pair below its query's threshold is
+// dropped with one maximum and one compare per four pairs; the others are
+// appended to the query's candidate buffer. Where the sample was a part of the
+// rows the buffer may run full; the wave then tightens T from the buffer
+// itself (bisection over ballots) and drops what falls below.
+// Two passes of MFMAs with 1.4 k appends per query cost less than one
+// pass with lists or a running threshold (k ln(n / k) appends): an append
+// takes as long as the MFMAs of some 1000 pairs.
+//
+// knn_stream_rerank_kernel: one wave per query merges the slices'
+// candidates, applies the same bound once more, re-scores what is left in the
+// reference's FP32 summation order (one candidate per lane) and writes the k
+// smallest by (distance, index): the rows and values of the exact scan.
+// Queries whose bound kept more than the buffer holds (many near-equal
+// distances) are flagged for another path.
+//
+// Measured on one MI355X: the self graph of 1M x 50, k = 30, maxima 3.5 ms,
+// candidates 130 ms (7.7e12 pairs/s, 0.98 PFLOP/s of FP16 with the padding to
+// 64 columns), rerank 5.4 ms; split-BF16 products with sorted lists per lane
+// column took 871 + 34 ms for the candidates. 100k x 50, k = 100: 1.0 + 2.8 +
+// 1.5 ms against 26.6 + 18.9 (scan of the queries the lists could not
+// certify) + 1.3. 10007 x 30011 x 100, k = 30: 0.33 ms against 23.1 ms of the
+// register scan. A running threshold without the maxima appended 3.5 times as
+// much: 316 ms at 1M rows, 18.3 ms at 100k.
+#include <hip/hip_runtime.h>
+
+#include <cfloat>
+#include <cmath>
+#include <cstdint>
+#include <type_traits>
+
+#include "knn_stream.h"
+
+namespace kodama_hip {
+
+namespace {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // a 16-byte operand piece
+
+constexpr int kWave = 64;
+constexpr int kChunk = 64;  // train rows per LDS stage
+
+__device__ __forceinline__ f16x8 as_f16x8(u32x4 v) { return __builtin_bit_cast(f16x8, v); }
+
+__device__ __forceinline__ uint32_t order_key(float v) {
+  const uint32_t b = __float_as_uint(v);
+  return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+__device__ __forceinline__ float key_value(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
+}
+
+// Power-of-two scale: the largest norm lands in (2^13, 2^14].
+__device__ __forceinline__ float operand_scale(const float* __restrict__ norm2_max) {
+  const float m = fmaxf(norm2_max[0], norm2_max[1]);
+  if (!(m > 0.0f)) return 1.0f;
+  int e;
+  (void)frexpf(sqrtf(m), &e);  // sqrt(m) <= 2^e
+  return ldexpf(1.0f, min(max(14 - e, -126), 126));
+}
+
+// Norm maxima outside this range (distances may overflow, or squares
+// underflow) are not served: every query is flagged.
+__device__ __forceinline__ bool norms_usable(const float* __restrict__ norm2_max) {
+  const float m = fmaxf(norm2_max[0], norm2_max[1]);
+  return m < 1e37f && (m == 0.0f || m > 1e-30f);
+}
+
+// Bound of |s - exact score| in scaled units, for a query of scaled norm q and
+// train rows of scaled norm <= t (u = 2^-11, FP16's unit roundoff; operands
+// below 2^-14 may be flushed):
+//   rounding of the operands  parts 1: (2u + u^2) q t; parts 3: 3.1 u^2 q t,
+//   flushed operands          2.1 2^-14 sqrt(p) (q + t) + 1,
+//   FP32 accumulation         K 2^-23 (q t + t^2 / 2), any order,
+//   the norm column           2^-22 t^2 / 2, and its FP32 sum (p + 2) 2^-25 t^2,
+//   the reference's own FP32 distance  50 2^-24 (q^2 + t^2) (p <= 256: at most
+//   8 block sums, the lane tree of 5 and 31 tail terms in sequence).
+__device__ __forceinline__ float pair_error(float q, float t, int p, int parts, int width) {
+  const float u = 0x1p-11f;
+  const float c1 = (parts == 1 ? 2.0f * u + u * u : 3.1f * u * u) + width * 0x1.04p-23f;
+  const float c2 = 0x1p-23f + (p + 2) * 0x1p-25f + 50.0f * 0x1p-24f + width * 0x1p-24f;
+  const float c3 = 2.1f * 0x1p-14f * sqrtf(static_cast<float>(p));
+  return 1.05f * (c1 * q * t + c2 * (q * q + t * t) + c3 * (q + t) + 1.0f);
+}
+
+// Wave maximum / minimum by DPP (gfx9 row shifts and row broadcasts), uniform.
+__device__ __forceinline__ uint32_t wave_max(uint32_t v) {
+#define KODAMA_DPP_MAX(ctrl, rows) \
+  v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), ctrl, rows, 0xf, false)))
+  KODAMA_DPP_MAX(0x111, 0xf);
+  KODAMA_DPP_MAX(0x112, 0xf);
+  KODAMA_DPP_MAX(0x114, 0xf);
+  KODAMA_DPP_MAX(0x118, 0xf);
+  KODAMA_DPP_MAX(0x142, 0xa);
+  KODAMA_DPP_MAX(0x143, 0xc);
+#undef KODAMA_DPP_MAX
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
+}
+
+// A key that at least k of the wave's keys (R per lane, 0 = empty, at least k
+// non-empty) reach and at most k + 2 unless ties or `exact`: bisection on
+// ballot counts. Uniform.
+template <int R>
+__device__ __forceinline__ uint32_t kth_largest(const uint32_t (&key)[R], int used, int k) {
+  uint32_t hi = 0, lo = 0;
+#pragma unroll
+  for (int i = 0; i < R; ++i) hi = max(hi, key[i]);
+  {
+    uint32_t inv = 0;  // smallest non-empty key, as the largest complement
+#pragma unroll
+    for (int i = 0; i < R; ++i) inv = max(inv, key[i] != 0u ? ~key[i] : 0u);
+    lo = ~wave_max(inv);
+  }
+  hi = wave_max(hi);  // count(>= lo) >= k; the answer is in [lo, hi]
+  while (lo < hi) {
+    const uint32_t mid = lo + (hi - lo + 1u) / 2u;  // lo < mid <= hi
+    int c = 0;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      if (i < used) c += __popcll(__ballot(key[i] >= mid));
+    }
+    if (c >= k) {
+      lo = mid;
+      if (c <= k + 2) break;
+    } else {
+      hi = mid - 1u;
+    }
+  }
+  return lo;
+}
+
+// T - 2E with room for its own rounding.
+__device__ __forceinline__ float drop_bound(float t, float err2) { return t - err2 - fabsf(t) * 0x1p-22f; }
+
+}  // namespace
+
+// 16 lanes per row; block maximum, one atomic per block (norms are >= 0, so
+// their bits order as integers; a NaN norm does not enter).
+__global__ void stream_norms_kernel(const float* __restrict__ x, int rows, int p, float* __restrict__ norm2,
+                                    float* __restrict__ norm2_max) {
+  __shared__ uint32_t s_max;
+  if (threadIdx.x == 0) s_max = 0u;
+  __syncthreads();
+  const int sub = threadIdx.x & 15;
+  for (size_t r = static_cast<size_t>(blockIdx.x) * 16 + (threadIdx.x >> 4); r < static_cast<size_t>(rows);
+       r += static_cast<size_t>(gridDim.x) * 16) {
+    const float* src = x + r * p;
+    float s = 0.0f;
+    for (int d = sub; d < p; d += 16) s = fmaf(src[d], src[d], s);
+    s += __shfl_xor(s, 1);
+    s += __shfl_xor(s, 2);
+    s += __shfl_xor(s, 4);
+    s += __shfl_xor(s, 8);
+    if (sub == 0) {
+      norm2[r] = s;
+      if (s >= 0.0f) atomicMax(&s_max, __float_as_uint(s));
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && s_max != 0u) atomicMax(reinterpret_cast<uint32_t*>(norm2_max), s_max);
+}
+
+// One thread per 16-byte fragment piece: piece ((tile * steps + step) * 64 +
+// lane) holds row tile * 16 + lane % 16, columns step * 32 + 8 (lane / 16)
+// .. + 7. Blocks cover 256 pieces; reads are 8 consecutive floats of 16 rows.
+__global__ void stream_operands_kernel(StreamOperandJob job, int steps) {
+  const size_t e = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const size_t total = static_cast<size_t>(job.pad_rows) / 16 * steps * 64;
+  if (e >= total) return;
+  const int lane = static_cast<int>(e & 63);
+  const size_t ts = e >> 6;
+  const int step = static_cast<int>(ts % steps);
+  const int prow = static_cast<int>(ts / steps) * 16 + (lane & 15);
+  int row = prow;
+  bool live = prow < job.rows;
+  if (job.block_run != nullptr) {
+    const int run = job.block_run[prow / kStreamBlockRows];
+    const int local = prow - job.pad_offsets[run];
+    live = local < job.run_offsets[run + 1] - job.run_offsets[run];
+    row = job.run_offsets[run] + local;
+  }
+  const float scale = operand_scale(job.norm2_max);
+  const int p = job.p;
+  const int c0 = step * 32 + 8 * (lane >> 4);
+  _Float16 tv[8], qv[8];
+  const float* src = job.x + static_cast<size_t>(live ? row : 0) * p;
+  const float nt = live && job.euclid ? -(job.norm2[row] * scale) * scale * 0x1p-14f : 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int c = c0 + i;
+    _Float16 a = static_cast<_Float16>(0.0f), b = static_cast<_Float16>(0.0f);
+    if (live) {
+      if (c < job.parts * p) {
+        const int seg = c / p, d = c - seg * p;
+        const float v = src[d] * scale;
+        const _Float16 h = static_cast<_Float16>(v);
+        const _Float16 l = static_cast<_Float16>(v - static_cast<float>(h));
+        a = seg == 1 ? l : h;  // train: hi, lo, hi
+        b = seg == 2 ? l : h;  // query: hi, hi, lo
+      } else if (job.euclid) {
+        const int j = c - job.parts * p;
+        const _Float16 h = static_cast<_Float16>(nt);
+        const float r1 = nt - static_cast<float>(h);
+        const _Float16 m = static_cast<_Float16>(r1);
+        const _Float16 l = static_cast<_Float16>(r1 - static_cast<float>(m));
+        const int parts = job.parts == 1 ? 2 : 3;
+        if (j < parts) {
+          a = j == 0 ? h : j == 1 ? m : l;
+          b = static_cast<_Float16>(8192.0f);
+        }
+      }
+    }
+    tv[i] = a;
+    qv[i] = b;
+  }
+  if (job.train_op != nullptr) {
+    f16x8 w;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = tv[i];
+    reinterpret_cast<u32x4*>(job.train_op)[e] = __builtin_bit_cast(u32x4, w);
+  }
+  if (job.query_op != nullptr) {
+    f16x8 w;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i] = qv[i];
+    reinterpret_cast<u32x4*>(job.query_op)[e] = __builtin_bit_cast(u32x4, w);
+  }
+}
+
+// The queries and train rows of one workgroup.
+struct StreamRange {
+  int t_begin, t_end, q_end;  // operand rows
+  int delta;                  // operand row -> row of x (tables: concatenated)
+};
+__device__ __forceinline__ StreamRange stream_range(const KnnStreamParams& prm, int q_block) {
+  StreamRange g{0, prm.train_rows, prm.query_rows, 0};
+  if (prm.block_run != nullptr) {
+    const int run = prm.block_run[q_block / kStreamBlockRows];
+    g.t_begin = prm.pad_offsets[run];
+    g.t_end = g.q_end = g.t_begin + (prm.run_offsets[run + 1] - prm.run_offsets[run]);
+    g.delta = prm.run_offsets[run] - g.t_begin;
+  }
+  return g;
+}
+
+// LDS staging of 64 train rows: the next chunk is loaded into registers while
+// this one is scored; two buffers, one barrier per chunk.
+constexpr int kThreads = 256;
+template <int KS>
+__device__ __forceinline__ void fetch_chunk(const KnnStreamParams& prm, const StreamRange& g, int c0, u32x4 (&pre)[KS],
+                                            int& pre_grp) {
+  const u32x4* src = reinterpret_cast<const u32x4*>(prm.train_op) + static_cast<size_t>(c0 / 16) * (KS * 64);
+#pragma unroll
+  for (int i = 0; i < KS; ++i) pre[i] = src[static_cast<int>(threadIdx.x) + i * kThreads];
+  if (prm.folds != nullptr && threadIdx.x < kChunk) {
+    const int j = c0 + static_cast<int>(threadIdx.x);
+    pre_grp = j < g.t_end ? prm.folds[j + g.delta] : -2;
+  }
+}
+template <int KS>
+__device__ __forceinline__ void store_chunk(const KnnStreamParams& prm, const u32x4 (&pre)[KS], int pre_grp, u32x4* s_t,
+                                            int* s_grp) {
+#pragma unroll
+  for (int i = 0; i < KS; ++i) s_t[static_cast<int>(threadIdx.x) + i * kThreads] = pre[i];
+  if (prm.folds != nullptr && threadIdx.x < kChunk) s_grp[threadIdx.x] = pre_grp;
+}
+
+template <int KS, int NQ>
+__device__ __forceinline__ void load_queries(const KnnStreamParams& prm, int q_wave, int q_end, int lane,
+                                             f16x8 (&bq)[NQ][KS]) {
+#pragma unroll
+  for (int t = 0; t < NQ; ++t) {
+    // Operand tiles exist for the padded rows; a wave past them reads none.
+    const u32x4* src =
+        reinterpret_cast<const u32x4*>(prm.query_op) + (static_cast<size_t>(q_wave / 16 + t) * KS) * 64 + lane;
+    const bool tile = q_wave + t * 16 < q_end;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) bq[t][ks] = as_f16x8(tile ? src[ks * 64] : u32x4{0, 0, 0, 0});
+  }
+}
+
+// KS: 32-deep steps. NQ: 16-query tiles per wave. blockIdx.x: query block,
+// blockIdx.y: share of the sampled chunks.
+template <int KS, int NQ, bool FOLDS>
+__global__ void __launch_bounds__(256, KS <= 2 ? 3 : 2) knn_maxima_kernel(KnnStreamParams prm) {
+  constexpr int kWaveQueries = NQ * 16;
+  __shared__ u32x4 s_t[2][KS * kThreads];  // 64 rows x KS x 64 bytes
+  __shared__ int s_grp[2][FOLDS ? kChunk : 4];
+  const int wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int grp = lane >> 4, col = lane & 15;
+  const int q_block = blockIdx.x * (4 * kWaveQueries);
+  const StreamRange g = stream_range(prm, q_block);
+  if (q_block >= g.q_end) return;
+  const int q_wave = q_block + wave * kWaveQueries;
+  f16x8 bq[NQ][KS];
+  load_queries<KS, NQ>(prm, q_wave, g.q_end, lane, bq);
+  int fold[NQ];
+  float top[NQ][8];  // class 2 sub + r / 2
+#pragma unroll
+  for (int t = 0; t < NQ; ++t) {
+    const int q = q_wave + t * 16 + col;
+    fold[t] = FOLDS && q < g.q_end ? prm.folds[q + g.delta] : -1;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) top[t][i] = -INFINITY;
+  }
+  // Sampled chunks, evenly spread and distinct (a row counted in two classes
+  // would spoil the threshold): chunk i of `picked` is floor(i chunks / picked).
+  const int chunks = (g.t_end - g.t_begin + kChunk - 1) / kChunk;
+  const int picked = min(chunks, prm.sample_chunks);
+  const int step = chunks / picked, rest = chunks - step * picked;
+  const int i0 = picked * static_cast<int>(blockIdx.y) / prm.max_slices;
+  const int i1 = picked * static_cast<int>(blockIdx.y + 1) / prm.max_slices;
+  auto chunk_row = [&](int i) {
+    return g.t_begin + (i * step + (rest != 0 ? i * rest / picked : 0)) * kChunk;
+  };
+  u32x4 pre[KS];
+  int pre_grp = -2;
+  if (i0 < i1) {
+    fetch_chunk<KS>(prm, g, chunk_row(i0), pre, pre_grp);
+    store_chunk<KS>(prm, pre, pre_grp, s_t[0], s_grp[0]);
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the operands too: no wait for them (and the prefetch) in the loop
+  __syncthreads();
+  int buf = 0;
+  for (int i = i0; i < i1; ++i, buf ^= 1) {
+    if (i + 1 < i1) fetch_chunk<KS>(prm, g, chunk_row(i + 1), pre, pre_grp);
+    const int c0 = chunk_row(i);
+    // `cut`: rows past the end (the last chunk only) must not count.
+    auto score = [&](auto cut) {
+#pragma unroll
+      for (int sub = 0; sub < kChunk / 16; ++sub) {
+        f32x4 acc[NQ];
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const f16x8 a = as_f16x8(s_t[buf][(sub * KS + ks) * 64 + lane]);
+#pragma unroll
+          for (int t = 0; t < NQ; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq[t][ks], acc[t], 0, 0, 0);
+        }
+        if constexpr (decltype(cut)::value) {
+          const int j0 = c0 + sub * 16 + 4 * grp;
+#pragma unroll
+          for (int t = 0; t < NQ; ++t) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[t][r] = j0 + r < g.t_end ? acc[t][r] : -INFINITY;
+          }
+        }
+        if constexpr (FOLDS) {
+          const int4 f = *reinterpret_cast<const int4*>(&s_grp[buf][sub * 16 + 4 * grp]);
+#pragma unroll
+          for (int t = 0; t < NQ; ++t) {
+            acc[t][0] = f.x != fold[t] ? acc[t][0] : -INFINITY;
+            acc[t][1] = f.y != fold[t] ? acc[t][1] : -INFINITY;
+            acc[t][2] = f.z != fold[t] ? acc[t][2] : -INFINITY;
+            acc[t][3] = f.w != fold[t] ? acc[t][3] : -INFINITY;
+          }
+        }
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) {
+          top[t][2 * sub] = fmaxf(fmaxf(top[t][2 * sub], acc[t][0]), acc[t][1]);
+          top[t][2 * sub + 1] = fmaxf(fmaxf(top[t][2 * sub + 1], acc[t][2]), acc[t][3]);
+        }
+      }
+    };
+    if (c0 + kChunk > g.t_end) score(std::true_type{});
+    else score(std::false_type{});
+    if (i + 1 < i1) store_chunk<KS>(prm, pre, pre_grp, s_t[buf ^ 1], s_grp[buf ^ 1]);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int t = 0; t < NQ; ++t) {
+    const int q = q_wave + t * 16 + col;
+    if (q < g.q_end) {
+      float4* dst = reinterpret_cast<float4*>(prm.maxima + (static_cast<size_t>(q) * prm.max_slices + blockIdx.y) * 32 +
+                                              grp * 8);
+      dst[0] = make_float4(top[t][0], top[t][1], top[t][2], top[t][3]);
+      dst[1] = make_float4(top[t][4], top[t][5], top[t][6], top[t][7]);
+    }
+  }
+}
+
+// One wave per operand row; REGS x 64 class maxima (empty ones -inf).
+template <int REGS>
+__global__ void __launch_bounds__(256) knn_threshold_kernel(KnnStreamParams prm, int rows, int per_query) {
+  const int q = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x / kWave));
+  const int lane = threadIdx.x & (kWave - 1);
+  if (q >= rows) return;
+  int delta = 0;
+  if (prm.block_run != nullptr) {
+    const StreamRange g = stream_range(prm, q);
+    if (q >= g.q_end) return;
+    delta = g.delta;
+  }
+  const float* src = prm.maxima + static_cast<size_t>(q) * per_query;
+  uint32_t key[REGS];
+  int valid = 0;
+#pragma unroll
+  for (int i = 0; i < REGS; ++i) {
+    const float v = i * kWave + lane < per_query ? src[i * kWave + lane] : -INFINITY;
+    key[i] = v > -INFINITY ? order_key(v) : 0u;
+    valid += __popcll(__ballot(key[i] != 0u));
+  }
+  // One more than k where a query may exclude a train row (tables mask the
+  // query's own fold before the maxima).
+  const int want = prm.k + (prm.exclude != nullptr ? 1 : 0);
+  float bound = norms_usable(prm.norm2_max) ? -INFINITY : INFINITY;
+  if (valid >= want && bound < 0.0f) {
+    const float scale = operand_scale(prm.norm2_max);
+    const float tmax = sqrtf(prm.norm2_max[0]) * scale * 1.0001f;
+    const float qn = sqrtf(prm.query_norm2[q + delta]) * scale * 1.0001f;
+    const int width = prm.parts * prm.dims + (prm.euclid ? 3 : 0);
+    bound = drop_bound(key_value(kth_largest<REGS>(key, REGS, want)),
+                       2.0f * pair_error(qn, tmax, prm.dims, prm.parts, width));
+  }
+  if (lane == 0) prm.threshold[q] = bound;
+}
+
+// R: capacity / 64. blockIdx.x: query block, blockIdx.y: slice of the train rows.
+template <int KS, int NQ, int R>
+__global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(KnnStreamParams prm) {
+  constexpr int kCap = 64 * R;
+  constexpr int kWaveQueries = NQ * 16;
+  __shared__ u32x4 s_t[2][KS * kThreads];  // 64 rows x KS x 64 bytes
+  __shared__ int s_grp[2][kChunk];
+  __shared__ int s_cnt[4][kWaveQueries];
+  __shared__ float s_th[4][kWaveQueries];
+  const int wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int grp = lane >> 4, col = lane & 15;
+  const int q_block = blockIdx.x * (4 * kWaveQueries);
+  StreamRange g = stream_range(prm, q_block);
+  if (q_block >= g.q_end) return;
+  // This slice's rows (a multiple of 64 except at the end; may be empty).
+  if (prm.slices > 1) {
+    const int rows = g.t_end - g.t_begin;
+    const int per = ((rows + prm.slices - 1) / prm.slices + kChunk - 1) / kChunk * kChunk;
+    g.t_begin += per * static_cast<int>(blockIdx.y);
+    g.t_end = min(g.t_end, g.t_begin + per);
+  }
+  const int q_wave = q_block + wave * kWaveQueries;
+  const size_t slot0 = static_cast<size_t>(q_wave) * prm.slices + blockIdx.y;  // query i: + i * slices
+  const bool usable = norms_usable(prm.norm2_max);
+
+  f16x8 bq[NQ][KS];
+  load_queries<KS, NQ>(prm, q_wave, g.q_end, lane, bq);
+  float th[NQ];
+  int ex[NQ];
+#pragma unroll
+  for (int t = 0; t < NQ; ++t) {
+    const int q = q_wave + t * 16 + col;
+    const bool live = q < g.q_end;
+    th[t] = live ? prm.threshold[q] : INFINITY;
+    ex[t] = -1;
+    if (live) {
+      if (prm.folds != nullptr) ex[t] = prm.folds[q + g.delta];
+      else if (prm.exclude != nullptr) ex[t] = prm.exclude[q];
+    }
+    if (grp == 0) {
+      s_cnt[wave][t * 16 + col] = usable ? 0 : -1;
+      s_th[wave][t * 16 + col] = th[t];
+    }
+  }
+
+  // Compaction of every query of the wave with more than `limit` candidates.
+  auto compact = [&](int limit) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");  // the appended entries and the counts
+    __builtin_amdgcn_wave_barrier();
+    const int mine = lane < kWaveQueries ? s_cnt[wave][lane] : 0;
+    uint64_t todo = __ballot(mine > limit);
+    const float scale = operand_scale(prm.norm2_max);
+    const float tmax = sqrtf(prm.norm2_max[0]) * scale * 1.0001f;
+    const int width = prm.parts * prm.dims + (prm.euclid ? 3 : 0);
+    while (todo != 0ull) {
+      const int q = __builtin_ctzll(todo);
+      todo &= todo - 1ull;
+      const int n = __builtin_amdgcn_readlane(mine, q);
+      uint2* base = prm.cand + (slot0 + static_cast<size_t>(q) * prm.slices) * kCap;
+      uint2 ent[R];
+      uint32_t key[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const int e = i * kWave + lane;
+        ent[i] = e < n ? base[e] : make_uint2(0xFF800000u, 0u);  // -inf
+        key[i] = e < n ? order_key(__uint_as_float(ent[i].x)) : 0u;
+      }
+      const float qn = sqrtf(prm.query_norm2[q_wave + q + g.delta]) * scale * 1.0001f;
+      const float bound = drop_bound(key_value(kth_largest<R>(key, R, prm.k)),
+                                     2.0f * pair_error(qn, tmax, prm.dims, prm.parts, width));
+      int kept = 0;
+      const uint64_t below = (1ull << lane) - 1ull;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const bool keep = key[i] != 0u && __uint_as_float(ent[i].x) >= bound;
+        const uint64_t m = __ballot(keep);
+        if (keep) base[kept + __popcll(m & below)] = ent[i];
+        kept += __popcll(m);
+      }
+      const bool over = kept > kCap - 32;
+      if (lane == 0) {
+        s_cnt[wave][q] = over ? -1 : kept;
+        s_th[wave][q] = over ? INFINITY : fmaxf(bound, s_th[wave][q]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int t = 0; t < NQ; ++t) th[t] = s_th[wave][t * 16 + col];
+  };
+
+  u32x4 pre[KS];
+  int pre_grp = -2;
+  if (g.t_begin < g.t_end) {
+    fetch_chunk<KS>(prm, g, g.t_begin, pre, pre_grp);
+    store_chunk<KS>(prm, pre, pre_grp, s_t[0], s_grp[0]);
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the operands too: no wait for them (and the prefetch) in the loop
+  __syncthreads();
+  int buf = 0;
+  for (int c0 = g.t_begin; c0 < g.t_end; c0 += kChunk, buf ^= 1) {
+    const bool more = c0 + kChunk < g.t_end;
+    if (more) fetch_chunk<KS>(prm, g, c0 + kChunk, pre, pre_grp);  // in flight during the scoring
+    const int limit = more ? c0 + kChunk : g.t_end;
+#pragma unroll 1
+    for (int sub = 0; sub < kChunk / 16; ++sub) {
+      f32x4 acc[NQ];
+#pragma unroll
+      for (int t = 0; t < NQ; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const f16x8 a = as_f16x8(s_t[buf][(sub * KS + ks) * 64 + lane]);
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq[t][ks], acc[t], 0, 0, 0);
+      }
+      uint64_t hit[NQ], any = 0ull;
+#pragma unroll
+      for (int t = 0; t < NQ; ++t) {
+        // Strictly above (the bound has slack): two three-way maxima and a compare.
+        hit[t] = __ballot(fmaxf(fmaxf(fmaxf(fmaxf(th[t], acc[t][0]), acc[t][1]), acc[t][2]), acc[t][3]) > th[t]);
+        any |= hit[t];
+      }
+      if (any != 0ull) {
+        const int j0 = c0 + sub * 16 + 4 * grp;
+        int4 gr = make_int4(j0, j0 + 1, j0 + 2, j0 + 3);
+        if (prm.folds != nullptr) gr = *reinterpret_cast<const int4*>(&s_grp[buf][sub * 16 + 4 * grp]);
+        const int row[4] = {gr.x, gr.y, gr.z, gr.w};
+        bool full = false;
+#pragma unroll
+        for (int t = 0; t < NQ; ++t) {
+          if (hit[t] == 0ull) continue;
+          bool pass[4];
+          int c = 0;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            pass[r] = acc[t][r] > th[t] && row[r] != ex[t] && j0 + r < limit;
+            c += pass[r] ? 1 : 0;
+          }
+          if (c > 0) {
+            // The lane's next slots of its query (four lanes share one).
+            const int slot = atomicAdd(&s_cnt[wave][t * 16 + col], c);
+            uint2* dst = prm.cand + (slot0 + static_cast<size_t>(t * 16 + col) * prm.slices) * kCap + slot;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              if (pass[r]) *dst++ = make_uint2(__float_as_uint(acc[t][r]), static_cast<uint32_t>(j0 + r + g.delta));
+            }
+            full = full || slot + c > kCap - 16;
+          }
+        }
+        if (__ballot(full) != 0ull) compact(kCap - 32);
+      }
+    }
+    if (more) store_chunk<KS>(prm, pre, pre_grp, s_t[buf ^ 1], s_grp[buf ^ 1]);
+    __syncthreads();
+  }
+  // Several slices: keep each list short enough for the rerank to hold all.
+  if (prm.slices > 1) compact(max(prm.k + 8, 24));
+#pragma unroll
+  for (int t = 0; t < NQ; ++t) {
+    const int q = q_wave + t * 16 + col;
+    if (grp == 0 && q < g.q_end) {
+      const size_t o = slot0 + static_cast<size_t>(t * 16 + col) * prm.slices;
+      prm.cand_count[o] = s_cnt[wave][t * 16 + col];
+      prm.cand_bound[o] = th[t];
+    }
+  }
+}
+
+// Reference-order FP32 distance (native_knn.cpp:41-95), one lane per train
+// row, the query row uniform over the wave (scalar loads).
+template <bool EUCLID>
+__device__ __forceinline__ float stream_exact_distance(const float* __restrict__ q, const float* __restrict__ c, int p) {
+  float acc[32];
+#pragma unroll
+  for (int s = 0; s < 32; ++s) acc[s] = 0.0f;
+  const int full = p & ~31;
+  for (int b = 0; b < full; b += 32) {
+#pragma unroll
+    for (int s = 0; s < 32; ++s) {
+      const float cv = c[b + s];
+      if (EUCLID) {
+        const float t = __fsub_rn(q[b + s], cv);
+        acc[s] = __fmaf_rn(t, t, acc[s]);
+      } else {
+        acc[s] = __fmaf_rn(q[b + s], cv, acc[s]);
+      }
+    }
+  }
+  float v4[4];
+#pragma unroll
+  for (int l = 0; l < 4; ++l) {
+    const float lo = __fadd_rn(__fadd_rn(acc[l], acc[8 + l]), __fadd_rn(acc[16 + l], acc[24 + l]));
+    const float hi = __fadd_rn(__fadd_rn(acc[4 + l], acc[12 + l]), __fadd_rn(acc[20 + l], acc[28 + l]));
+    v4[l] = __fadd_rn(lo, hi);
+  }
+  float r = __fadd_rn(__fadd_rn(v4[0], v4[1]), __fadd_rn(v4[2], v4[3]));
+  // Tail of up to 31 columns: loads first (clamped), then the chain.
+  float tail[32];
+#pragma unroll
+  for (int s = 0; s < 31; ++s) tail[s] = full + s < p ? c[full + s] : 0.0f;
+#pragma unroll
+  for (int s = 0; s < 31; ++s) {
+    if (full + s < p) {
+      if (EUCLID) {
+        const float t = __fsub_rn(q[full + s], tail[s]);
+        r = __fmaf_rn(t, t, r);
+      } else {
+        r = __fmaf_rn(q[full + s], tail[s], r);
+      }
+    }
+  }
+  return EUCLID ? r : -r;
+}
+
+template <bool EUCLID>
+__global__ void __launch_bounds__(256) knn_stream_rerank_kernel(KnnStreamParams prm) {
+  constexpr int kRegs = kStreamMerge / kWave;
+  __shared__ uint2 s_ent[4][kStreamMerge];
+  const int wave = threadIdx.x / kWave;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int q = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + wave);
+  if (q >= prm.query_rows) return;  // whole waves; no block barrier below
+  const int k = prm.k, p = prm.dims, cap = 16 * prm.list;
+  int op_row = q;  // operand (padded) row of a table query
+  if (prm.block_run != nullptr) {
+    int lo = 0, hi = prm.pad_rows / kStreamBlockRows - 1;
+    // The run of concatenated row q: block_run is ascending over the padded
+    // blocks, so search the runs through it.
+    hi = prm.block_run[hi];
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (prm.run_offsets[mid] <= q) lo = mid; else hi = mid - 1;
+    }
+    op_row = prm.pad_offsets[lo] + (q - prm.run_offsets[lo]);
+  }
+  uint2* ent = s_ent[wave];
+  const uint64_t below = (1ull << lane) - 1ull;
+  // Merge: what scores at or above the tightest slice's bound.
+  bool bad = false;
+  float bound = -INFINITY;
+  for (int sl = 0; sl < prm.slices; ++sl) {
+    const size_t o = static_cast<size_t>(op_row) * prm.slices + sl;
+    bad = bad || prm.cand_count[o] < 0;
+    bound = fmaxf(bound, prm.cand_bound[o]);
+  }
+  int n = 0;
+  for (int sl = 0; sl < prm.slices && !bad; ++sl) {
+    const size_t o = static_cast<size_t>(op_row) * prm.slices + sl;
+    const int c = prm.cand_count[o];
+    for (int e0 = 0; e0 < c; e0 += kWave) {
+      const int e = e0 + lane;
+      const uint2 v = e < c ? prm.cand[o * cap + e] : make_uint2(0xFF800000u, 0u);
+      const bool keep = e < c && __uint_as_float(v.x) >= bound;
+      const uint64_t m = __ballot(keep);
+      const int add = __popcll(m);
+      if (n + add > kStreamMerge) {
+        bad = true;
+        break;
+      }
+      if (keep) ent[n + __popcll(m & below)] = v;
+      n += add;
+    }
+  }
+  if (bad) {
+    if (lane == 0) prm.flags[q] = 1;
+    return;
+  }
+  if (lane == 0) prm.flags[q] = 0;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  if (n > k) {
+    uint32_t key[kRegs];
+#pragma unroll
+    for (int i = 0; i < kRegs; ++i) {
+      key[i] = 0u;
+      if (i * kWave < n) key[i] = i * kWave + lane < n ? order_key(__uint_as_float(ent[i * kWave + lane].x)) : 0u;
+    }
+    const float scale = operand_scale(prm.norm2_max);
+    const float tmax = sqrtf(prm.norm2_max[0]) * scale * 1.0001f;
+    const float qn = sqrtf(prm.query_norm2[q]) * scale * 1.0001f;
+    const int width = prm.parts * p + (prm.euclid ? 3 : 0);
+    bound = drop_bound(key_value(kth_largest<kRegs>(key, (n + kWave - 1) / kWave, k)),
+                       2.0f * pair_error(qn, tmax, p, prm.parts, width));
+    // In-place compaction: a register's entries go to slots at or before
+    // their own, and each is read before a later register's is written.
+    int kept = 0;
+    for (int e0 = 0; e0 < n; e0 += kWave) {
+      const int e = e0 + lane;
+      const uint2 v = e < n ? ent[e] : make_uint2(0xFF800000u, 0u);
+      const bool keep = e < n && __uint_as_float(v.x) >= bound;
+      const uint64_t m = __ballot(keep);
+      __builtin_amdgcn_wave_barrier();
+      if (keep) ent[kept + __popcll(m & below)] = v;
+      __builtin_amdgcn_wave_barrier();
+      kept += __popcll(m);
+    }
+    n = kept;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  // Exact distances as sortable (distance, row) pairs.
+  const float* qrow = prm.query + static_cast<size_t>(q) * p;
+  for (int e = lane; e < n; e += kWave) {
+    const int row = static_cast<int>(ent[e].y);
+    const float d = stream_exact_distance<EUCLID>(qrow, prm.train + static_cast<size_t>(row) * p, p);
+    ent[e].x = __float_as_uint(d);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  int* out_i = prm.out_index + static_cast<size_t>(q) * k;
+  float* out_d = prm.out_dist + static_cast<size_t>(q) * k;
+  for (int e = lane; e < n; e += kWave) {
+    const uint2 v = ent[e];
+    const float d = __uint_as_float(v.x);
+    int rank = 0;
+    for (int t = 0; t < n; ++t) {
+      const uint2 o = ent[t];
+      const float od = __uint_as_float(o.x);
+      rank += od < d || (od == d && o.y < v.y) ? 1 : 0;
+    }
+    if (rank < k) {
+      out_i[rank] = static_cast<int>(v.y);
+      out_d[rank] = d;
+    }
+  }
+  for (int t = n + lane; t < k; t += kWave) {
+    out_i[t] = -1;
+    out_d[t] = INFINITY;
+  }
+}
+
+hipError_t launch_stream_norms(const float* x, int rows, int p, float* norm2, float* norm2_max, hipStream_t s) {
+  if (rows == 0) return hipSuccess;
+  const int blocks = (rows + 15) / 16;
+  hipLaunchKernelGGL(stream_norms_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, x,
+                     rows, p, norm2, norm2_max);
+  return hipGetLastError();
+}
+
+hipError_t launch_stream_operands(const StreamOperandJob& job, hipStream_t s) {
+  if (job.pad_rows == 0) return hipSuccess;
+  const int steps = stream_steps(job.p, job.parts, job.euclid != 0);
+  if (job.pad_rows % kStreamBlockRows != 0 || job.p < 1 || steps > kStreamMaxSteps ||
+      (job.parts != 1 && job.parts != 3)) {
+    return hipErrorInvalidValue;
+  }
+  const size_t total = static_cast<size_t>(job.pad_rows) / 16 * steps * 64;
+  hipLaunchKernelGGL(stream_operands_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, s, job,
+                     steps);
+  return hipGetLastError();
+}
+
+template <int KS>
+static void launch_steps(const KnnStreamParams& prm, hipStream_t s) {
+  const int rows = prm.block_run != nullptr ? prm.pad_rows : prm.query_rows;
+  constexpr int NQ = KS <= 4 ? 4 : 2;
+  const int qpb = 4 * NQ * 16;
+  const unsigned qblocks = static_cast<unsigned>((rows + qpb - 1) / qpb);
+  const dim3 mgrid(qblocks, static_cast<unsigned>(prm.max_slices));
+  if (prm.folds != nullptr) hipLaunchKernelGGL((knn_maxima_kernel<KS, NQ, true>), mgrid, dim3(256), 0, s, prm);
+  else hipLaunchKernelGGL((knn_maxima_kernel<KS, NQ, false>), mgrid, dim3(256), 0, s, prm);
+  const int per_query = prm.max_slices * 32;
+  const dim3 tgrid(static_cast<unsigned>((rows + 3) / 4));
+  if (per_query <= 64) hipLaunchKernelGGL((knn_threshold_kernel<1>), tgrid, dim3(256), 0, s, prm, rows, per_query);
+  else if (per_query <= 128) hipLaunchKernelGGL((knn_threshold_kernel<2>), tgrid, dim3(256), 0, s, prm, rows, per_query);
+  else if (per_query <= 256) hipLaunchKernelGGL((knn_threshold_kernel<4>), tgrid, dim3(256), 0, s, prm, rows, per_query);
+  else hipLaunchKernelGGL((knn_threshold_kernel<8>), tgrid, dim3(256), 0, s, prm, rows, per_query);
+  const dim3 grid(qblocks, static_cast<unsigned>(prm.slices));
+  if (prm.list == 8) hipLaunchKernelGGL((knn_candidates_kernel<KS, NQ, 2>), grid, dim3(256), 0, s, prm);
+  else hipLaunchKernelGGL((knn_candidates_kernel<KS, NQ, 4>), grid, dim3(256), 0, s, prm);
+}
+
+hipError_t launch_knn_stream(const KnnStreamParams& prm, hipStream_t s) {
+  if (prm.query_rows == 0) return hipSuccess;
+  const int steps = stream_steps(prm.dims, prm.parts, prm.euclid != 0);
+  if (prm.dims < 1 || steps > kStreamMaxSteps || prm.k < 1 || prm.k > kStreamMaxK || prm.train_rows < 1 ||
+      prm.slices < 1 || prm.max_slices < 1 || prm.max_slices > kStreamMaxSlices || prm.sample_chunks < 1 || (prm.list != 8 && prm.list != 16) || (prm.list == 8 && prm.k > 32) ||
+      (prm.block_run != nullptr) != (prm.folds != nullptr) || prm.pad_rows % kStreamBlockRows != 0) {
+    return hipErrorInvalidValue;
+  }
+  switch (steps) {
+    case 1: launch_steps<1>(prm, s); break;
+    case 2: launch_steps<2>(prm, s); break;
+    case 3: launch_steps<3>(prm, s); break;
+    case 4: launch_steps<4>(prm, s); break;
+    case 5: launch_steps<5>(prm, s); break;
+    case 6: launch_steps<6>(prm, s); break;
+    case 7: launch_steps<7>(prm, s); break;
+    case 8: launch_steps<8>(prm, s); break;
+    default: launch_steps<9>(prm, s); break;
+  }
+  const unsigned rblocks = static_cast<unsigned>((prm.query_rows + 3) / 4);
+  if (prm.euclid) hipLaunchKernelGGL((knn_stream_rerank_kernel<true>), dim3(rblocks), dim3(256), 0, s, prm);
+  else hipLaunchKernelGGL((knn_stream_rerank_kernel<false>), dim3(rblocks), dim3(256), 0, s, prm);
+  return hipGetLastError();
+}
+
+}  // namespace kodama_hip

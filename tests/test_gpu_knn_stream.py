@@ -1,0 +1,79 @@
+"""FP16 matrix-core candidates of the exact kNN (class maxima, threshold,
+candidates, exact rerank): neighbours and distances bit-identical to the
+oracle's exhaustive search where the operand width, the number of parts, the
+sample, the slices and the candidate buffers change."""
+import numpy as np
+import pytest
+
+import kodama_amd as K
+from kodama_amd import datasets as D
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(oracle, train, query, k, name, exclude=None, most=0):
+    idx, dist = K.exact_knn_search(train, query, k, name, exclude=exclude)
+    fb = K.last_knn_fallbacks()
+    want = oracle.exact_knn(train, query, k, K._metric(name), exclude=exclude)
+    assert np.array_equal(idx, want[0])
+    assert np.array_equal(dist, want[1])
+    assert 0 <= fb <= most, fb
+
+
+# Columns at the edges of the operand: one step (three parts up to 9 columns,
+# one part up to 30), two (20 / 21: three parts or one; 62 / 63), the widths
+# past 64 (from 1024 queries on) up to nine steps, where the second pass with
+# three parts ends (95 / 96).
+@pytest.mark.parametrize("p", [1, 9, 10, 20, 21, 30, 31, 62, 63, 64, 65, 95, 96, 126, 127, 200, 256])
+@pytest.mark.parametrize("name", ["euclidean", "inner_product"])
+def test_operand_widths(oracle, p, name):
+    queries = 257 if p <= 64 else 1024
+    x, _ = D.config3(n=4099 + queries, p=p, seed=p)
+    # Very few columns put many rows within the rounding bound of each other.
+    _check(oracle, x[:4099], x[4099:], 7, name, most=0 if p > 2 else queries)
+
+
+# k at the edges of the buffers (32 / 33), of the class maxima (1, 15, 16, 121,
+# 128) and of the sample (16 k chunks of 64 rows: 4100 to 20000 rows are a
+# sample below k = 20 and all rows above); queries at the edges of a tile, a
+# wave and a workgroup.
+@pytest.mark.parametrize("k", [1, 2, 15, 16, 32, 33, 121, 128])
+@pytest.mark.parametrize("rows,queries", [(4096, 1), (4161, 255), (20000, 17)])
+def test_neighbour_counts_and_ragged_sizes(oracle, k, rows, queries):
+    x, _ = D.config3(n=rows + queries, p=50, seed=k)
+    ex = (np.arange(queries, dtype=np.int32) * 37) % rows
+    _check(oracle, x[:rows], x[rows:], k, "euclidean", exclude=ex, most=queries // 20)
+
+
+def test_rows_sorted_by_distance_refill_the_buffers(oracle):
+    """Train rows that come ever closer: the evenly spread sample sets a bound
+    that the last rows all pass, so the buffers fill and are tightened."""
+    x, _ = D.config3(n=60000, p=24, seed=3)
+    query = x[:64] * np.float32(0.01)
+    order = np.argsort(-np.linalg.norm(x - query.mean(0), axis=1), kind="stable")
+    _check(oracle, np.ascontiguousarray(x[order]), query, 2, "euclidean")
+
+
+def test_cosine_graph_prepares_rows_as_the_host(oracle):
+    x, _ = D.config3(n=4500, p=37, seed=8)
+    x[17] = 0.0  # a row without a norm keeps its values
+    g = K.KODAMA_knn_graph(x, k=12, metric="cosine")
+    idx, dist = oracle.knn_graph(x, 12, 0)
+    assert np.array_equal(g["indices"], idx) and np.array_equal(g["distances"], dist)
+
+
+@pytest.mark.parametrize("scale", [1e-14, 1e17, 1e-17, 1e19])
+def test_extreme_scales(oracle, scale):
+    """Norms at both ends of the served range, and past it, where every query
+    takes the scan."""
+    x, _ = D.config3(n=4300, p=16, seed=2)
+    x = (x * np.float32(scale)).astype(np.float32)
+    _check(oracle, x[:4200], x[4200:], 9, "euclidean", most=100)
+
+
+def test_outlying_rows_loosen_the_bound_but_not_the_result(oracle):
+    """One train row 1000 times the others: the bound follows its norm, so the
+    first pass certifies little and the others answer."""
+    x, _ = D.config3(n=5000, p=50, seed=12)
+    x[40] *= 1000.0
+    _check(oracle, x[:4900], x[4900:], 20, "euclidean", most=100)
