@@ -107,10 +107,11 @@ const char* kodama_hip_version(void);
 /* No counterpart in the reference: for callers that check which path the last
  * exact kNN search of the calling thread took (kodama_hip_exact_knn_search,
  * kodama_hip_knn_graph, and the per-fold tables of the kNN classifier calls).
- * With at most 64 dimensions, k <= 128 and (for a search) at least 4096 train
- * rows the search runs split-BF16 MFMA candidates with an exact FP32 rerank and
- * returns the number of queries (table rows) that fell back to the exact scan;
- * -1 when the exact scan served every query. Results are identical either way. */
+ * With k <= 128 and, for a search, at least 4096 train rows (beyond 64 columns
+ * also at least 1024 queries) the search runs FP16 matrix-core candidates with
+ * an exact FP32 rerank and returns the number of queries (table rows) that
+ * fell back to the exact scan; -1 when the exact scan served every query.
+ * Results are identical either way. */
 int kodama_hip_last_knn_fallbacks(void);
 
 /* Per-fold kNN tables of a batch of runs: replaces precompute_knn_cv_cuda
@@ -122,9 +123,8 @@ int kodama_hip_last_knn_fallbacks(void);
  * ids in (distance, id) order and scores = minus the internal distance, -1 /
  * -inf past the available rows -- the reference's per-fold exact tables,
  * bit-identical. path: 1 the register scan in the reference's summation
- * order; 2 split-BF16 MFMA candidates with the exact FP32 rerank (p <= 64,
- * k <= 128; otherwise the scan); 0 the process-wide setting below. Both paths
- * give identical tables. *path_used (may be NULL) = the path that ran. */
+ * order; 2 matrix-core candidates with the exact FP32 rerank; 0 the
+ * process-wide setting below. Both paths give identical tables. *path_used (may be NULL) = the path that ran. */
 int kodama_hip_knn_fold_tables(const float* x, int32_t n, int32_t p, int32_t runs, const int32_t* run_offsets,
                                const int32_t* rows, const int32_t* fold_ids, int32_t k, int32_t metric,
                                int32_t path, int32_t device, int32_t* neighbors, float* scores,
@@ -132,30 +132,23 @@ int kodama_hip_knn_fold_tables(const float* x, int32_t n, int32_t p, int32_t run
 
 /* No counterpart in the reference: the process-wide path of the per-fold
  * tables that every kNN classifier call builds (KNNCV, CoreKNN, the batches,
- * KODAMA.matrix): 1 scan, 2 MFMA, 0 (default) tuned -- the first table of a
- * shape bucket (columns, k class, metric, log2 of the largest run and of all
- * rows, folds) runs both paths, timed, and the faster serves the bucket for
- * the rest of the process. kodama_hip_last_fold_table_path returns the path
- * the calling thread's last table build used (0 before any). */
+ * KODAMA.matrix): 1 scan, 2 matrix cores, 0 (default) by rule -- the scan where
+ * the largest run has fewer than 64 rows. kodama_hip_last_fold_table_path
+ * returns the path the calling thread's last table build used (0 before any). */
 int kodama_hip_set_fold_table_path(int32_t path);
 int kodama_hip_last_fold_table_path(void);
-/* The tuner's full schedule (no reference counterpart): path as above; for
- * the MFMA path the candidates kept per (query, lane column), list = 8 (k <=
- * 32) or 16, and the waves of 16 queries per workgroup, waves = 4 or 8; 0 =
- * tuned. With path 0 the first table of a shape bucket times the scan (below
- * the bucket sizes where MFMA is known to win) and every MFMA schedule the
- * forced values leave, and the fastest serves the bucket from then on; all
- * schedules give identical tables. A forced list that excludes the job's k
- * leaves the scan. kodama_hip_last_fold_table_schedule reports the calling
- * thread's last build (list and waves 0 for the scan). */
+/* The full schedule (no reference counterpart): path as above; for the
+ * matrix-core path the candidates kept per query and slice, 16 x list, list =
+ * 8 (k <= 32) or 16; 0 = 8 where k allows it. waves (4, 8 or 0) is kept for
+ * callers: it is reported back and chooses nothing, every workgroup has four
+ * waves. All schedules give identical tables. A forced list that excludes the
+ * job's k leaves the scan. kodama_hip_last_fold_table_schedule reports the
+ * calling thread's last build (list and waves 0 for the scan). */
 int kodama_hip_set_fold_table_schedule(int32_t path, int32_t list, int32_t waves);
 int kodama_hip_last_fold_table_schedule(int32_t* path, int32_t* list, int32_t* waves);
-/* Candidate lists of the MFMA kNN path (no reference counterpart), process
- * wide: on = 1 (the default) keeps each candidate as one 32-bit key, the
- * value's order bits with the row's index within its lane column in the low
- * bits, wherever a search's train rows (a batch's largest run) number at most
- * 32768; on = 0 keeps separate values and indices. Both give the same
- * neighbours. */
+/* Kept for callers (no reference counterpart): the candidate buffers hold
+ * (score, row) pairs for every size, so on = 1 (the default) and on = 0 run the
+ * same code; other values are EINVAL. */
 int kodama_hip_set_mfma_packed_lists(int32_t on);
 
 /* Tuning control of the device-resident evolution (no reference counterpart:

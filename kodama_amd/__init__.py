@@ -605,17 +605,17 @@ def set_fold_table_path(path="tuned"):
 
 
 def set_fold_table_schedule(path="tuned", list=0, waves=0):
-    """Process-wide schedule of the per-fold tables: path ("tuned", "scan",
-    "mfma"), and for the MFMA path the candidate list length (8 or 16) and the
-    waves per workgroup (4 or 8); 0 = tuned. Tables are identical for all."""
+    """Process-wide schedule of the per-fold tables: path ("tuned": by rule,
+    "scan", "mfma"), and for the matrix-core path the candidates kept per query
+    and slice, 16 x list (8 or 16; 0 = by k). waves (4, 8 or 0) is reported back
+    and chooses nothing. Tables are identical for all."""
     N.call("kodama_hip_set_fold_table_schedule", C.c_int32(_TABLE_PATHS[path]), C.c_int32(int(list)),
            C.c_int32(int(waves)))
 
 
 def set_mfma_packed_lists(on=True):
-    """Process-wide form of the MFMA kNN candidate lists: packed 32-bit keys
-    (value order bits and column index; the default, where the train rows
-    number at most 32768) or separate values and indices. Same neighbours."""
+    """Kept for callers: the candidate buffers have one form, both settings run
+    the same code."""
     N.call("kodama_hip_set_mfma_packed_lists", C.c_int32(1 if on else 0))
 
 

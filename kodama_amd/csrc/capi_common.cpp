@@ -18,19 +18,6 @@ void set_last_error(const std::string& msg) { g_last_error = msg; }
 
 int& last_knn_fallbacks() { return g_knn_fallbacks; }
 
-float max_row_norm2(const float* x, int rows, int p) {
-  double best = 0.0;
-  for (int r = 0; r < rows; ++r) {
-    double s = 0.0;
-    for (int j = 0; j < p; ++j) {
-      const double v = x[static_cast<size_t>(r) * p + j];
-      s += v * v;
-    }
-    best = s > best ? s : best;
-  }
-  return static_cast<float>(best * (1.0 + 1e-6));
-}
-
 void select_device(int device) {
   int count = 0;
   if (hipGetDeviceCount(&count) != hipSuccess || count <= 0) {

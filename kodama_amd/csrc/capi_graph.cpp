@@ -10,7 +10,7 @@
 #include "capi_common.h"
 #include "engine.h"
 #include "graph_launch.h"
-#include "knn_mfma.h"
+#include "knn_search.h"
 #include "launch.h"
 
 using namespace kodama_hip;

@@ -16,7 +16,7 @@
 #include "batch_api.h"
 #include "evolve_device.h"
 #include "evolve_launch.h"
-#include "knn_mfma.h"
+#include "knn_search.h"
 #include "launch.h"
 #include "mlp.h"
 
@@ -441,8 +441,7 @@ int kodama_hip_set_fold_table_schedule(int32_t path, int32_t list, int32_t waves
 
 int kodama_hip_set_mfma_packed_lists(int32_t on) {
   return guarded([&] {
-    require(on == 0 || on == 1, "on must be 0 or 1.");
-    set_mfma_packed_lists(on);
+    require(on == 0 || on == 1, "on must be 0 or 1.");  // one form of the candidate buffers for both
   });
 }
 

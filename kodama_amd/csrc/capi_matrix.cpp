@@ -20,7 +20,7 @@
 #include "engine.h"
 #include "batch_api.h"
 #include "graph_launch.h"
-#include "knn_mfma.h"
+#include "knn_search.h"
 #include "launch.h"
 #include "matrix.h"
 #include "matrix_launch.h"

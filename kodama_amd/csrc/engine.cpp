@@ -13,7 +13,7 @@
 #include <omp.h>
 
 #include "capi_common.h"
-#include "knn_mfma.h"
+#include "knn_search.h"
 #include "launch.h"
 
 namespace kodama_hip {
@@ -732,8 +732,7 @@ KnnBatch::KnnBatch(int device, const float* x, int n, int p, const IVec& run_off
   job.d_pad_offsets = d_pad_off_.get();
   job.pad_total = pad_total_;
   job.max_rows = max_rows;
-  for (int f : folds) job.folds = std::max(job.folds, f + 1);
-  job.norm2_max = max_row_norm2(x, n, p);
+  job.d_block_run = d_block_run_.get();
   job.path = table_path;
   job.fallbacks = &last_knn_fallbacks();
   job.d_nbr = d_nbr_.get();

@@ -1,19 +1,14 @@
 // Host driver of the exact kNN on the device: matrix-core candidates with the
-// exact rerank where they apply (FP16 stream for searches, split BF16 for the
-// per-fold tables), the register scan otherwise and for the queries the
-// rerank flags.
+// exact rerank where they apply, the register scan otherwise and for the
+// queries the rerank flags.
 #include <algorithm>
 #include <atomic>
-#include <chrono>
 #include <functional>
-#include <map>
-#include <mutex>
-#include <tuple>
 #include <vector>
 
 #include "../../include/kodama_hip.h"
 #include "device.h"
-#include "knn_mfma.h"
+#include "knn_search.h"
 #include "knn_stream.h"
 #include "launch.h"
 
@@ -29,8 +24,35 @@ constexpr int kTableTargetBlocks = 2048; // sliced rescans of flagged table rows
 constexpr int kStreamMinTrain = 4096;     // smaller train sets use the register scan
 constexpr int kStreamWideQueries = 1024;  // queries beyond 64 dimensions for the matrix cores
 constexpr int kStreamTargetBlocks = 2048; // eight workgroups per CU
-constexpr int kStreamSliceRows = 1024;    // train rows per slice at least
+constexpr int kStreamSliceRows = 256;     // train rows per slice at least
 constexpr size_t kStreamCandBytes = size_t(1) << 30;  // candidate buffers per launch
+
+// How one pass is cut: slices of the candidates and of the maxima that bring
+// about eight workgroups per CU, each with at least kStreamSliceRows train
+// rows, the candidate buffers within kStreamCandBytes where slices allow it.
+struct StreamPlan {
+  int slices, max_slices, list, k;
+  size_t query_bytes;  // buffer of one query: its candidates, before them its maxima
+  StreamPlan(int query_rows, int train_rows, int k_, int list_, int steps) : list(list_), k(k_) {
+    const int per_block = 4 * stream_queries_per_wave(steps);
+    const int blocks = (query_rows + per_block - 1) / per_block;
+    const int want = std::min((kStreamTargetBlocks + blocks - 1) / blocks,
+                              std::min(kStreamMaxSlices, std::max(1, train_rows / kStreamSliceRows)));
+    const size_t list_bytes = static_cast<size_t>(stream_capacity(list)) * sizeof(uint2);
+    const size_t fit = kStreamCandBytes / (list_bytes * blocks * per_block);
+    slices = std::max(1, std::min(want, static_cast<int>(std::min<size_t>(fit, kStreamMaxSlices))));
+    max_slices = std::min(kStreamMaxSlices, std::max(stream_min_max_slices(k), want));
+    query_bytes = std::max(list_bytes * slices, static_cast<size_t>(max_slices) * 32 * sizeof(float));
+  }
+  void apply(KnnStreamParams& m, unsigned char* buffer) const {
+    m.slices = slices;
+    m.list = list;
+    m.sample_chunks = stream_sample_chunks(k);
+    m.max_slices = max_slices;
+    m.maxima = reinterpret_cast<float*>(buffer);  // read before the candidates are written
+    m.cand = reinterpret_cast<uint2*>(buffer);
+  }
+};
 
 }  // namespace
 
@@ -117,24 +139,13 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
       op.query_op = q_op.get();
       check(launch_stream_operands(op, s), "stream_operands launch");
     }
-    // Slices: about eight workgroups per CU in all, each scanning at least
-    // kStreamSliceRows rows, the candidate buffers within kStreamCandBytes.
-    const int per_block = 4 * stream_queries_per_wave(steps);
-    const int blocks = (rows + per_block - 1) / per_block;
-    const int most = std::min(kStreamMaxSlices, std::max(1, train_rows / kStreamSliceRows));
-    const int cap = stream_capacity(list);
-    const size_t row_bytes = static_cast<size_t>(cap) * sizeof(uint2);
-    int slices = std::min(most, (kStreamTargetBlocks + blocks - 1) / blocks);
-    slices = std::max(1, std::min(slices, static_cast<int>(kStreamCandBytes / (row_bytes * q_pad))));
-    const int max_slices =
-      std::min(kStreamMaxSlices, std::max(stream_min_max_slices(k), std::min(most, (kStreamTargetBlocks + blocks - 1) / blocks)));
-    // The maxima are read before the candidates are written: one buffer.
-    const size_t query_bytes = std::max(row_bytes * slices, static_cast<size_t>(max_slices) * 32 * sizeof(float));
+    const StreamPlan plan(rows, train_rows, k, list, steps);
+    const size_t query_bytes = plan.query_bytes;
     const size_t fit = kStreamCandBytes / query_bytes;
     const int batch = std::min(q_pad, static_cast<int>(std::max<size_t>(1, fit / kStreamBlockRows) * kStreamBlockRows));
     DeviceBuffer<unsigned char> cand(static_cast<size_t>(batch) * query_bytes);
     DeviceBuffer<float> threshold(static_cast<size_t>(batch));
-    DeviceBuffer<int> count(static_cast<size_t>(batch) * slices), flags(static_cast<size_t>(rows));
+    DeviceBuffer<int> count(static_cast<size_t>(batch) * plan.slices), flags(static_cast<size_t>(rows));
     DeviceBuffer<float> bound(count.size());
     KnnStreamParams m;
     m.train = d_train;
@@ -145,13 +156,8 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
     m.k = k;
     m.parts = parts;
     m.euclid = euclid ? 1 : 0;
-    m.slices = slices;
-    m.list = list;
-    m.sample_chunks = stream_sample_chunks(k);
-    m.max_slices = max_slices;
-    m.maxima = reinterpret_cast<float*>(cand.get());
+    plan.apply(m, cand.get());
     m.threshold = threshold.get();
-    m.cand = reinterpret_cast<uint2*>(cand.get());
     m.cand_count = count.get();
     m.cand_bound = bound.get();
     for (int q0 = 0; q0 < rows; q0 += batch) {
@@ -213,36 +219,15 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
 
 namespace {
 
-// Tuning cache of the per-fold tables: shape bucket -> the fastest schedule.
-struct TableShape {
-  int p, kmax, euclid, rows_log2, total_log2, folds;
-  bool operator<(const TableShape& o) const {
-    return std::tie(p, kmax, euclid, rows_log2, total_log2, folds) <
-           std::tie(o.p, o.kmax, o.euclid, o.rows_log2, o.total_log2, o.folds);
-  }
-};
-// Shapes the tuner does not time: the largest run and the landmark rows in
-// all runs at or above these take the MFMA path.
-constexpr int kMfmaSureRows = 2048;
-constexpr long long kMfmaSureTotal = 1ll << 16;
-std::mutex g_tune_mutex;
-std::map<TableShape, TableSchedule> g_tuned;
+// From this many rows in the largest run the matrix-core path builds the
+// tables: its ten launches cost about what the scan (a serial chain of one
+// distance after the other per query) needs for so many rows.
+constexpr int kTableStreamRows = 64;
+// Flagged rows that rerun the tables with three operand parts and the larger
+// buffers, in place of the scan.
+constexpr int kTableRerunShare = 16;
 std::atomic<int> g_table_path{0}, g_table_list{0}, g_table_waves{0};
 thread_local TableSchedule g_last_table;
-
-int ceil_log2(int v) {
-  int b = 0;
-  while ((1 << b) < v) ++b;
-  return b;
-}
-
-double seconds_of(const std::function<void()>& f, hipStream_t s) {
-  check(hipStreamSynchronize(s), "tuning sync");
-  const auto t0 = std::chrono::steady_clock::now();
-  f();
-  check(hipStreamSynchronize(s), "tuning sync");
-  return std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-}
 
 }  // namespace
 
@@ -261,189 +246,142 @@ int device_fold_tables(const FoldTableJob& job, hipStream_t s) {
   if (job.fallbacks) *job.fallbacks = -1;  // -1: the register scan served every row
   const int runs = static_cast<int>(job.run_offsets.size()) - 1;
   const int total = job.run_offsets[runs];
-  const bool mfma_ok = job.p <= 64 && job.k <= kMfmaMaxK;
+  const int forced = g_table_list.load();
+  const int narrow = stream_steps(job.p, 1, euclid);
+  // A forced list of 8 leaves k > 32 to the scan.
+  const bool stream_ok = narrow <= kStreamMaxSteps && job.k <= kStreamMaxK && !(forced == 8 && job.k > 32);
   int path = job.path != 0 ? job.path : g_table_path.load();
-  if (path == 2 && !mfma_ok) path = 1;
+  if (path == 0) path = job.max_rows >= kTableStreamRows ? 2 : 1;
+  if (path == 2 && !stream_ok) path = 1;
 
-  // Register scan of every row of every run, or of listed rows only.
-  auto scan = [&](const int* d_qlist, const int* d_qlist_offsets, int max_queries) {
-    KnnTopkParams prm;
-    prm.train = job.d_x;
-    prm.dims = job.p;
-    prm.k = job.k;
-    prm.rows = job.d_rows;
-    prm.folds = job.d_folds;
-    prm.run_offsets = job.d_run_offsets;
-    prm.pad_offsets = job.d_pad_offsets;
-    prm.pad_total = job.pad_total;
-    prm.qlist = d_qlist;
-    prm.qlist_offsets = d_qlist_offsets;
-    prm.out_index = job.d_nbr;
-    prm.out_dist = job.d_score;
-    check(launch_knn_topk(prm, 1, euclid, max_queries, runs, s), "knn_topk launch");
-  };
-  // Split-BF16 MFMA candidates (with `list` candidates per lane column and
-  // `waves` waves of queries per workgroup), exact rerank, the flagged rows
-  // rescanned.
-  auto mfma = [&](int list, int waves) {
-    DeviceBuffer<float> xc(static_cast<size_t>(total) * job.p);
-    check(launch_gather_rows(job.d_x, job.d_rows, total, job.p, xc.get(), s), "gather_rows launch");
-    DeviceBuffer<unsigned short> hi(static_cast<size_t>(total) * 64), lo(hi.size());
-    DeviceBuffer<float> n2(static_cast<size_t>(total));
-    check(launch_split_rows(xc.get(), total, job.p, hi.get(), lo.get(), n2.get(), s), "split_rows launch");
-    const size_t cand = static_cast<size_t>(total) * 16 * list;
-    DeviceBuffer<float> c_val(cand), r_dist(static_cast<size_t>(total) * job.k);
-    DeviceBuffer<int> c_idx(cand), flags(static_cast<size_t>(total)), r_idx(r_dist.size());
-    KnnMfmaParams m;
-    m.train = xc.get();
-    m.query = xc.get();
-    m.train_hi = m.query_hi = hi.get();
-    m.train_lo = m.query_lo = lo.get();
-    m.train_norm2 = m.query_norm2 = n2.get();
-    m.train_norm2_max = job.norm2_max;
+  KnnTopkParams scan;
+  scan.train = job.d_x;
+  scan.dims = job.p;
+  scan.k = job.k;
+  scan.rows = job.d_rows;
+  scan.folds = job.d_folds;
+  scan.run_offsets = job.d_run_offsets;
+  scan.pad_offsets = job.d_pad_offsets;
+  scan.pad_total = job.pad_total;
+  scan.out_index = job.d_nbr;
+  scan.out_dist = job.d_score;
+  if (path == 1) {
+    check(launch_knn_topk(scan, 1, euclid, job.max_rows, runs, s), "knn_topk launch");
+    g_last_table = TableSchedule{1, 0, 0};
+    return 1;
+  }
+
+  DeviceBuffer<float> xc(static_cast<size_t>(total) * job.p), n2(static_cast<size_t>(total)), n2_max(2);
+  DeviceBuffer<int> flags(static_cast<size_t>(total));
+  check(launch_gather_rows(job.d_x, job.d_rows, total, job.p, xc.get(), s), "gather_rows launch");
+  check(hipMemsetAsync(n2_max.get(), 0, 2 * sizeof(float), s), "memset");
+  check(launch_stream_norms(xc.get(), total, job.p, n2.get(), n2_max.get(), s), "stream_norms launch");
+  std::vector<int> h_flags(static_cast<size_t>(total));
+  auto pass = [&](int parts, int list) {
+    const int steps = stream_steps(job.p, parts, euclid);
+    DeviceBuffer<unsigned char> t_op(stream_operand_bytes(static_cast<size_t>(job.pad_total), steps)), q_op(t_op.size());
+    StreamOperandJob op;
+    op.x = xc.get();
+    op.norm2 = n2.get();
+    op.norm2_max = n2_max.get();
+    op.rows = total;
+    op.p = job.p;
+    op.parts = parts;
+    op.euclid = euclid ? 1 : 0;
+    op.pad_rows = job.pad_total;
+    op.block_run = job.d_block_run;
+    op.run_offsets = job.d_run_offsets;
+    op.pad_offsets = job.d_pad_offsets;
+    op.train_op = t_op.get();
+    op.query_op = q_op.get();
+    check(launch_stream_operands(op, s), "stream_operands launch");
+    const StreamPlan plan(job.pad_total, job.max_rows, job.k, list, steps);
+    DeviceBuffer<unsigned char> cand(static_cast<size_t>(job.pad_total) * plan.query_bytes);
+    DeviceBuffer<int> count(static_cast<size_t>(job.pad_total) * plan.slices);
+    DeviceBuffer<float> bound(count.size()), threshold(static_cast<size_t>(job.pad_total));
+    KnnStreamParams m;
+    m.train = m.query = xc.get();
+    m.train_op = t_op.get();
+    m.query_op = q_op.get();
+    m.query_norm2 = n2.get();
+    m.norm2_max = n2_max.get();
     m.train_rows = m.query_rows = total;
     m.dims = job.p;
     m.k = job.k;
+    m.parts = parts;
+    m.euclid = euclid ? 1 : 0;
+    m.block_run = job.d_block_run;
     m.run_offsets = job.d_run_offsets;
+    m.pad_offsets = job.d_pad_offsets;
     m.folds = job.d_folds;
-    m.cand_value = c_val.get();
-    m.cand_index = c_idx.get();
+    m.pad_rows = job.pad_total;
+    plan.apply(m, cand.get());
+    m.threshold = threshold.get();
+    m.cand_count = count.get();
+    m.cand_bound = bound.get();
     m.flags = flags.get();
-    m.out_index = r_idx.get();
-    m.out_dist = r_dist.get();
-    m.list = list;
-    m.waves = waves;
-    check(launch_knn_mfma_tables(m, euclid, runs, job.max_rows, s), "knn_mfma_tables launch");
-    check(launch_publish_tables(r_idx.get(), r_dist.get(), flags.get(), job.d_run_offsets, runs, job.d_pad_offsets,
-                                job.pad_total, total, job.k, job.d_nbr, job.d_score, s),
-          "publish_tables launch");
-    std::vector<int> h_flags(static_cast<size_t>(total));
+    m.out_index = job.d_nbr;
+    m.out_dist = job.d_score;
+    check(launch_knn_stream(m, s), "knn_stream launch");
     flags.download(h_flags.data(), h_flags.size(), s);
     check(hipStreamSynchronize(s), "fold tables sync");
-    std::vector<int> qlist, qrun, qoff(static_cast<size_t>(runs) + 1, 0);
-    int max_q = 0;
-    for (int r = 0; r < runs; ++r) {
-      for (int i = job.run_offsets[r]; i < job.run_offsets[r + 1]; ++i) {
-        if (h_flags[i]) {
-          qlist.push_back(i - job.run_offsets[r]);
-          qrun.push_back(r);
-        }
-      }
-      qoff[r + 1] = static_cast<int>(qlist.size());
-      max_q = std::max(max_q, qoff[r + 1] - qoff[r]);
-    }
-    const int nflag = static_cast<int>(qlist.size());
-    if (job.fallbacks) *job.fallbacks = nflag;
-    if (nflag == 0) return;
-    DeviceBuffer<int> d_ql(qlist.size()), d_qo(qoff.size()), d_qr(qrun.size());
-    d_ql.upload(qlist.data(), qlist.size(), s);
-    d_qo.upload(qoff.data(), qoff.size(), s);
-    d_qr.upload(qrun.data(), qrun.size(), s);
-    // A few flagged rows per run would leave one block per run scanning the
-    // whole run; their train rows are cut into slices (about 2048 blocks in
-    // all, at most 64 slices) whose lists are merged.
-    const int gx = (max_q + kScanBlock - 1) / kScanBlock;
-    int slices = std::min(kMaxSlices, std::max(1, (kTableTargetBlocks + gx * runs - 1) / (gx * runs)));
-    int slice_rows = (job.max_rows + slices - 1) / slices;
-    slice_rows = std::max(kSliceAlign, (slice_rows + kSliceAlign - 1) / kSliceAlign * kSliceAlign);
-    slices = (job.max_rows + slice_rows - 1) / slice_rows;
-    if (slices <= 1) {
-      scan(d_ql.get(), d_qo.get(), max_q);
-    } else {
-      DeviceBuffer<int> part_idx(static_cast<size_t>(slices) * nflag * job.k), m_idx(static_cast<size_t>(nflag) * job.k);
-      DeviceBuffer<float> part_dist(part_idx.size()), m_dist(m_idx.size());
-      KnnTopkParams prm;
-      prm.train = job.d_x;
-      prm.dims = job.p;
-      prm.k = job.k;
-      prm.rows = job.d_rows;
-      prm.folds = job.d_folds;
-      prm.run_offsets = job.d_run_offsets;
-      prm.pad_offsets = job.d_pad_offsets;
-      prm.pad_total = job.pad_total;
-      prm.qlist = d_ql.get();
-      prm.qlist_offsets = d_qo.get();
-      prm.list_total = nflag;
-      prm.slice_rows = slice_rows;
-      prm.out_index = part_idx.get();
-      prm.out_dist = part_dist.get();
-      check(launch_knn_topk(prm, 1, euclid, max_q, runs, s, slices), "knn_topk launch");
-      check(launch_knn_merge_slices(part_idx.get(), part_dist.get(), slices, nflag, job.k, m_idx.get(), m_dist.get(), s),
-            "knn_merge_slices launch");
-      check(launch_publish_listed(m_idx.get(), m_dist.get(), d_ql.get(), d_qr.get(), job.d_pad_offsets,
-                                  job.pad_total, nflag, job.k, job.d_nbr, job.d_score, s),
-            "publish_listed launch");
-    }
-    check(hipStreamSynchronize(s), "fold tables sync");
   };
+  int parts = stream_steps(job.p, 3, euclid) == narrow ? 3 : 1;
+  int list = forced != 0 ? forced : job.k <= 32 ? 8 : 16;
+  g_last_table = TableSchedule{2, list, g_table_waves.load() != 0 ? g_table_waves.load() : 4};
+  pass(parts, list);
+  const long long first = std::count(h_flags.begin(), h_flags.end(), 1);
+  const int wide = stream_steps(job.p, 3, euclid) <= kStreamMaxSteps ? 3 : 1;
+  if (first > total / kTableRerunShare && (wide != parts || list != 16)) pass(wide, 16);
 
-  // MFMA schedules: lists of 8 (k <= 32) and 16 candidates, 4 and 8 waves
-  // per workgroup; a forced list or wave count narrows them.
-  std::vector<TableSchedule> schedules;
-  for (int list : {8, 16}) {
-    if (list == 8 && job.k > 32) continue;
-    if (g_table_list.load() != 0 && list != g_table_list.load()) continue;
-    for (int waves : {8, 4}) {
-      if (g_table_waves.load() != 0 && waves != g_table_waves.load()) continue;
-      schedules.push_back(TableSchedule{2, list, waves});
-    }
-  }
-  // A forced list that the job's k excludes leaves the scan.
-  const bool mfma_usable = mfma_ok && !schedules.empty();
-  TableSchedule choice{path == 2 && !mfma_usable ? 1 : path, 0, 0};
-  if (path == 0) {
-    if (!mfma_usable) {
-      choice = TableSchedule{1, 0, 0};
-    } else {
-      // k enters by its power-of-two bucket (8, 16, 32, 64, 128): the
-      // schedules open to a k differ across 32 (lists of 8 need k <= 32).
-      const TableShape key{job.p, 1 << std::max(3, ceil_log2(job.k)), euclid ? 1 : 0, ceil_log2(job.max_rows),
-                           ceil_log2(total), job.folds};
-      bool cached = false;
-      {
-        std::lock_guard<std::mutex> lock(g_tune_mutex);
-        auto it = g_tuned.find(key);
-        if (it != g_tuned.end()) {
-          choice = it->second;
-          cached = true;
-        }
-      }
-      if (!cached) {
-        // First use of this shape bucket: time every candidate schedule (they
-        // give identical tables) and keep the fastest. Runs this large sit
-        // well inside the region where the MFMA path measured several times
-        // faster than the scan (7.1 against 29.7 ms for 100 runs of
-        // 1000-5000 rows, p = 50, k = 30): the scan is not timed there.
-        const bool sure = job.max_rows >= kMfmaSureRows && total >= kMfmaSureTotal;
-        double best = 0.0;
-        if (!sure) {
-          best = seconds_of([&] { scan(nullptr, nullptr, job.max_rows); }, s);
-          choice = TableSchedule{1, 0, 0};
-        }
-        for (const TableSchedule& t : schedules) {
-          const double sec = seconds_of([&] { mfma(t.list, t.waves); }, s);
-          if (choice.path == 0 || sec < best) {
-            best = sec;
-            choice = t;
-          }
-        }
-        std::lock_guard<std::mutex> lock(g_tune_mutex);
-        g_tuned[key] = choice;
-        g_last_table = choice;
-        return choice.path;
+  std::vector<int> qlist, qrun, qoff(static_cast<size_t>(runs) + 1, 0);
+  int max_q = 0;
+  for (int r = 0; r < runs; ++r) {
+    for (int i = job.run_offsets[r]; i < job.run_offsets[r + 1]; ++i) {
+      if (h_flags[i]) {
+        qlist.push_back(i - job.run_offsets[r]);
+        qrun.push_back(r);
       }
     }
-  } else if (choice.path == 2) {
-    choice = schedules.front();
+    qoff[r + 1] = static_cast<int>(qlist.size());
+    max_q = std::max(max_q, qoff[r + 1] - qoff[r]);
   }
-  if (choice.path == 2) {
-    mfma(choice.list, choice.waves);
-  } else {
-    choice = TableSchedule{1, 0, 0};
-    scan(nullptr, nullptr, job.max_rows);
+  const int nflag = static_cast<int>(qlist.size());
+  if (job.fallbacks) *job.fallbacks = nflag;
+  if (nflag == 0) return 2;
+  DeviceBuffer<int> d_ql(qlist.size()), d_qo(qoff.size()), d_qr(qrun.size());
+  d_ql.upload(qlist.data(), qlist.size(), s);
+  d_qo.upload(qoff.data(), qoff.size(), s);
+  d_qr.upload(qrun.data(), qrun.size(), s);
+  // A few flagged rows per run would leave one block per run scanning the
+  // whole run; their train rows are cut into slices (about 2048 blocks in
+  // all, at most 64 slices) whose lists are merged.
+  const int gx = (max_q + kScanBlock - 1) / kScanBlock;
+  int slices = std::min(kMaxSlices, std::max(1, (kTableTargetBlocks + gx * runs - 1) / (gx * runs)));
+  int slice_rows = (job.max_rows + slices - 1) / slices;
+  slice_rows = std::max(kSliceAlign, (slice_rows + kSliceAlign - 1) / kSliceAlign * kSliceAlign);
+  slices = (job.max_rows + slice_rows - 1) / slice_rows;
+  scan.qlist = d_ql.get();
+  scan.qlist_offsets = d_qo.get();
+  if (slices <= 1) {
+    check(launch_knn_topk(scan, 1, euclid, max_q, runs, s), "knn_topk launch");
+    check(hipStreamSynchronize(s), "fold tables sync");
+    return 2;
   }
-  g_last_table = choice;
-  return choice.path;
+  DeviceBuffer<int> part_idx(static_cast<size_t>(slices) * nflag * job.k), m_idx(static_cast<size_t>(nflag) * job.k);
+  DeviceBuffer<float> part_dist(part_idx.size()), m_dist(m_idx.size());
+  scan.list_total = nflag;
+  scan.slice_rows = slice_rows;
+  scan.out_index = part_idx.get();
+  scan.out_dist = part_dist.get();
+  check(launch_knn_topk(scan, 1, euclid, max_q, runs, s, slices), "knn_topk launch");
+  check(launch_knn_merge_slices(part_idx.get(), part_dist.get(), slices, nflag, job.k, m_idx.get(), m_dist.get(), s),
+        "knn_merge_slices launch");
+  check(launch_publish_listed(m_idx.get(), m_dist.get(), d_ql.get(), d_qr.get(), job.d_pad_offsets, job.pad_total,
+                              nflag, job.k, job.d_nbr, job.d_score, s),
+        "publish_listed launch");
+  check(hipStreamSynchronize(s), "fold tables sync");
+  return 2;
 }
 
 }  // namespace kodama_hip

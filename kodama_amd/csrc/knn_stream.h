@@ -60,8 +60,8 @@ struct KnnStreamParams {
   int* cand_count = nullptr;        // [query rows][slices], -1 = overflowed
   float* cand_bound = nullptr;      // [query rows][slices] scores below it were dropped
   int* flags = nullptr;             // [query rows] 1 = needs another path
-  int* out_index = nullptr;         // [query rows x k]
-  float* out_dist = nullptr;
+  int* out_index = nullptr;         // [query rows x k]; tables: the vote layout [k x pad_rows]
+  float* out_dist = nullptr;        // internal distances; tables: scores (minus the distance)
 };
 
 // Squared norms [rows] and their maximum (into *norm2_max, which the caller

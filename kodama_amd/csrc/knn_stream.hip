@@ -665,21 +665,13 @@ __global__ void __launch_bounds__(256) knn_stream_rerank_kernel(KnnStreamParams 
   __shared__ uint2 s_ent[4][kStreamMerge];
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
-  const int q = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + wave);
-  if (q >= prm.query_rows) return;  // whole waves; no block barrier below
+  const int op_row = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + wave);
   const int k = prm.k, p = prm.dims, cap = 16 * prm.list;
-  int op_row = q;  // operand (padded) row of a table query
-  if (prm.block_run != nullptr) {
-    int lo = 0, hi = prm.pad_rows / kStreamBlockRows - 1;
-    // The run of concatenated row q: block_run is ascending over the padded
-    // blocks, so search the runs through it.
-    hi = prm.block_run[hi];
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (prm.run_offsets[mid] <= q) lo = mid; else hi = mid - 1;
-    }
-    op_row = prm.pad_offsets[lo] + (q - prm.run_offsets[lo]);
-  }
+  const bool tables = prm.block_run != nullptr;
+  if (op_row >= (tables ? prm.pad_rows : prm.query_rows)) return;  // whole waves; no block barrier below
+  const StreamRange g = stream_range(prm, op_row);
+  if (op_row >= g.q_end) return;
+  const int q = op_row + g.delta;
   uint2* ent = s_ent[wave];
   const uint64_t below = (1ull << lane) - 1ull;
   // Merge: what scores at or above the tightest slice's bound.
@@ -754,8 +746,11 @@ __global__ void __launch_bounds__(256) knn_stream_rerank_kernel(KnnStreamParams 
   }
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  int* out_i = prm.out_index + static_cast<size_t>(q) * k;
-  float* out_d = prm.out_dist + static_cast<size_t>(q) * k;
+  // [query x k] rows and distances; for tables the transposed vote layout
+  // [k x pad_rows]: padded rows and scores (minus the distance).
+  const size_t step = tables ? static_cast<size_t>(prm.pad_rows) : 1;
+  int* out_i = prm.out_index + (tables ? static_cast<size_t>(op_row) : static_cast<size_t>(q) * k);
+  float* out_d = prm.out_dist + (tables ? static_cast<size_t>(op_row) : static_cast<size_t>(q) * k);
   for (int e = lane; e < n; e += kWave) {
     const uint2 v = ent[e];
     const float d = __uint_as_float(v.x);
@@ -766,13 +761,13 @@ __global__ void __launch_bounds__(256) knn_stream_rerank_kernel(KnnStreamParams 
       rank += od < d || (od == d && o.y < v.y) ? 1 : 0;
     }
     if (rank < k) {
-      out_i[rank] = static_cast<int>(v.y);
-      out_d[rank] = d;
+      out_i[rank * step] = static_cast<int>(v.y) - (tables ? g.delta : 0);
+      out_d[rank * step] = tables ? -d : d;
     }
   }
   for (int t = n + lane; t < k; t += kWave) {
-    out_i[t] = -1;
-    out_d[t] = INFINITY;
+    out_i[t * step] = -1;
+    out_d[t * step] = tables ? -INFINITY : INFINITY;
   }
 }
 
@@ -836,7 +831,7 @@ hipError_t launch_knn_stream(const KnnStreamParams& prm, hipStream_t s) {
     case 8: launch_steps<8>(prm, s); break;
     default: launch_steps<9>(prm, s); break;
   }
-  const unsigned rblocks = static_cast<unsigned>((prm.query_rows + 3) / 4);
+  const unsigned rblocks = static_cast<unsigned>(((prm.block_run != nullptr ? prm.pad_rows : prm.query_rows) + 3) / 4);
   if (prm.euclid) hipLaunchKernelGGL((knn_stream_rerank_kernel<true>), dim3(rblocks), dim3(256), 0, s, prm);
   else hipLaunchKernelGGL((knn_stream_rerank_kernel<false>), dim3(rblocks), dim3(256), 0, s, prm);
   return hipGetLastError();

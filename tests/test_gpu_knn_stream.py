@@ -77,3 +77,57 @@ def test_outlying_rows_loosen_the_bound_but_not_the_result(oracle):
     x, _ = D.config3(n=5000, p=50, seed=12)
     x[40] *= 1000.0
     _check(oracle, x[:4900], x[4900:], 20, "euclidean", most=100)
+
+
+def _uneven(x, sizes, folds, seed):
+    """Runs whose first fold holds nine rows in ten."""
+    rng = np.random.default_rng(seed)
+    rows, fids = [], []
+    for n in sizes:
+        rows.append(np.sort(rng.choice(x.shape[0], n, replace=False)).astype(np.int32))
+        f = np.where(rng.random(n) < 0.9, 0, rng.integers(0, folds, n)).astype(np.int32)
+        f[:folds] = np.arange(folds)
+        fids.append(f)
+    return rows, fids
+
+
+# Run sizes at the edges of a chunk (64), the padding (256) and a slice; wide
+# rows; a fold that leaves a query few candidates (fewer than k in the small
+# runs); every k class.
+@pytest.mark.parametrize("p", [2, 21, 65, 200])
+@pytest.mark.parametrize("k", [1, 32, 33, 64])
+def test_fold_tables_match_oracle(oracle, p, k):
+    x, _ = D.config3(n=2500, p=p, seed=p + k)
+    rows, fids = _uneven(x, [64, 3, 255, 256, 257, 63, 1025], folds=3, seed=k)
+    for name in ("euclidean", "cosine"):
+        nbr, score, used = K.knn_fold_tables(x, rows, fids, k, name, path="mfma")
+        assert used == "mfma"
+        for r, (rw, f) in enumerate(zip(rows, fids)):
+            wn, ws = oracle.precompute_knn_cv(x[rw], f, k, K._metric(name))
+            assert np.array_equal(nbr[r], wn), (name, r)
+            assert np.array_equal(score[r], ws), (name, r)
+
+
+def test_fold_tables_rule_by_run_size(oracle):
+    """The scan below 64 rows in the largest run, the matrix cores from there."""
+    x, _ = D.config3(n=400, p=12, seed=1)
+    for n, path in ((63, "scan"), (64, "mfma")):
+        rows, fids = _uneven(x, [n, 20], folds=4, seed=n)
+        nbr, score, used = K.knn_fold_tables(x, rows, fids, 6, "euclidean")
+        assert used == path
+        for r, (rw, f) in enumerate(zip(rows, fids)):
+            wn, ws = oracle.precompute_knn_cv(x[rw], f, 6, 2)
+            assert np.array_equal(nbr[r], wn) and np.array_equal(score[r], ws)
+
+
+def test_fold_tables_of_equal_rows(oracle):
+    """Forty copies of each row fill no buffer; 300 copies fill them all, the
+    wider second pass too, and the scan answers."""
+    base, _ = D.config3(n=6, p=30, seed=4)
+    for copies in (40, 300):
+        x = np.repeat(base, copies, axis=0)
+        rows, fids = [np.arange(x.shape[0], dtype=np.int32)], [(np.arange(x.shape[0]) % 5).astype(np.int32)]
+        nbr, score, _ = K.knn_fold_tables(x, rows, fids, 20, "euclidean", path="mfma")
+        assert (K.last_knn_fallbacks() == 0) == (copies == 40)
+        wn, ws = oracle.precompute_knn_cv(x, fids[0], 20, 2)
+        assert np.array_equal(nbr[0], wn) and np.array_equal(score[0], ws)
