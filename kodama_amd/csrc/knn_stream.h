@@ -68,14 +68,15 @@ struct KnnStreamParams {
 // cleared to 0).
 hipError_t launch_stream_norms(const float* x, int rows, int p, float* norm2, float* norm2_max, hipStream_t s);
 // Rows -> operand fragments of `steps` x 32 columns, rows padded with zeros to
-// a multiple of 256; either output may be null. norm2_max [2] scales them.
+// pad_rows; either output may be null. norm2_max [2] scales them.
 // For the padded table layout pass block_run / run_offsets / pad_offsets.
 struct StreamOperandJob {
   const float* x = nullptr;
   const float* norm2 = nullptr;
   const float* norm2_max = nullptr;
   int rows = 0, p = 0, parts = 1, euclid = 0;
-  int pad_rows = 0;                 // multiple of 256
+  int pad_rows = 0;                 // multiple of 16
+  int group_rows = 0, group_pad = 0;  // equal groups of group_rows rows, padded to group_pad (0: one group)
   const int* block_run = nullptr;   // tables: run of each 256 padded rows
   const int* run_offsets = nullptr;
   const int* pad_offsets = nullptr;

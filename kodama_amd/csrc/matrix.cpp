@@ -13,6 +13,7 @@
 #include <stdexcept>
 
 #include "device.h"
+#include "knn_stream.h"
 #include "matrix_launch.h"
 
 namespace kodama_hip {
@@ -108,6 +109,86 @@ void split_empty_clusters(int rows, int p, int k, std::vector<float>& sizes, std
 
 }  // namespace
 
+namespace {
+
+// Device state of `runs` k-means problems of n rows and k clusters: the score
+// operands of the rows are made once, those of the centroids per assignment.
+struct DeviceLloyd {
+  const float* d_x;
+  int runs, n, p, k, parts, steps, pad_n, pad_k;
+  hipStream_t s;
+  DeviceBuffer<float> xn, cent, cn, sizes, norm2_max;
+  DeviceBuffer<int> asg, changed, offsets, members;
+  DeviceBuffer<unsigned char> row_op, cent_op;
+
+  DeviceLloyd(const float* x, int runs_, int n_, int p_, int k_, hipStream_t stream)
+      : d_x(x), runs(runs_), n(n_), p(p_), k(k_), s(stream), xn(static_cast<size_t>(runs) * n),
+        cent(static_cast<size_t>(runs) * k * p), cn(static_cast<size_t>(runs) * k), sizes(cn.size()), norm2_max(2),
+        asg(xn.size()), changed(static_cast<size_t>(runs)),
+        offsets(static_cast<size_t>(runs) * k * kmeans_segments(n)), members(xn.size()) {
+    // Three FP16 parts where they are as wide as one.
+    parts = stream_steps(p, 3, true) == stream_steps(p, 1, true) ? 3 : 1;
+    steps = stream_steps(p, parts, true);
+    pad_n = (n + 15) / 16 * 16;
+    pad_k = (k + 63) / 64 * 64;
+    row_op.resize(stream_operand_bytes(static_cast<size_t>(runs) * pad_n, steps));
+    cent_op.resize(stream_operand_bytes(static_cast<size_t>(runs) * pad_k, steps));
+    check(launch_sse_norms(d_x, runs * n, p, xn.get(), s), "sse_norms launch");
+    check(hipMemsetAsync(asg.get(), 0xFF, sizeof(int) * asg.size(), s), "memset");  // -1: unassigned
+    check(hipMemsetAsync(norm2_max.get(), 0, 2 * sizeof(float), s), "memset");
+    check(launch_norms_max(xn.get(), xn.size(), norm2_max.get(), s), "norms_max launch");
+    StreamOperandJob op = operand_job(d_x, xn.get(), n, pad_n);
+    op.query_op = row_op.get();
+    check(launch_stream_operands(op, s), "stream_operands launch");
+  }
+  StreamOperandJob operand_job(const float* x, const float* norm2, int rows, int pad) const {
+    StreamOperandJob op;
+    op.x = x;
+    op.norm2 = norm2;
+    op.norm2_max = norm2_max.get();
+    op.p = p;
+    op.parts = parts;
+    op.euclid = 1;
+    op.pad_rows = runs * pad;
+    op.group_rows = rows;
+    op.group_pad = pad;
+    return op;
+  }
+  // Assignment to the centroids in `cent`; counts the changes.
+  void assign(const int* active) {
+    check(launch_sse_norms(cent.get(), runs * k, p, cn.get(), s), "sse_norms launch");
+    StreamOperandJob op = operand_job(cent.get(), cn.get(), k, pad_k);
+    op.train_op = cent_op.get();
+    check(launch_stream_operands(op, s), "stream_operands launch");
+    check(hipMemsetAsync(changed.get(), 0, sizeof(int) * changed.size(), s), "memset");
+    KmeansAssignParams a;
+    a.x = d_x;
+    a.n = n;
+    a.p = p;
+    a.x_norm = xn.get();
+    a.centroids = cent.get();
+    a.c_norm = cn.get();
+    a.k = k;
+    a.assign = asg.get();
+    a.changed = changed.get();
+    a.active = active;
+    a.row_op = row_op.get();
+    a.centroid_op = cent_op.get();
+    a.norm2_max = norm2_max.get();
+    a.parts = parts;
+    a.pad_n = pad_n;
+    a.pad_k = pad_k;
+    check(launch_kmeans_assign(a, s, runs), "kmeans_assign launch");
+  }
+  void update(const int* active) {
+    check(launch_kmeans_update(d_x, n, p, asg.get(), k, offsets.get(), members.get(), cent.get(), sizes.get(), s, runs,
+                               active),
+          "kmeans_update launch");
+  }
+};
+
+}  // namespace
+
 IVec device_kmeans(const float* h_x, const float* d_x, int n, int p, int k, std::mt19937_64& rng, int max_iter,
                    hipStream_t s) {
   k = std::max(1, std::min(k, n));
@@ -115,34 +196,27 @@ IVec device_kmeans(const float* h_x, const float* d_x, int n, int p, int k, std:
   const IVec order = seed_order(n, kseed + 1u);
   std::vector<float> cent(static_cast<size_t>(k) * p), sizes(static_cast<size_t>(k));
   for (int c = 0; c < k; ++c) std::copy_n(h_x + static_cast<size_t>(order[c]) * p, p, cent.data() + static_cast<size_t>(c) * p);
-  DeviceBuffer<float> d_xn(static_cast<size_t>(n)), d_cent(cent.size()), d_cn(static_cast<size_t>(k)),
-    d_sizes(static_cast<size_t>(k));
-  DeviceBuffer<int> d_asg(static_cast<size_t>(n)), d_changed(1);
-  check(launch_sse_norms(d_x, n, p, d_xn.get(), s), "sse_norms launch");
-  check(hipMemsetAsync(d_asg.get(), 0xFF, sizeof(int) * d_asg.size(), s), "memset");  // -1: unassigned
+  DeviceLloyd dev(d_x, 1, n, p, k, s);
   auto assign = [&]() {
-    d_cent.upload(cent.data(), cent.size(), s);
-    check(launch_sse_norms(d_cent.get(), k, p, d_cn.get(), s), "sse_norms launch");
-    check(hipMemsetAsync(d_changed.get(), 0, sizeof(int), s), "memset");
-    check(launch_kmeans_assign(d_x, n, p, d_xn.get(), d_cent.get(), d_cn.get(), k, d_asg.get(), d_changed.get(), s),
-          "kmeans_assign launch");
+    dev.cent.upload(cent.data(), cent.size(), s);
+    dev.assign(nullptr);
     int changed = 0;
-    d_changed.download(&changed, 1, s);
+    dev.changed.download(&changed, 1, s);
     check(hipStreamSynchronize(s), "kmeans sync");
     return changed;
   };
   for (int it = 0; it < std::max(1, max_iter); ++it) {
     const int changed = assign();
-    check(launch_kmeans_update(d_x, n, p, d_asg.get(), k, d_cent.get(), d_sizes.get(), s), "kmeans_update launch");
-    d_cent.download(cent.data(), cent.size(), s);
-    d_sizes.download(sizes.data(), sizes.size(), s);
+    dev.update(nullptr);
+    dev.cent.download(cent.data(), cent.size(), s);
+    dev.sizes.download(sizes.data(), sizes.size(), s);
     check(hipStreamSynchronize(s), "kmeans sync");
     split_empty_clusters(n, p, k, sizes, cent);
     if (changed == 0) break;
   }
   assign();
   IVec labels(static_cast<size_t>(n));
-  d_asg.download(labels.data(), labels.size(), s);
+  dev.asg.download(labels.data(), labels.size(), s);
   check(hipStreamSynchronize(s), "kmeans sync");
   for (int& l : labels) ++l;
   return labels;
@@ -161,12 +235,8 @@ std::vector<IVec> device_kmeans_batch(const float* h_x, const int* rows, const f
       std::copy_n(h_x + static_cast<size_t>(data_row) * p, p, cent.data() + r * kp + static_cast<size_t>(c) * p);
     }
   }
-  DeviceBuffer<float> d_xn(static_cast<size_t>(runs) * n), d_cent(cent.size()), d_cn(static_cast<size_t>(runs) * k),
-    d_sizes(sizes.size());
-  DeviceBuffer<int> d_asg(static_cast<size_t>(runs) * n), d_changed(static_cast<size_t>(runs)),
-    d_active(static_cast<size_t>(runs));
-  check(launch_sse_norms(d_rows, runs * n, p, d_xn.get(), s), "sse_norms launch");
-  check(hipMemsetAsync(d_asg.get(), 0xFF, sizeof(int) * d_asg.size(), s), "memset");  // -1: unassigned
+  DeviceLloyd dev(d_rows, runs, n, p, k, s);
+  DeviceBuffer<int> d_active(static_cast<size_t>(runs));
   // Phase of each problem: Lloyd rounds (assign, update, split), then one
   // final assignment with the last centroids, then done.
   enum Phase { kLoop, kFinal, kDone };
@@ -179,14 +249,10 @@ std::vector<IVec> device_kmeans_batch(const float* h_x, const int* rows, const f
       any = any || act[r];
     }
     if (!any) break;
-    d_cent.upload(cent.data(), cent.size(), s);
-    check(launch_sse_norms(d_cent.get(), runs * k, p, d_cn.get(), s), "sse_norms launch");
-    check(hipMemsetAsync(d_changed.get(), 0, sizeof(int) * runs, s), "memset");
+    dev.cent.upload(cent.data(), cent.size(), s);
     d_active.upload(act.data(), act.size(), s);
-    check(launch_kmeans_assign(d_rows, n, p, d_xn.get(), d_cent.get(), d_cn.get(), k, d_asg.get(), d_changed.get(), s,
-                               runs, d_active.get()),
-          "kmeans_assign launch");
-    d_changed.download(changed.data(), changed.size(), s);
+    dev.assign(d_active.get());
+    dev.changed.download(changed.data(), changed.size(), s);
     check(hipStreamSynchronize(s), "kmeans sync");  // act and changed are reused below
     bool update = false;
     for (int r = 0; r < runs; ++r) {
@@ -195,10 +261,9 @@ std::vector<IVec> device_kmeans_batch(const float* h_x, const int* rows, const f
     }
     if (update) {
       d_active.upload(act.data(), act.size(), s);
-      check(launch_kmeans_update(d_rows, n, p, d_asg.get(), k, d_cent.get(), d_sizes.get(), s, runs, d_active.get()),
-            "kmeans_update launch");
-      d_cent.download(cent.data(), cent.size(), s);
-      d_sizes.download(sizes.data(), sizes.size(), s);
+      dev.update(d_active.get());
+      dev.cent.download(cent.data(), cent.size(), s);
+      dev.sizes.download(sizes.data(), sizes.size(), s);
       check(hipStreamSynchronize(s), "kmeans sync");
 #pragma omp parallel for schedule(dynamic)
       for (int r = 0; r < runs; ++r) {
@@ -219,7 +284,7 @@ std::vector<IVec> device_kmeans_batch(const float* h_x, const int* rows, const f
     }
   }
   std::vector<int> flat(static_cast<size_t>(runs) * n);
-  d_asg.download(flat.data(), flat.size(), s);
+  dev.asg.download(flat.data(), flat.size(), s);
   check(hipStreamSynchronize(s), "kmeans sync");
   std::vector<IVec> labels(static_cast<size_t>(runs));
   for (int r = 0; r < runs; ++r) {

@@ -12,21 +12,48 @@ namespace kodama_hip {
 // out[r] = dot(x_r, x_r) in the reference's float order (see matrix_kernels.hip).
 hipError_t launch_sse_norms(const float* x, int rows, int p, float* out, hipStream_t s);
 
+// *out = max(*out, the largest of the norms); the caller cleared *out.
+hipError_t launch_norms_max(const float* norms, size_t count, float* out, hipStream_t s);
+
 // Nearest centroid of every row (smallest (|x|^2 + |c|^2) - 2 x.c, first
 // cluster on ties); rows whose assignment changes are counted in *changed.
 // With runs > 1, `runs` problems of n rows and k clusters each, laid out one
 // after another (x, x_norm, centroids, c_norm, assign, changed strided by
 // problem), solved by one launch; active (may be null) skips problems whose
-// entry is 0.
-hipError_t launch_kmeans_assign(const float* x, int n, int p, const float* x_norm, const float* centroids,
-                                const float* c_norm, int k, int* assign, int* changed, hipStream_t s,
-                                int runs = 1, const int* active = nullptr);
+// entry is 0. row_op / centroid_op: score operands (knn_stream.h) of the rows
+// and the centroids, Euclidean, `parts` parts, each problem's rows padded to
+// pad_n (a multiple of 16) and its centroids to pad_k (a multiple of 64).
+struct KmeansAssignParams {
+  const float* x = nullptr;
+  int n = 0, p = 0;
+  const float* x_norm = nullptr;
+  const float* centroids = nullptr;
+  const float* c_norm = nullptr;
+  int k = 0;
+  int* assign = nullptr;
+  int* changed = nullptr;
+  const int* active = nullptr;
+  const void* row_op = nullptr;
+  const void* centroid_op = nullptr;
+  const float* norm2_max = nullptr;  // [2]: the largest row norm, 0
+  int parts = 1, pad_n = 0, pad_k = 0;
+};
+hipError_t launch_kmeans_assign(const KmeansAssignParams& prm, hipStream_t s, int runs = 1);
 
 // Per cluster: member rows summed in ascending row order, then scaled by
 // 1 / count (clusters without members stay zero); sizes as float counts.
-// Batched as launch_kmeans_assign.
-hipError_t launch_kmeans_update(const float* x, int n, int p, const int* assign, int k, float* centroids,
-                                float* sizes, hipStream_t s, int runs = 1, const int* active = nullptr);
+// Batched as launch_kmeans_assign. Workspaces: offsets [runs x k x
+// kmeans_segments(n)], members [runs x n].
+int kmeans_segments(int n);
+hipError_t launch_kmeans_update(const float* x, int n, int p, const int* assign, int k, int* offsets, int* members,
+                                float* centroids, float* sizes, hipStream_t s, int runs = 1,
+                                const int* active = nullptr);
+
+// Runs per row of the projection's table (whole 64-lane groups) and the most
+// landmarks whose positions fit 16 bits.
+inline int project_run_stride(int runs) { return (runs + 63) / 64 * 64; }
+constexpr int kProjectNarrow = 65535;
+size_t project_local_bytes(int n, int runs, int max_landmarks);
 
 struct ProjectParams {
   const int* graph = nullptr;        // [n x neighbors] 0-based ids, -1 = none
@@ -38,14 +65,15 @@ struct ProjectParams {
   int runs = 0;
   int votes = 0;                     // most landmark neighbours that vote (1..64)
   int max_landmarks = 0;             // largest run's landmark count
-  int* local = nullptr;              // workspace [runs x n]: landmark position of each row, or -1
+  void* local = nullptr;             // workspace [n x run_stride], project_local_bytes: landmark position or -1
+  int run_stride = 0;                // project_run_stride(runs)
   int* res = nullptr;                // [runs x n]
 };
 
 // res[r][i]: the landmark's own label, else the majority label (smallest on
 // ties) of the first `votes` landmarks in row i's graph neighbours, else the
-// run's first landmark label. Fills prm.local first (row -> position in the
-// run's landmark list), so each lookup is one load.
+// run's first landmark label. Fills prm.local first (row and run -> position in
+// the run's landmark list).
 hipError_t launch_project(const ProjectParams& prm, hipStream_t s);
 
 }  // namespace kodama_hip
