@@ -2,6 +2,7 @@
 #include "capi_common.h"
 
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <vector>
 
@@ -12,7 +13,52 @@ thread_local std::string g_last_error;
 thread_local int g_knn_fallbacks = -1;
 std::mutex g_arch_mutex;
 std::vector<int> g_arch_ok;  // -1 unknown, 0 not gfx950, 1 gfx950
+
+// Idle streams by device; never destroyed at exit (the runtime may be gone).
+struct IdleStreams {
+  std::mutex mutex;
+  std::map<int, std::vector<hipStream_t>> by_device;
+};
+IdleStreams& idle_streams() {
+  static IdleStreams* const pool = new IdleStreams;
+  return *pool;
+}
 }  // namespace
+
+hipStream_t take_stream(int device) {
+  IdleStreams& pool = idle_streams();
+  {
+    std::lock_guard<std::mutex> lock(pool.mutex);
+    std::vector<hipStream_t>& idle = pool.by_device[device];
+    if (!idle.empty()) {
+      const hipStream_t s = idle.back();
+      idle.pop_back();
+      return s;
+    }
+  }
+  hipStream_t s = nullptr;
+  check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
+  return s;
+}
+
+void give_stream(int device, hipStream_t s) {
+  // A call that failed may leave work behind: wait for it. A stream that
+  // cannot be waited for (a broken capture, a device error) is not used again.
+  const bool idle_now = hipStreamSynchronize(s) == hipSuccess;
+  if (idle_now) {
+    pool_settle(device, s);
+    IdleStreams& pool = idle_streams();
+    std::lock_guard<std::mutex> lock(pool.mutex);
+    std::vector<hipStream_t>& idle = pool.by_device[device];
+    if (idle.size() < kIdleStreams) {
+      idle.push_back(s);
+      return;
+    }
+  } else {
+    pool_drop(device, s);
+  }
+  (void)hipStreamDestroy(s);
+}
 
 void set_last_error(const std::string& msg) { g_last_error = msg; }
 

@@ -10,6 +10,7 @@
 #include "capi_common.h"
 #include "engine.h"
 #include "graph_launch.h"
+#include "host_pages.h"
 #include "knn_search.h"
 #include "launch.h"
 
@@ -36,7 +37,11 @@ int kodama_hip_knn_graph(const float* x, int32_t n, int32_t p, int32_t k, int32_
             "graph neighbours above 128 (above 64 beyond 128 feature columns) are not supported by the HIP kNN kernel.");
     require(p <= kMaxDims, "the HIP kNN kernel supports 1..256 feature columns.");
     select_device(device);
+    PageWarmer pages;
+    pages.add(indices_one_based, static_cast<size_t>(n) * kk * sizeof(int32_t));
+    pages.add(distances, static_cast<size_t>(n) * kk * sizeof(float));
     Stream st(device);
+    const StreamScope scope(st);
     const hipStream_t s = st.get();
     DeviceBuffer<float> d_x(static_cast<size_t>(n) * p);
     DeviceBuffer<int> d_ex(static_cast<size_t>(n));
@@ -52,6 +57,7 @@ int kodama_hip_knn_graph(const float* x, int32_t n, int32_t p, int32_t k, int32_
     device_exact_knn(d_x.get(), n, d_x.get(), n, p, kk, metric, d_ex.get(), d_idx.get(), d_dist.get(),
                      s, &last_knn_fallbacks());
     check(launch_graph_publish(d_idx.get(), d_dist.get(), d_idx.size(), metric, s), "graph_publish launch");
+    pages.wait();
     d_idx.download(indices_one_based, d_idx.size(), s);
     d_dist.download(distances, d_dist.size(), s);
     st.sync();
@@ -66,6 +72,7 @@ int kodama_hip_dissimilarity_inplace(int32_t* indices_one_based, float* distance
     require(dissimilarity_lds_bytes(neighbors) <= 64 * 1024, "dissimilarity supports up to 1365 neighbours per row.");
     select_device(device);
     Stream st(device);
+    const StreamScope scope(st);
     const hipStream_t s = st.get();
     const int stride = (runs + 3) / 4 * 4;
     const size_t edges = static_cast<size_t>(samples) * neighbors;
@@ -144,6 +151,7 @@ int kodama_hip_graph_build(const float* x, int32_t n, int32_t p, int32_t k, int3
     g->idx.resize(static_cast<size_t>(n) * kk);
     g->dist.resize(static_cast<size_t>(n) * kk);
     Stream st(device);
+    const StreamScope scope(st);
     const hipStream_t s = st.get();
     DeviceBuffer<float> d_x(static_cast<size_t>(n) * p);
     DeviceBuffer<int> d_ex(static_cast<size_t>(n));
@@ -178,6 +186,7 @@ int kodama_hip_graph_materialize(kodama_hip_graph* graph, int32_t* indices_one_b
     std::lock_guard<std::mutex> hold(graph->lock);
     select_device(graph->device);
     Stream st(graph->device);
+    const StreamScope scope(st);
     graph->idx.download(indices_one_based, graph->idx.size(), st.get());
     graph->dist.download(distances, graph->dist.size(), st.get());
     st.sync();
@@ -194,6 +203,7 @@ int kodama_hip_graph_dissimilarity(kodama_hip_graph* graph, const int32_t* run_l
     std::lock_guard<std::mutex> hold(graph->lock);
     select_device(graph->device);
     Stream st(graph->device);
+    const StreamScope scope(st);
     const hipStream_t s = st.get();
     const int n = graph->samples;
     const int stride = (runs + 3) / 4 * 4;

@@ -16,6 +16,7 @@
 #include "batch_api.h"
 #include "evolve_device.h"
 #include "evolve_launch.h"
+#include "host_pages.h"
 #include "knn_search.h"
 #include "launch.h"
 #include "mlp.h"
@@ -84,7 +85,10 @@ void run_knn_batch(const BatchRequest& q, int mode, const float* mlp_params, flo
     codes(static_cast<size_t>(runs)), cons(static_cast<size_t>(runs)), fixed(static_cast<size_t>(runs));
   IVec fold_concat(static_cast<size_t>(total));
   int classes = 1;
+  bool one_fold = false, bad_folds = !q.fold_ids && options->folds < 2;
+#pragma omp parallel for schedule(dynamic, 4) reduction(max : classes) reduction(|| : one_fold) if (total > (1 << 14) && !bad_folds)
   for (int r = 0; r < runs; ++r) {
+    if (bad_folds) continue;  // refused below
     const int L = offsets[r + 1] - offsets[r];
     const int* lab = q.initial_labels + offsets[r];
     if (q.constrain) cons[r].assign(q.constrain + offsets[r], q.constrain + offsets[r + 1]);
@@ -92,21 +96,21 @@ void run_knn_batch(const BatchRequest& q, int mode, const float* mlp_params, flo
     folds[r] = q.fold_ids ? IVec(q.fold_ids + offsets[r], q.fold_ids + offsets[r + 1])
                           : make_folds(IVec(lab, lab + L), cons[r], options->folds, options->stratified != 0,
                                        options->cv_seed + static_cast<std::uint64_t>(r));
-    {
-      // Two folds or more: every row then has training rows, so the exact
-      // search gives it at least one neighbour.
-      const auto mm = std::minmax_element(folds[r].begin(), folds[r].end());
-      require(*mm.first != *mm.second, "every run needs at least two distinct folds.");
-    }
+    // Two folds or more: every row then has training rows, so the exact
+    // search gives it at least one neighbour.
+    const auto mm = std::minmax_element(folds[r].begin(), folds[r].end());
+    one_fold = one_fold || *mm.first == *mm.second;
     encode_labels(lab, L, values[r], codes[r]);
     classes = std::max(classes, static_cast<int>(values[r].size()));
     std::copy(folds[r].begin(), folds[r].end(), fold_concat.begin() + offsets[r]);
   }
+  require(!bad_folds, "Number of folds must be at least 2.");
+  require(!one_fold, "every run needs at least two distinct folds.");
   std::unique_ptr<KnnBatch> owned;
   if (tables) {
     owned = std::make_unique<KnnBatch>(options->device, q.table_nbr, q.table_score, offsets, q.table_k, classes);
   } else {
-    const std::vector<float> xs = prepare_rows(x, n, p, options->metric, 0);
+    const PreparedRows xs(x, n, p, options->metric, 0);
     owned = std::make_unique<KnnBatch>(options->device, xs.data(), n, p, offsets, rows, fold_concat, options->k,
                                        options->metric, classes);
   }
@@ -181,7 +185,11 @@ int kodama_hip_exact_knn_search(const float* train, int32_t train_rows, const fl
             "k above 128 (above 64 beyond 128 feature columns) is not supported by the HIP kNN kernel.");
     require(dimensions <= kMaxDims, "the HIP kNN kernel supports 1..256 feature columns.");
     select_device(device);
+    PageWarmer pages;
+    pages.add(out_indices, static_cast<size_t>(query_rows) * k * sizeof(int32_t));
+    pages.add(out_distances, static_cast<size_t>(query_rows) * k * sizeof(float));
     Stream st(device);
+    const StreamScope scope(st);
     const hipStream_t s = st.get();
     DeviceBuffer<float> d_train(static_cast<size_t>(train_rows) * dimensions);
     DeviceBuffer<float> d_query(static_cast<size_t>(query_rows) * dimensions);
@@ -194,6 +202,7 @@ int kodama_hip_exact_knn_search(const float* train, int32_t train_rows, const fl
     device_exact_knn(d_train.get(), train_rows, d_query.get(), query_rows, dimensions, k, metric,
                      query_train_indices ? d_ex.get() : nullptr, d_idx.get(), d_dist.get(), s,
                      &last_knn_fallbacks());
+    pages.wait();
     d_idx.download(out_indices, d_idx.size(), s);
     d_dist.download(out_distances, d_dist.size(), s);
     st.sync();
@@ -245,7 +254,7 @@ int kodama_hip_knncv(const float* x, int32_t n, int32_t p, const int32_t* labels
                                   options->cv_seed);
     IVec values, codes;
     encode_labels(labels, n, values, codes);
-    const std::vector<float> xs = prepare_rows(x, n, p, options->metric, 1);
+    const PreparedRows xs(x, n, p, options->metric, 1);
     IVec rows(static_cast<size_t>(n));
     std::iota(rows.begin(), rows.end(), 0);
     for (int f : folds) require(f >= 0, "invalid fold id.");
@@ -308,7 +317,7 @@ int kodama_hip_core_knn(const float* x, int32_t n, int32_t p, const int32_t* lab
     }
     IVec values, codes;
     encode_labels(labels, n, values, codes);
-    const std::vector<float> xs = prepare_rows(x, n, p, options->metric, 0);
+    const PreparedRows xs(x, n, p, options->metric, 0);
     IVec rows(static_cast<size_t>(n));
     std::iota(rows.begin(), rows.end(), 0);
     KnnBatch batch(options->device, xs.data(), n, p, IVec{0, n}, rows, folds, options->k, options->metric,
@@ -411,7 +420,7 @@ int kodama_hip_knn_fold_tables(const float* x, int32_t n, int32_t p, int32_t run
     const IVec rw(rows, rows + total), folds(fold_ids, fold_ids + total);
     for (int v : rw) require(v >= 0 && v < n, "run row outside the data matrix.");
     for (int f : folds) require(f >= 0, "invalid fold id.");
-    const std::vector<float> xs = prepare_rows(x, n, p, metric, 0);
+    const PreparedRows xs(x, n, p, metric, 0);
     KnnBatch batch(device, xs.data(), n, p, offsets, rw, folds, k, metric, 1, path);
     for (int r = 0; r < runs; ++r) {
       batch.download_tables(r, neighbors + static_cast<size_t>(offsets[r]) * k,

@@ -20,6 +20,7 @@
 #include "engine.h"
 #include "batch_api.h"
 #include "graph_launch.h"
+#include "host_pages.h"
 #include "knn_search.h"
 #include "launch.h"
 #include "matrix.h"
@@ -204,7 +205,14 @@ void matrix_impl(const float* x, int32_t n, int32_t p, const kodama_hip_matrix_o
   require(o.form == 0 || (identity && !any_fixed),
           "the device-resident forms support neither constraint groups nor fixed rows.");
   select_device(o.device);
+  PageWarmer pages;
+  pages.add(res, static_cast<size_t>(o.runs) * n * sizeof(int32_t));
+  if (want_graph && build_graph) {
+    pages.add(graph_indices_one_based, static_cast<size_t>(n) * z.neighbors * sizeof(int32_t));
+    pages.add(graph_distances, static_cast<size_t>(n) * z.neighbors * sizeof(float));
+  }
   Stream st(o.device);
+  const StreamScope scope(st);
   const hipStream_t s = st.get();
   auto clock = std::chrono::steady_clock::now();
   double t[6] = {0, 0, 0, 0, 0, 0};
@@ -394,6 +402,7 @@ void matrix_impl(const float* x, int32_t n, int32_t p, const kodama_hip_matrix_o
     pp.run_stride = project_run_stride(o.runs);
     pp.res = d_res.get();
     check(launch_project(pp, s), "project launch");
+    pages.wait();
     d_res.download(res, d_res.size(), s);
     check(hipStreamSynchronize(s), "projection sync");
   } else {

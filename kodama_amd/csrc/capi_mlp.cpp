@@ -39,6 +39,7 @@ int kodama_hip_mlp_features(const int32_t* neighbors, const int32_t* labels, int
     for (int i = 0; i < rows; ++i) require(labels[i] >= 0 && labels[i] < 0xFFFF, "label codes must be in 0..65534.");
     select_device(device);
     Stream st(device);
+    const StreamScope scope(st);
     const hipStream_t s = st.get();
     DeviceBuffer<int> d_nbr(static_cast<size_t>(rows) * k), d_lab(static_cast<size_t>(rows));
     DeviceBuffer<float> d_feat(static_cast<size_t>(rows) * kMlpIn);
@@ -60,6 +61,7 @@ int kodama_hip_mlp_forward(const float* params, const float* features, int32_t r
     require(rows >= 1, "rows must be positive.");
     select_device(device);
     Stream st(device);
+    const StreamScope scope(st);
     const hipStream_t s = st.get();
     DeviceBuffer<float> d_par(kMlpParams), d_feat(static_cast<size_t>(rows) * kMlpIn),
       d_prob(static_cast<size_t>(rows) * kMlpOut);
@@ -81,6 +83,7 @@ int kodama_hip_mlp_gradients(const float* params, const float* features, const i
     for (int i = 0; i < rows; ++i) require(targets[i] >= 0 && targets[i] <= kMlpKeep, "targets must be in 0..30.");
     select_device(device);
     Stream st(device);
+    const StreamScope scope(st);
     const hipStream_t s = st.get();
     DeviceBuffer<float> d_par(kMlpParams), d_vel(kMlpParams), d_feat(static_cast<size_t>(rows) * kMlpIn),
       d_part(static_cast<size_t>(kMlpGradWaves) * (kMlpParams + 1)), d_loss(1);

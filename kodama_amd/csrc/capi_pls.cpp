@@ -180,16 +180,20 @@ void run_plslda_batch(const BatchRequest& q, int32_t* clbest, double* accbest, d
   require(offsets[0] == 0, "run_offsets[0] must be 0.");
   for (int r = 0; r < runs; ++r) require(offsets[r + 1] > offsets[r] + 1, "every run needs at least two rows.");
   const int total = offsets[runs];
-  std::vector<float> xcat(static_cast<size_t>(total) * p);
   for (int i = 0; i < total; ++i) {
-    const int row = q.landmark_rows[i];
-    require(row >= 0 && row < n, "landmark row outside the data matrix.");
-    std::copy(x + static_cast<size_t>(row) * p, x + static_cast<size_t>(row + 1) * p,
-              xcat.begin() + static_cast<size_t>(i) * p);
+    require(q.landmark_rows[i] >= 0 && q.landmark_rows[i] < n, "landmark row outside the data matrix.");
+  }
+  // The runs' rows overlap: where they outnumber the data rows the data go to
+  // the device once and are gathered there.
+  const bool on_device = total >= n;
+  std::vector<float> xcat(on_device ? 0 : static_cast<size_t>(total) * p);
+  for (int i = 0; i < total && !on_device; ++i) {
+    std::copy_n(x + static_cast<size_t>(q.landmark_rows[i]) * p, p, xcat.begin() + static_cast<size_t>(i) * p);
   }
   std::vector<IVec> values(static_cast<size_t>(runs)), codes(static_cast<size_t>(runs)),
     cons(static_cast<size_t>(runs)), fixed(static_cast<size_t>(runs));
   int classes = 1;
+#pragma omp parallel for schedule(dynamic, 4) reduction(max : classes) if (total > (1 << 14))
   for (int r = 0; r < runs; ++r) {
     encode_labels(q.initial_labels + offsets[r], offsets[r + 1] - offsets[r], values[r], codes[r]);
     classes = std::max(classes, static_cast<int>(values[r].size()));
@@ -219,7 +223,8 @@ void run_plslda_batch(const BatchRequest& q, int32_t* clbest, double* accbest, d
     require(*mm.first != *mm.second, "every run needs at least two distinct folds.");
     set_folds(r, fo);
   }
-  PlsCv pls(options->device, xcat.data(), total, p, *options, classes, offsets);
+  PlsCv pls(options->device, on_device ? x : xcat.data(), total, p, *options, classes, offsets,
+            on_device ? q.landmark_rows : nullptr, n);
   std::vector<RunEvolution> ev;
   ev.reserve(static_cast<size_t>(runs));
   for (int r = 0; r < runs; ++r) {

@@ -4,7 +4,6 @@
 
 #include <hip/hip_runtime_api.h>
 
-#include <atomic>
 #include <cstddef>
 #include <cstdint>
 #include <stdexcept>
@@ -23,6 +22,45 @@ inline void check(hipError_t e, const char* what) {
   }
 }
 
+// Device memory kept from one call for the next (device_pool.cpp). hipFree
+// waits for the whole device and its cost is not bounded by the size: the ten
+// frees of a batch's table build took 1.8 ms, 14 ms once a process had freed
+// some thousand blocks. A block freed under a stream may still be read or
+// written by work queued there, so it goes only to allocations under the same
+// stream until that stream has been settled (its work done); then to any.
+// At most kPoolBytes per device stay in the pool, the rest is freed, and a
+// failed allocation empties it first.
+constexpr size_t kPoolBytes = size_t(2) << 30;
+struct PoolBlock {
+  void* p = nullptr;
+  size_t bytes = 0;         // of the block
+  int device = -1;
+  hipStream_t tag = nullptr;  // null: not from the pool
+};
+PoolBlock pool_take(size_t bytes, int device, hipStream_t tag);
+void pool_give(const PoolBlock& block);
+void pool_settle(int device, hipStream_t tag);  // every block of this tag is idle
+void pool_drop(int device, hipStream_t tag);    // free them instead (their work is unknown)
+
+// The stream under which the calling thread's DeviceBuffers allocate; scopes
+// nest. Without one they use hipMalloc and hipFree.
+class Stream;
+class StreamScope {
+ public:
+  explicit StreamScope(const Stream& s);
+  ~StreamScope();
+  StreamScope(const StreamScope&) = delete;
+  StreamScope& operator=(const StreamScope&) = delete;
+  static hipStream_t current();
+  static int current_device();
+
+ private:
+  hipStream_t before_;
+  int before_device_;
+};
+
+// All work on a buffer that is not yet done when it is released must be on
+// the stream it was allocated under.
 template <class T>
 class DeviceBuffer {
  public:
@@ -31,44 +69,48 @@ class DeviceBuffer {
   ~DeviceBuffer() { release(); }
   DeviceBuffer(const DeviceBuffer&) = delete;
   DeviceBuffer& operator=(const DeviceBuffer&) = delete;
-  DeviceBuffer(DeviceBuffer&& o) noexcept : p_(o.p_), n_(o.n_) { o.p_ = nullptr; o.n_ = 0; }
+  DeviceBuffer(DeviceBuffer&& o) noexcept : block_(o.block_), n_(o.n_) { o.block_ = PoolBlock(); o.n_ = 0; }
   DeviceBuffer& operator=(DeviceBuffer&& o) noexcept {
     if (this != &o) {
       release();
-      p_ = o.p_; n_ = o.n_;
-      o.p_ = nullptr; o.n_ = 0;
+      block_ = o.block_; n_ = o.n_;
+      o.block_ = PoolBlock(); o.n_ = 0;
     }
     return *this;
   }
   void resize(size_t n) {
     if (n == n_) return;
     release();
-    if (n > 0) check(hipMalloc(reinterpret_cast<void**>(&p_), n * sizeof(T)), "hipMalloc");
+    if (n > 0) {
+      if (StreamScope::current() != nullptr) {
+        block_ = pool_take(n * sizeof(T), StreamScope::current_device(), StreamScope::current());
+      } else {
+        check(hipMalloc(&block_.p, n * sizeof(T)), "hipMalloc");
+      }
+    }
     n_ = n;
   }
   void release() {
-    if (p_ != nullptr) (void)hipFree(p_);
-    p_ = nullptr;
+    if (block_.tag != nullptr) pool_give(block_);
+    else if (block_.p != nullptr) (void)hipFree(block_.p);
+    block_ = PoolBlock();
     n_ = 0;
   }
-  T* get() const { return p_; }
+  T* get() const { return static_cast<T*>(block_.p); }
   size_t size() const { return n_; }
   void upload(const T* src, size_t n, hipStream_t s, size_t offset = 0) {
-    if (n) check(hipMemcpyAsync(p_ + offset, src, n * sizeof(T), hipMemcpyHostToDevice, s), "upload");
+    if (n) check(hipMemcpyAsync(get() + offset, src, n * sizeof(T), hipMemcpyHostToDevice, s), "upload");
   }
   void download(T* dst, size_t n, hipStream_t s, size_t offset = 0) const {
-    if (n) check(hipMemcpyAsync(dst, p_ + offset, n * sizeof(T), hipMemcpyDeviceToHost, s), "download");
+    if (n) check(hipMemcpyAsync(dst, get() + offset, n * sizeof(T), hipMemcpyDeviceToHost, s), "download");
   }
 
  private:
-  T* p_ = nullptr;
+  PoolBlock block_;
   size_t n_ = 0;
 };
 
-// Stream-ordered device memory from the device's default memory pool. The
-// pool keeps freed memory (its release threshold is raised once per device),
-// so an evolution that follows another of similar size allocates and frees
-// without a trip to the driver.
+// One pool block under a given stream.
 class PoolBuffer {
  public:
   PoolBuffer() = default;
@@ -77,33 +119,20 @@ class PoolBuffer {
   PoolBuffer& operator=(const PoolBuffer&) = delete;
   void allocate(size_t bytes, int device, hipStream_t s) {
     release();
-    retain_pool(device);
-    check(hipMallocAsync(&p_, bytes, s), "hipMallocAsync");
+    block_ = pool_take(bytes, device, s);
     bytes_ = bytes;
-    s_ = s;
   }
   void release() {
-    if (p_ != nullptr) (void)hipFreeAsync(p_, s_);
-    p_ = nullptr;
+    if (block_.p != nullptr) pool_give(block_);
+    block_ = PoolBlock();
     bytes_ = 0;
   }
-  unsigned char* get() const { return static_cast<unsigned char*>(p_); }
+  unsigned char* get() const { return static_cast<unsigned char*>(block_.p); }
   size_t size() const { return bytes_; }
 
  private:
-  static void retain_pool(int device) {
-    static std::atomic<bool> done[64];
-    if (device < 0 || device >= 64 || done[device].load(std::memory_order_acquire)) return;
-    hipMemPool_t pool = nullptr;
-    check(hipDeviceGetDefaultMemPool(&pool, device), "hipDeviceGetDefaultMemPool");
-    uint64_t threshold = UINT64_MAX;  // setting it twice from two threads is harmless
-    check(hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &threshold), "hipMemPoolSetAttribute");
-    done[device].store(true, std::memory_order_release);
-  }
-
-  void* p_ = nullptr;
+  PoolBlock block_;
   size_t bytes_ = 0;
-  hipStream_t s_ = nullptr;
 };
 
 template <class T>
@@ -135,15 +164,23 @@ class PinnedBuffer {
   size_t n_ = 0;
 };
 
+// Idle streams kept for the next call on their device (creating and destroying
+// one takes 0.24 ms, a small call a few times that): at most kIdleStreams per
+// device, the rest destroyed. A stream comes back when its work is done, and
+// its pool blocks are settled then.
+constexpr size_t kIdleStreams = 8;
+hipStream_t take_stream(int device);
+void give_stream(int device, hipStream_t s);
+
 // A stream on a chosen device, default priority.
 class Stream {
  public:
   explicit Stream(int device) : device_(device) {
     check(hipSetDevice(device), "hipSetDevice");
-    check(hipStreamCreateWithFlags(&s_, hipStreamNonBlocking), "hipStreamCreate");
+    s_ = take_stream(device);
   }
   ~Stream() {
-    if (s_ != nullptr) (void)hipStreamDestroy(s_);
+    if (s_ != nullptr) give_stream(device_, s_);
   }
   Stream(const Stream&) = delete;
   Stream& operator=(const Stream&) = delete;

@@ -7,7 +7,6 @@
 #include <limits>
 #include <map>
 #include <numeric>
-#include <thread>
 #include <unordered_map>
 
 #include <omp.h>
@@ -96,6 +95,7 @@ IVec make_folds(const IVec& labels, const IVec& constrain, int folds, bool strat
 std::vector<float> prepare_rows(const float* x, int n, int p, int metric, int variant) {
   std::vector<float> out(x, x + static_cast<size_t>(n) * p);
   if (metric != KODAMA_HIP_COSINE) return out;
+#pragma omp parallel for if (static_cast<long long>(n) * p > (1 << 18))
   for (int r = 0; r < n; ++r) {
     const float* row = x + static_cast<size_t>(r) * p;
     float* dst = out.data() + static_cast<size_t>(r) * p;
@@ -138,10 +138,26 @@ CoreFlags CoreFlags::from(const kodama_hip_core_options& o) {
 }
 
 void encode_labels(const int* labels, int n, IVec& values, IVec& codes) {
+  codes.resize(static_cast<size_t>(n));
+  values.clear();
+  if (n == 0) return;
+  const auto mm = std::minmax_element(labels, labels + n);
+  const long long lo = *mm.first, span = static_cast<long long>(*mm.second) - lo + 1;
+  if (span <= 4ll * n + 1024) {
+    // Values close together (class numbers are): a table instead of a sort.
+    IVec code(static_cast<size_t>(span), -1);
+    for (int i = 0; i < n; ++i) code[labels[i] - lo] = 0;
+    for (long long v = 0; v < span; ++v) {
+      if (code[v] < 0) continue;
+      code[v] = static_cast<int>(values.size());
+      values.push_back(static_cast<int>(lo + v));
+    }
+    for (int i = 0; i < n; ++i) codes[i] = code[labels[i] - lo];
+    return;
+  }
   values.assign(labels, labels + n);
   std::sort(values.begin(), values.end());
   values.erase(std::unique(values.begin(), values.end()), values.end());
-  codes.resize(static_cast<size_t>(n));
   for (int i = 0; i < n; ++i) {
     codes[i] = static_cast<int>(std::lower_bound(values.begin(), values.end(), labels[i]) - values.begin());
   }
@@ -674,6 +690,7 @@ KnnBatch::KnnBatch(int device, const int* neighbors, const float* scores, const 
       run_offsets_(run_offsets) {
   if (k < 1 || k > kMaxK) throw InvalidArgument("neighbours per row must be in 1..64.");
   if (runs_ < 1) throw InvalidArgument("at least one run is required.");
+  const StreamScope scope(stream_);
   allocate(run_offsets_);
   // Transpose into the padded vote layout with padded row ids, filled slots
   // first so that empty rows are detectable from column 0.
@@ -710,6 +727,7 @@ KnnBatch::KnnBatch(int device, const float* x, int n, int p, const IVec& run_off
   if (classes < 1) throw InvalidArgument("at least one class is required.");
   if (runs_ < 1) throw InvalidArgument("at least one run is required.");
   const hipStream_t s = stream_.get();
+  const StreamScope scope(stream_);
   allocate(run_offsets);
   int max_rows = 0;
   for (int r = 0; r < runs_; ++r) max_rows = std::max(max_rows, run_offsets[r + 1] - run_offsets[r]);
@@ -816,7 +834,9 @@ void KnnBatch::download_tables(int r, int* nbr, float* score) {
 }
 
 int resolve_threads(int requested, int runs) {
-  int t = requested > 0 ? requested : static_cast<int>(std::thread::hardware_concurrency());
+  // Automatic: what OpenMP would use, which follows the process's share of the
+  // host (affinity, OMP_NUM_THREADS).
+  int t = requested > 0 ? requested : omp_get_max_threads();
   if (t < 1) t = 1;
   return std::max(1, std::min(t, runs));
 }

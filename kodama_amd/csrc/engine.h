@@ -26,6 +26,23 @@ IVec make_folds(const IVec& labels, const IVec& constrain, int folds, bool strat
 // Row preparation for cosine search: variant 0 as core.cpp:159-193 (CoreKNN),
 // variant 1 as native_knn.cpp:1005-1035 (KNNCV, graphs). Other metrics copy.
 std::vector<float> prepare_rows(const float* x, int n, int p, int metric, int variant);
+// The same rows without a copy where the metric leaves them as they are (x
+// then outlives this).
+class PreparedRows {
+ public:
+  PreparedRows(const float* x, int n, int p, int metric, int variant) : x_(x) {
+    if (metric != KODAMA_HIP_COSINE) return;
+    own_ = prepare_rows(x, n, p, metric, variant);
+    x_ = own_.data();
+  }
+  PreparedRows(const PreparedRows&) = delete;
+  PreparedRows& operator=(const PreparedRows&) = delete;
+  const float* data() const { return x_; }
+
+ private:
+  std::vector<float> own_;
+  const float* x_;
+};
 
 // Options of maximize_core (core.cpp:1268-1549) in boolean form.
 struct CoreFlags {

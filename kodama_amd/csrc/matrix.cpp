@@ -187,6 +187,11 @@ struct DeviceLloyd {
   }
 };
 
+// Whether split_empty_clusters would change anything.
+bool has_empty(const float* sizes, int rows, int k) {
+  return rows > k && std::find(sizes, sizes + k, 0.0f) != sizes + k;
+}
+
 }  // namespace
 
 IVec device_kmeans(const float* h_x, const float* d_x, int n, int p, int k, std::mt19937_64& rng, int max_iter,
@@ -197,27 +202,27 @@ IVec device_kmeans(const float* h_x, const float* d_x, int n, int p, int k, std:
   std::vector<float> cent(static_cast<size_t>(k) * p), sizes(static_cast<size_t>(k));
   for (int c = 0; c < k; ++c) std::copy_n(h_x + static_cast<size_t>(order[c]) * p, p, cent.data() + static_cast<size_t>(c) * p);
   DeviceLloyd dev(d_x, 1, n, p, k, s);
-  auto assign = [&]() {
-    dev.cent.upload(cent.data(), cent.size(), s);
+  dev.cent.upload(cent.data(), cent.size(), s);
+  for (int it = 0; it < std::max(1, max_iter); ++it) {
     dev.assign(nullptr);
+    dev.update(nullptr);
     int changed = 0;
     dev.changed.download(&changed, 1, s);
-    check(hipStreamSynchronize(s), "kmeans sync");
-    return changed;
-  };
-  for (int it = 0; it < std::max(1, max_iter); ++it) {
-    const int changed = assign();
-    dev.update(nullptr);
-    dev.cent.download(cent.data(), cent.size(), s);
     dev.sizes.download(sizes.data(), sizes.size(), s);
     check(hipStreamSynchronize(s), "kmeans sync");
-    split_empty_clusters(n, p, k, sizes, cent);
+    // The centroids stay on the device unless an empty cluster must be split.
+    if (has_empty(sizes.data(), n, k)) {
+      dev.cent.download(cent.data(), cent.size(), s);
+      check(hipStreamSynchronize(s), "kmeans sync");
+      split_empty_clusters(n, p, k, sizes, cent);
+      dev.cent.upload(cent.data(), cent.size(), s);
+    }
     if (changed == 0) break;
   }
-  assign();
+  dev.assign(nullptr);
   IVec labels(static_cast<size_t>(n));
   dev.asg.download(labels.data(), labels.size(), s);
-  check(hipStreamSynchronize(s), "kmeans sync");
+  check(hipStreamSynchronize(s), "kmeans sync");  // cent is read until here
   for (int& l : labels) ++l;
   return labels;
 }
@@ -227,6 +232,7 @@ std::vector<IVec> device_kmeans_batch(const float* h_x, const int* rows, const f
   k = std::max(1, std::min(k, n));
   const size_t kp = static_cast<size_t>(k) * p;
   std::vector<float> cent(static_cast<size_t>(runs) * kp), sizes(static_cast<size_t>(runs) * k);
+#pragma omp parallel for schedule(dynamic)
   for (int r = 0; r < runs; ++r) {
     const std::uint64_t kseed = rngs[r]() & 0x7fffffffULL;
     const IVec order = seed_order(n, kseed + 1u);
@@ -236,43 +242,47 @@ std::vector<IVec> device_kmeans_batch(const float* h_x, const int* rows, const f
     }
   }
   DeviceLloyd dev(d_rows, runs, n, p, k, s);
-  DeviceBuffer<int> d_active(static_cast<size_t>(runs));
+  DeviceBuffer<int> d_active(2 * static_cast<size_t>(runs));
+  dev.cent.upload(cent.data(), cent.size(), s);
   // Phase of each problem: Lloyd rounds (assign, update, split), then one
   // final assignment with the last centroids, then done.
   enum Phase { kLoop, kFinal, kDone };
   std::vector<int> phase(static_cast<size_t>(runs), kLoop), rounds(static_cast<size_t>(runs), 0),
-    act(static_cast<size_t>(runs)), changed(static_cast<size_t>(runs));
+    act(2 * static_cast<size_t>(runs)), changed(static_cast<size_t>(runs));
   for (;;) {
-    bool any = false;
+    bool any = false, update = false;
     for (int r = 0; r < runs; ++r) {
       act[r] = phase[r] != kDone ? 1 : 0;
+      act[runs + r] = phase[r] == kLoop ? 1 : 0;
       any = any || act[r];
+      update = update || act[runs + r];
     }
     if (!any) break;
-    dev.cent.upload(cent.data(), cent.size(), s);
     d_active.upload(act.data(), act.size(), s);
     dev.assign(d_active.get());
     dev.changed.download(changed.data(), changed.size(), s);
-    check(hipStreamSynchronize(s), "kmeans sync");  // act and changed are reused below
-    bool update = false;
-    for (int r = 0; r < runs; ++r) {
-      act[r] = phase[r] == kLoop ? 1 : 0;
-      update = update || act[r];
-    }
     if (update) {
-      d_active.upload(act.data(), act.size(), s);
-      dev.update(d_active.get());
-      dev.cent.download(cent.data(), cent.size(), s);
+      dev.update(d_active.get() + runs);
       dev.sizes.download(sizes.data(), sizes.size(), s);
-      check(hipStreamSynchronize(s), "kmeans sync");
-#pragma omp parallel for schedule(dynamic)
+    }
+    check(hipStreamSynchronize(s), "kmeans sync");  // act is reused
+    if (update) {
+      // The centroids stay on the device, but for runs with an empty cluster.
+      std::vector<int> split;
       for (int r = 0; r < runs; ++r) {
-        if (!act[r]) continue;
+        if (act[runs + r] && has_empty(sizes.data() + static_cast<size_t>(r) * k, n, k)) split.push_back(r);
+      }
+      for (int r : split) dev.cent.download(cent.data() + r * kp, kp, s, r * kp);
+      if (!split.empty()) check(hipStreamSynchronize(s), "kmeans sync");
+#pragma omp parallel for schedule(dynamic)
+      for (size_t i = 0; i < split.size(); ++i) {
+        const int r = split[i];
         std::vector<float> sz(sizes.begin() + static_cast<size_t>(r) * k, sizes.begin() + static_cast<size_t>(r + 1) * k);
         std::vector<float> ce(cent.begin() + r * kp, cent.begin() + (r + 1) * kp);
         split_empty_clusters(n, p, k, sz, ce);
         std::copy(ce.begin(), ce.end(), cent.begin() + r * kp);
       }
+      for (int r : split) dev.cent.upload(cent.data() + r * kp, kp, s, r * kp);
     }
     for (int r = 0; r < runs; ++r) {
       if (phase[r] == kFinal) {

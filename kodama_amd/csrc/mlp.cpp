@@ -166,6 +166,7 @@ void mlp_train(int device, const float* feat, const int* target, int samples, in
     if (target[s] < 0 || target[s] > kMlpKeep) throw InvalidArgument("MLP target outside 0..30.");
   }
   Stream st(device);
+  const StreamScope scope(st);
   const hipStream_t s = st.get();
   DeviceBuffer<float> d_feat(static_cast<size_t>(samples) * kMlpIn), d_params(kMlpParams), d_vel(kMlpParams),
     d_partial(static_cast<size_t>(kMlpGradWaves) * (kMlpParams + 1));

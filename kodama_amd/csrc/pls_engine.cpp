@@ -6,10 +6,12 @@
 #include "pls_engine.h"
 
 #include <algorithm>
-#include <map>
+#include <numeric>
 #include <random>
 #include <stdexcept>
 
+#include "engine.h"
+#include "knn_search.h"
 #include "pls_launch.h"
 
 namespace kodama_hip {
@@ -48,25 +50,27 @@ struct PlsCv::Impl {
 };
 
 void PlsCv::Impl::rebuild_folds(const IVec& folds) {
+  const StreamScope scope(stream);
   // A fold belongs to the group (run) of its rows; its training rows are the
   // other rows of that group only.
-  std::map<int, int> group_of;
+  IVec fold_code;
+  encode_labels(folds.data(), static_cast<int>(folds.size()), fold_ids, fold_code);
+  IVec group_of(fold_ids.size(), -1);  // by fold code
   for (int g = 0; g + 1 < static_cast<int>(groups.size()); ++g) {
     for (int i = groups[g]; i < groups[g + 1]; ++i) {
-      const auto it = group_of.emplace(folds[i], g).first;
-      if (it->second != g) throw InvalidArgument("a fold id spans two runs.");
+      int& of = group_of[fold_code[i]];
+      if (of < 0) of = g;
+      if (of != g) throw InvalidArgument("a fold id spans two runs.");
     }
   }
-  fold_ids.clear();
-  for (const auto& kv : group_of) fold_ids.push_back(kv.first);
   const int F = static_cast<int>(fold_ids.size());
   // Each fold's training sums are its run's other folds' sums: the folds of a
   // run must be consecutive in fold-id order.
   IVec h_first(static_cast<size_t>(F)), h_end(static_cast<size_t>(F));
   for (int f = 0; f < F;) {
-    const int g = group_of[fold_ids[f]];
+    const int g = group_of[f];
     int e = f + 1;
-    while (e < F && group_of[fold_ids[e]] == g) ++e;
+    while (e < F && group_of[e] == g) ++e;
     for (int t = f; t < e; ++t) {
       h_first[t] = f;
       h_end[t] = e;
@@ -76,21 +80,23 @@ void PlsCv::Impl::rebuild_folds(const IVec& folds) {
   {
     std::vector<char> seen(groups.size(), 0);
     for (int f = 0; f < F; ++f) {
-      const int g = group_of[fold_ids[f]];
+      const int g = group_of[f];
       if (h_first[f] == f && seen[g]) throw InvalidArgument("the fold ids of a run must be consecutive.");
       seen[g] = 1;
     }
   }
-  h_val_rows.clear();
-  h_val_off.assign(1, 0);
+  // Each fold's rows, ascending.
+  h_val_off.assign(static_cast<size_t>(F) + 1, 0);
+  for (int c : fold_code) ++h_val_off[c + 1];
+  std::partial_sum(h_val_off.begin(), h_val_off.end(), h_val_off.begin());
+  h_val_rows.resize(fold_code.size());
+  {
+    IVec at(h_val_off.begin(), h_val_off.end() - 1);
+    for (size_t i = 0; i < fold_code.size(); ++i) h_val_rows[at[fold_code[i]]++] = static_cast<int>(i);
+  }
   IVec h_shift(static_cast<size_t>(F));
   for (int f = 0; f < F; ++f) {
-    const int fid = fold_ids[f];
-    const int g = group_of[fid];
-    for (int i = groups[g]; i < groups[g + 1]; ++i) {
-      if (folds[i] == fid) h_val_rows.push_back(i);
-    }
-    h_val_off.push_back(static_cast<int>(h_val_rows.size()));
+    const int g = group_of[f];
     if (h_val_off[f + 1] - h_val_off[f] == groups[g + 1] - groups[g]) {
       throw std::runtime_error("PLS fold has no training samples.");
     }
@@ -177,10 +183,11 @@ void PlsCv::Impl::rebuild_folds(const IVec& folds) {
 }
 
 PlsCv::PlsCv(int device, const float* x, int n, int p, const kodama_hip_core_options& o, int classes,
-             const IVec& run_offsets) {
+             const IVec& run_offsets, const int* rows, int x_rows) {
   if (o.max_components < 1) throw InvalidArgument("PLSOptions::max_components must be positive.");
   if (p > kPlsMaxDims) throw InvalidArgument("the HIP PLS-LDA kernels support up to 256 feature columns.");
   Impl* m = new Impl(device);
+  const StreamScope scope(m->stream);
   m->n = n;
   m->p = p;
   m->groups = run_offsets.empty() ? IVec{0, n} : run_offsets;
@@ -200,7 +207,16 @@ PlsCv::PlsCv(int device, const float* x, int n, int p, const kodama_hip_core_opt
   }
   const hipStream_t s = m->stream.get();
   m->x.resize(static_cast<size_t>(n) * p);
-  m->x.upload(x, m->x.size(), s);
+  if (rows != nullptr) {
+    DeviceBuffer<float> source(static_cast<size_t>(x_rows) * p);
+    DeviceBuffer<int> d_rows(static_cast<size_t>(n));
+    source.upload(x, source.size(), s);
+    d_rows.upload(rows, d_rows.size(), s);
+    check(launch_gather_rows(source.get(), d_rows.get(), n, p, m->x.get(), s), "gather_rows launch");
+    m->stream.sync();
+  } else {
+    m->x.upload(x, m->x.size(), s);
+  }
   const std::vector<double> w0 = pls_start_vector(p);
   m->w0.resize(w0.size());
   m->w0.upload(w0.data(), w0.size(), s);
@@ -371,6 +387,7 @@ PlsGeneralResult pls_general_fit(int device, const float* x, const float* y, int
     throw InvalidArgument("the HIP PLS kernels hold responses x predictors <= 8192 and predictors + responses <= 448.");
   }
   Stream st(device);
+  const StreamScope scope(st);
   const hipStream_t s = st.get();
   DeviceBuffer<float> dx(static_cast<size_t>(n) * p), dy(static_cast<size_t>(n) * q);
   dx.upload(x, dx.size(), s);

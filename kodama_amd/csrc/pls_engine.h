@@ -25,9 +25,10 @@ class PlsCv {
   // x [n x p] host rows; `classes` = number of label codes (0..classes-1).
   // With run_offsets, rows [run_offsets[r], run_offsets[r+1]) form run r: a
   // fold's ids belong to one run and it trains on that run's other rows only
-  // (empty: one run of all rows).
+  // (empty: one run of all rows). With rows, row i is row rows[i] of x
+  // [x_rows x p], gathered on the device.
   PlsCv(int device, const float* x, int n, int p, const kodama_hip_core_options& options, int classes,
-        const IVec& run_offsets = IVec());
+        const IVec& run_offsets = IVec(), const int* rows = nullptr, int x_rows = 0);
   ~PlsCv();
   PlsCv(const PlsCv&) = delete;
   PlsCv& operator=(const PlsCv&) = delete;
