@@ -619,11 +619,11 @@ hipError_t launch_vote_reset(int* counts, int* firsts, int* matches, int runs, i
 }
 
 __global__ void gather_rows_kernel(const float* __restrict__ src, const int* __restrict__ rows, int count, int p,
-                                   float* __restrict__ dst) {
+                                   float* __restrict__ dst, int stride) {
   const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= static_cast<size_t>(count) * p) return;
-  const int r = static_cast<int>(i / p), d = static_cast<int>(i % p);
-  dst[i] = src[static_cast<size_t>(rows[r]) * p + d];
+  if (i >= static_cast<size_t>(count) * stride) return;
+  const int r = static_cast<int>(i / stride), d = static_cast<int>(i % stride);
+  dst[i] = d < p ? src[static_cast<size_t>(rows != nullptr ? rows[r] : r) * p + d] : 0.0f;
 }
 
 __global__ void scatter_results_kernel(const int* __restrict__ src_idx, const float* __restrict__ src_dist,
@@ -662,11 +662,13 @@ hipError_t launch_publish_listed(const int* idx, const float* dist, const int* q
   return hipGetLastError();
 }
 
-hipError_t launch_gather_rows(const float* src, const int* rows, int count, int p, float* dst, hipStream_t s) {
-  const size_t total = static_cast<size_t>(count) * p;
+hipError_t launch_gather_rows(const float* src, const int* rows, int count, int p, float* dst, hipStream_t s,
+                              int stride) {
+  if (stride == 0) stride = p;
+  const size_t total = static_cast<size_t>(count) * stride;
   if (total == 0) return hipSuccess;
   hipLaunchKernelGGL(gather_rows_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, s, src,
-                     rows, count, p, dst);
+                     rows, count, p, dst, stride);
   return hipGetLastError();
 }
 

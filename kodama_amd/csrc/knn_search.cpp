@@ -105,7 +105,14 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
   const bool same = d_query == d_train;
   DeviceBuffer<float> t_n2(static_cast<size_t>(train_rows)), n2_max(2);
   check(hipMemsetAsync(n2_max.get(), 0, 2 * sizeof(float), s), "memset");
-  check(launch_stream_norms(d_train, train_rows, dims, t_n2.get(), n2_max.get(), s), "stream_norms launch");
+  check(launch_stream_norms(d_train, train_rows, dims, dims, t_n2.get(), n2_max.get(), s), "stream_norms launch");
+  // The rerank's 16-byte loads need rows of whole ones: a padded copy where
+  // the columns are not a multiple of four (0.1 ms per million rows of 50).
+  const int stride = stream_row_stride(dims);
+  DeviceBuffer<float> padded(stride != dims ? static_cast<size_t>(train_rows) * stride : 0);
+  if (stride != dims) {
+    check(launch_gather_rows(d_train, nullptr, train_rows, dims, padded.get(), s, stride), "gather_rows launch");
+  }
   // One pass over `rows` queries; returns the flagged ones.
   auto pass = [&](const float* q, int rows, const int* ex, int parts, int list, bool self, int* idx, float* dist) {
     const int steps = stream_steps(dims, parts, euclid);
@@ -116,7 +123,7 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
     DeviceBuffer<float> q_n2;
     if (!self) {
       q_n2.resize(static_cast<size_t>(rows));
-      check(launch_stream_norms(q, rows, dims, q_n2.get(), n2_max.get() + 1, s), "stream_norms launch");
+      check(launch_stream_norms(q, rows, dims, dims, q_n2.get(), n2_max.get() + 1, s), "stream_norms launch");
     }
     StreamOperandJob op;
     op.x = d_train;
@@ -148,7 +155,9 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
     DeviceBuffer<int> count(static_cast<size_t>(batch) * plan.slices), flags(static_cast<size_t>(rows));
     DeviceBuffer<float> bound(count.size());
     KnnStreamParams m;
-    m.train = d_train;
+    m.train = stride != dims ? padded.get() : d_train;
+    m.train_stride = stride;
+    m.query_stride = dims;
     m.train_op = t_op.get();
     m.norm2_max = n2_max.get();
     m.train_rows = train_rows;
@@ -271,17 +280,19 @@ int device_fold_tables(const FoldTableJob& job, hipStream_t s) {
     return 1;
   }
 
-  DeviceBuffer<float> xc(static_cast<size_t>(total) * job.p), n2(static_cast<size_t>(total)), n2_max(2);
+  const int stride = stream_row_stride(job.p);
+  DeviceBuffer<float> xc(static_cast<size_t>(total) * stride), n2(static_cast<size_t>(total)), n2_max(2);
   DeviceBuffer<int> flags(static_cast<size_t>(total));
-  check(launch_gather_rows(job.d_x, job.d_rows, total, job.p, xc.get(), s), "gather_rows launch");
+  check(launch_gather_rows(job.d_x, job.d_rows, total, job.p, xc.get(), s, stride), "gather_rows launch");
   check(hipMemsetAsync(n2_max.get(), 0, 2 * sizeof(float), s), "memset");
-  check(launch_stream_norms(xc.get(), total, job.p, n2.get(), n2_max.get(), s), "stream_norms launch");
+  check(launch_stream_norms(xc.get(), total, job.p, stride, n2.get(), n2_max.get(), s), "stream_norms launch");
   std::vector<int> h_flags(static_cast<size_t>(total));
   auto pass = [&](int parts, int list) {
     const int steps = stream_steps(job.p, parts, euclid);
     DeviceBuffer<unsigned char> t_op(stream_operand_bytes(static_cast<size_t>(job.pad_total), steps)), q_op(t_op.size());
     StreamOperandJob op;
     op.x = xc.get();
+    op.stride = stride;
     op.norm2 = n2.get();
     op.norm2_max = n2_max.get();
     op.rows = total;
@@ -301,6 +312,7 @@ int device_fold_tables(const FoldTableJob& job, hipStream_t s) {
     DeviceBuffer<float> bound(count.size()), threshold(static_cast<size_t>(job.pad_total));
     KnnStreamParams m;
     m.train = m.query = xc.get();
+    m.train_stride = m.query_stride = stride;
     m.train_op = t_op.get();
     m.query_op = q_op.get();
     m.query_norm2 = n2.get();

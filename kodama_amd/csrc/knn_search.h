@@ -15,8 +15,10 @@ namespace kodama_hip {
 hipError_t launch_publish_listed(const int* idx, const float* dist, const int* qlist, const int* qrun,
                                  const int* pad_offsets, int pad_total, int count, int k, int* out_index,
                                  float* out_score, hipStream_t s);
-// rows[i] of src [* x p] -> dst [count x p]; and the inverse scatter of [count x k] results.
-hipError_t launch_gather_rows(const float* src, const int* rows, int count, int p, float* dst, hipStream_t s);
+// Rows rows[i] of src [* x p] (null: row i) -> dst, `stride` floats apart (0:
+// p), zeros past p; and the inverse scatter of [count x k] results.
+hipError_t launch_gather_rows(const float* src, const int* rows, int count, int p, float* dst, hipStream_t s,
+                              int stride = 0);
 hipError_t launch_scatter_results(const int* src_idx, const float* src_dist, const int* rows, int count, int k,
                                   int* dst_idx, float* dst_dist, hipStream_t s);
 

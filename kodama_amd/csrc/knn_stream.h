@@ -11,7 +11,7 @@ namespace kodama_hip {
 constexpr int kStreamMaxSteps = 9;     // 32-deep MFMA steps per pair (operand width / 32)
 constexpr int kStreamMaxK = 128;       // neighbours served
 constexpr int kStreamBlockRows = 256;  // operand rows are padded to this multiple per set or run
-constexpr int kStreamMerge = 1024;     // candidates the rerank holds per query (all slices)
+constexpr int kStreamMerge = 512;      // candidates the rerank holds per query (all slices)
 constexpr int kStreamMaxSlices = 16;
 
 // Operand width of one pair: `parts` 1 (FP16 of the rows) or 3 (high and low
@@ -33,8 +33,11 @@ inline int stream_min_max_slices(int k) { return (21 * k / 10 + 31) / 32; }
 inline int stream_sample_chunks(int k) { return 16 * k; }
 
 struct KnnStreamParams {
-  const float* train = nullptr;     // [train rows x dims], for the exact re-score
+  // Rows for the exact re-score; train_stride is a multiple of 4 floats, train
+  // 16-byte aligned.
+  const float* train = nullptr;
   const float* query = nullptr;
+  int train_stride = 0, query_stride = 0;
   const void* train_op = nullptr;   // operand fragments (launch_stream_operands)
   const void* query_op = nullptr;
   const float* query_norm2 = nullptr;  // [query rows]
@@ -64,14 +67,17 @@ struct KnnStreamParams {
   float* out_dist = nullptr;        // internal distances; tables: scores (minus the distance)
 };
 
-// Squared norms [rows] and their maximum (into *norm2_max, which the caller
-// cleared to 0).
-hipError_t launch_stream_norms(const float* x, int rows, int p, float* norm2, float* norm2_max, hipStream_t s);
+// Squared norms [rows] (rows `stride` floats apart) and their maximum (into
+// *norm2_max, which the caller cleared to 0).
+hipError_t launch_stream_norms(const float* x, int rows, int p, int stride, float* norm2, float* norm2_max,
+                               hipStream_t s);
+inline int stream_row_stride(int p) { return (p + 3) / 4 * 4; }
 // Rows -> operand fragments of `steps` x 32 columns, rows padded with zeros to
 // pad_rows; either output may be null. norm2_max [2] scales them.
 // For the padded table layout pass block_run / run_offsets / pad_offsets.
 struct StreamOperandJob {
   const float* x = nullptr;
+  int stride = 0;                   // floats between rows (0: p)
   const float* norm2 = nullptr;
   const float* norm2_max = nullptr;
   int rows = 0, p = 0, parts = 1, euclid = 0;

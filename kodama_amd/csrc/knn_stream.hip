@@ -35,15 +35,22 @@
 // knn_stream_rerank_kernel: one wave per query merges the slices'
 // candidates, applies the same bound once more, re-scores what is left in the
 // reference's FP32 summation order (one candidate per lane) and writes the k
-// smallest by (distance, index): the rows and values of the exact scan.
+// smallest by (distance, index): the rows and values of the exact scan. Its
+// time is the gathered rows (a lane's own row, 16 bytes a load: the copy is
+// padded to 4 columns) and the ranking of n ~ k candidates against each other,
+// so that the second bound is only taken where it saves a round of 64
+// distances, and distance and row are one 64-bit key, read two at a time.
+// Rows staged through LDS for coalesced loads left fewer waves in flight:
+// 1.9 ms against 1.5 at k = 100.
 // Queries whose bound kept more than the buffer holds (many near-equal
 // distances) are flagged for another path.
 //
 // Measured on one MI355X: the self graph of 1M x 50, k = 30, maxima 3.5 ms,
 // candidates 130 ms (7.7e12 pairs/s, 0.98 PFLOP/s of FP16 with the padding to
-// 64 columns), rerank 5.4 ms; split-BF16 products with sorted lists per lane
+// 64 columns), rerank 4.1 ms (5.4 with 4-byte loads, a bound for every query and
+// keys of two words); split-BF16 products with sorted lists per lane
 // column took 871 + 34 ms for the candidates. 100k x 50, k = 100: 1.0 + 2.8 +
-// 1.5 ms against 26.6 + 18.9 (scan of the queries the lists could not
+// 1.06 ms (1.5) against 26.6 + 18.9 (scan of the queries the lists could not
 // certify) + 1.3. 10007 x 30011 x 100, k = 30: 0.33 ms against 23.1 ms of the
 // register scan. A running threshold without the maxima appended 3.5 times as
 // much: 316 ms at 1M rows, 18.3 ms at 100k.
@@ -100,7 +107,7 @@ __device__ __forceinline__ uint32_t kth_largest(const uint32_t (&key)[R], int us
 
 // 16 lanes per row; block maximum, one atomic per block (norms are >= 0, so
 // their bits order as integers; a NaN norm does not enter).
-__global__ void stream_norms_kernel(const float* __restrict__ x, int rows, int p, float* __restrict__ norm2,
+__global__ void stream_norms_kernel(const float* __restrict__ x, int rows, int p, int stride, float* __restrict__ norm2,
                                     float* __restrict__ norm2_max) {
   __shared__ uint32_t s_max;
   if (threadIdx.x == 0) s_max = 0u;
@@ -108,7 +115,7 @@ __global__ void stream_norms_kernel(const float* __restrict__ x, int rows, int p
   const int sub = threadIdx.x & 15;
   for (size_t r = static_cast<size_t>(blockIdx.x) * 16 + (threadIdx.x >> 4); r < static_cast<size_t>(rows);
        r += static_cast<size_t>(gridDim.x) * 16) {
-    const float* src = x + r * p;
+    const float* src = x + r * stride;
     float s = 0.0f;
     for (int d = sub; d < p; d += 16) s = fmaf(src[d], src[d], s);
     s += __shfl_xor(s, 1);
@@ -152,7 +159,7 @@ __global__ void stream_operands_kernel(StreamOperandJob job, int steps) {
   const int p = job.p;
   const int c0 = step * 32 + 8 * (lane >> 4);
   _Float16 tv[8], qv[8];
-  const float* src = job.x + static_cast<size_t>(live ? row : 0) * p;
+  const float* src = job.x + static_cast<size_t>(live ? row : 0) * (job.stride != 0 ? job.stride : p);
   const float nt = live && job.euclid ? -(job.norm2[row] * scale) * scale * 0x1p-14f : 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
@@ -556,17 +563,23 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(Kn
 }
 
 // Reference-order FP32 distance (native_knn.cpp:41-95), one lane per train
-// row, the query row uniform over the wave (scalar loads).
+// row, the query row uniform over the wave (scalar loads). The train row's
+// stride is a multiple of four floats: each lane reads its own row, so every
+// load costs the L1 one line per lane, and 16-byte loads take a quarter of
+// what single columns do.
 template <bool EUCLID>
-__device__ __forceinline__ float stream_exact_distance(const float* __restrict__ q, const float* __restrict__ c, int p) {
+__device__ __forceinline__ float stream_exact_distance(const float* __restrict__ q, const f32x4* __restrict__ c, int p) {
   float acc[32];
 #pragma unroll
   for (int s = 0; s < 32; ++s) acc[s] = 0.0f;
   const int full = p & ~31;
   for (int b = 0; b < full; b += 32) {
+    f32x4 v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = c[b / 4 + i];
 #pragma unroll
     for (int s = 0; s < 32; ++s) {
-      const float cv = c[b + s];
+      const float cv = v[s / 4][s % 4];
       if (EUCLID) {
         const float t = __fsub_rn(q[b + s], cv);
         acc[s] = __fmaf_rn(t, t, acc[s]);
@@ -575,6 +588,10 @@ __device__ __forceinline__ float stream_exact_distance(const float* __restrict__
       }
     }
   }
+  // The tail of up to 31 columns, in flight while the lane tree is summed.
+  f32x4 tail[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) tail[i] = full + 4 * i < p ? c[full / 4 + i] : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   float v4[4];
 #pragma unroll
   for (int l = 0; l < 4; ++l) {
@@ -583,28 +600,35 @@ __device__ __forceinline__ float stream_exact_distance(const float* __restrict__
     v4[l] = __fadd_rn(lo, hi);
   }
   float r = __fadd_rn(__fadd_rn(v4[0], v4[1]), __fadd_rn(v4[2], v4[3]));
-  // Tail of up to 31 columns: loads first (clamped), then the chain.
-  float tail[32];
-#pragma unroll
-  for (int s = 0; s < 31; ++s) tail[s] = full + s < p ? c[full + s] : 0.0f;
 #pragma unroll
   for (int s = 0; s < 31; ++s) {
     if (full + s < p) {
+      const float cv = tail[s / 4][s % 4];
       if (EUCLID) {
-        const float t = __fsub_rn(q[full + s], tail[s]);
+        const float t = __fsub_rn(q[full + s], cv);
         r = __fmaf_rn(t, t, r);
       } else {
-        r = __fmaf_rn(q[full + s], tail[s], r);
+        r = __fmaf_rn(q[full + s], cv, r);
       }
     }
   }
   return EUCLID ? r : -r;
 }
 
+// The k-th largest of n scores in LDS entries, in R registers per lane.
+template <int R>
+__device__ __forceinline__ uint32_t kth_of_entries(const uint2* ent, int n, int k, int lane) {
+  uint32_t key[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) key[i] = i * kWave + lane < n ? order_key(__uint_as_float(ent[i * kWave + lane].x)) : 0u;
+  return kth_largest<R>(key, (n + kWave - 1) / kWave, k);
+}
+
 template <bool EUCLID>
-__global__ void __launch_bounds__(256) knn_stream_rerank_kernel(KnnStreamParams prm) {
-  constexpr int kRegs = kStreamMerge / kWave;
-  __shared__ uint2 s_ent[4][kStreamMerge];
+__global__ void __launch_bounds__(256, 4) knn_stream_rerank_kernel(KnnStreamParams prm) {
+  // Two entries past the end: the ranking reads pairs.
+  __shared__ __align__(16) uint2 s_ent[4][kStreamMerge + 2];
+  __shared__ float s_dist[4][kStreamMerge];
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   const int op_row = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + wave);
@@ -649,19 +673,16 @@ __global__ void __launch_bounds__(256) knn_stream_rerank_kernel(KnnStreamParams 
   if (lane == 0) prm.flags[q] = 0;
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
-  if (n > k) {
-    uint32_t key[kRegs];
-#pragma unroll
-    for (int i = 0; i < kRegs; ++i) {
-      key[i] = 0u;
-      if (i * kWave < n) key[i] = i * kWave + lane < n ? order_key(__uint_as_float(ent[i * kWave + lane].x)) : 0u;
-    }
+  // A tighter bound only where it can save a round of 64 exact distances.
+  if ((n + kWave - 1) / kWave > (k + kWave - 1) / kWave) {
     const float scale = operand_scale(prm.norm2_max);
     const float tmax = sqrtf(prm.norm2_max[0]) * scale * 1.0001f;
     const float qn = sqrtf(prm.query_norm2[q]) * scale * 1.0001f;
     const int width = prm.parts * p + (prm.euclid ? 3 : 0);
-    bound = drop_bound(key_value(kth_largest<kRegs>(key, (n + kWave - 1) / kWave, k)),
-                       2.0f * pair_error(qn, tmax, p, prm.parts, width));
+    const uint32_t kth = n <= 2 * kWave   ? kth_of_entries<2>(ent, n, k, lane)
+                         : n <= 4 * kWave ? kth_of_entries<4>(ent, n, k, lane)
+                                          : kth_of_entries<kStreamMerge / kWave>(ent, n, k, lane);
+    bound = drop_bound(key_value(kth), 2.0f * pair_error(qn, tmax, p, prm.parts, width));
     // In-place compaction: a register's entries go to slots at or before
     // their own, and each is read before a later register's is written.
     int kept = 0;
@@ -679,13 +700,17 @@ __global__ void __launch_bounds__(256) knn_stream_rerank_kernel(KnnStreamParams 
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
-  // Exact distances as sortable (distance, row) pairs.
-  const float* qrow = prm.query + static_cast<size_t>(q) * p;
+  // Exact distances, as (distance order, row) keys: .y above .x.
+  const float* qrow = prm.query + static_cast<size_t>(q) * prm.query_stride;
   for (int e = lane; e < n; e += kWave) {
-    const int row = static_cast<int>(ent[e].y);
-    const float d = stream_exact_distance<EUCLID>(qrow, prm.train + static_cast<size_t>(row) * p, p);
-    ent[e].x = __float_as_uint(d);
+    const uint32_t row = ent[e].y;
+    const float d = stream_exact_distance<EUCLID>(
+        qrow, reinterpret_cast<const f32x4*>(prm.train + static_cast<size_t>(row) * prm.train_stride), p);
+    // -0 sorts with +0, as the float comparison has it.
+    ent[e] = make_uint2(row, order_key(d + 0.0f));
+    s_dist[wave][e] = d;
   }
+  if (lane < 2) ent[n + lane] = make_uint2(0xFFFFFFFFu, 0xFFFFFFFFu);
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
   // [query x k] rows and distances; for tables the transposed vote layout
@@ -693,17 +718,18 @@ __global__ void __launch_bounds__(256) knn_stream_rerank_kernel(KnnStreamParams 
   const size_t step = tables ? static_cast<size_t>(prm.pad_rows) : 1;
   int* out_i = prm.out_index + (tables ? static_cast<size_t>(op_row) : static_cast<size_t>(q) * k);
   float* out_d = prm.out_dist + (tables ? static_cast<size_t>(op_row) : static_cast<size_t>(q) * k);
+  const ulonglong2* keys = reinterpret_cast<const ulonglong2*>(ent);
   for (int e = lane; e < n; e += kWave) {
-    const uint2 v = ent[e];
-    const float d = __uint_as_float(v.x);
+    const unsigned long long mine = reinterpret_cast<const unsigned long long*>(ent)[e];
     int rank = 0;
-    for (int t = 0; t < n; ++t) {
-      const uint2 o = ent[t];
-      const float od = __uint_as_float(o.x);
-      rank += od < d || (od == d && o.y < v.y) ? 1 : 0;
+#pragma unroll 4
+    for (int t = 0; t < (n + 1) / 2; ++t) {
+      const ulonglong2 o = keys[t];
+      rank += (o.x < mine ? 1 : 0) + (o.y < mine ? 1 : 0);
     }
     if (rank < k) {
-      out_i[rank * step] = static_cast<int>(v.y) - (tables ? g.delta : 0);
+      const float d = s_dist[wave][e];
+      out_i[rank * step] = static_cast<int>(static_cast<uint32_t>(mine)) - (tables ? g.delta : 0);
       out_d[rank * step] = tables ? -d : d;
     }
   }
@@ -713,11 +739,12 @@ __global__ void __launch_bounds__(256) knn_stream_rerank_kernel(KnnStreamParams 
   }
 }
 
-hipError_t launch_stream_norms(const float* x, int rows, int p, float* norm2, float* norm2_max, hipStream_t s) {
+hipError_t launch_stream_norms(const float* x, int rows, int p, int stride, float* norm2, float* norm2_max,
+                               hipStream_t s) {
   if (rows == 0) return hipSuccess;
   const int blocks = (rows + 15) / 16;
   hipLaunchKernelGGL(stream_norms_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, x,
-                     rows, p, norm2, norm2_max);
+                     rows, p, stride, norm2, norm2_max);
   return hipGetLastError();
 }
 
@@ -758,7 +785,7 @@ hipError_t launch_knn_stream(const KnnStreamParams& prm, hipStream_t s) {
   if (prm.query_rows == 0) return hipSuccess;
   const int steps = stream_steps(prm.dims, prm.parts, prm.euclid != 0);
   if (prm.dims < 1 || steps > kStreamMaxSteps || prm.k < 1 || prm.k > kStreamMaxK || prm.train_rows < 1 ||
-      prm.slices < 1 || prm.max_slices < 1 || prm.max_slices > kStreamMaxSlices || prm.sample_chunks < 1 || (prm.list != 8 && prm.list != 16) || (prm.list == 8 && prm.k > 32) ||
+      prm.train_stride % 4 != 0 || prm.train_stride < prm.dims || prm.query_stride < prm.dims || prm.slices < 1 || prm.max_slices < 1 || prm.max_slices > kStreamMaxSlices || prm.sample_chunks < 1 || (prm.list != 8 && prm.list != 16) || (prm.list == 8 && prm.k > 32) ||
       (prm.block_run != nullptr) != (prm.folds != nullptr) || prm.pad_rows % kStreamBlockRows != 0) {
     return hipErrorInvalidValue;
   }
