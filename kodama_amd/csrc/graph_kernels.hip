@@ -5,10 +5,13 @@
 // Dissimilarity layout: the run labels res [runs x samples] are transposed once
 // to sample-major rows of `stride` int32 (runs rounded up to a multiple of 4,
 // padded with 0 = unassigned, which never counts as valid). One wave owns one
-// graph row: per edge each lane loads 4 of the neighbour's labels (one 16-byte
-// load, the whole row in one coalesced instruction for up to 256 runs) and the
-// co-assignment counts come from ballots. The row is then ordered stably by
-// (rewritten distance, output id) by rank counting in LDS.
+// graph row: per edge each lane loads 4 of the neighbour's labels (16 bytes; a
+// half wave per edge for up to 128 runs, the whole wave beyond), eight loads
+// in flight, and the co-assignment counts come from ballots. The distances are
+// then rewritten one edge per lane and the row ordered stably by (rewritten
+// distance, output id) by rank counting in LDS. Bound by the label rows: 4 GB
+// from the caches for 100k rows, 100 neighbours, 100 runs, in 0.83 ms (1.92
+// with one edge at a time, a wave per edge, both label rows loaded for each).
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -71,43 +74,79 @@ __global__ void labels_transpose_kernel(const int* __restrict__ res, int runs, i
 }
 
 // One wave per graph row. `keys`/`ids` live in dynamic LDS: kRowsPerBlock x
-// neighbors entries each.
+// neighbors entries each; a key holds its edge's counts (same, valid) before.
+// LANES per edge: 32 (quads <= 32) or 64.
+// The vectors are the compiler's own type: an array of int4 goes to scratch.
+using i32x4 = __attribute__((ext_vector_type(4))) int;
+
+template <int LANES>
 __global__ void __launch_bounds__(kWave * kRowsPerBlock)
 dissimilarity_kernel(int* __restrict__ indices, float* __restrict__ distances, int samples, int neighbors,
                      const int* __restrict__ labels, int stride, int input_one_based, int output_one_based) {
+  constexpr int kInFlight = 8;
+  constexpr int kEdges = kWave / LANES;  // per step
   extern __shared__ unsigned long long dis_lds[];
-  const int wave = threadIdx.x / kWave;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const int lane = threadIdx.x & (kWave - 1);
   const int row = blockIdx.x * kRowsPerBlock + wave;
-  const bool live = row < samples;  // every wave reaches the barrier below
+  if (row >= samples) return;  // whole waves; no block barrier below
   unsigned long long* keys = dis_lds + static_cast<size_t>(wave) * neighbors;
   int* ids = reinterpret_cast<int*>(dis_lds + static_cast<size_t>(kRowsPerBlock) * neighbors) +
              static_cast<size_t>(wave) * neighbors;
   const int quads = stride >> 2;
-  const int4* lab4 = reinterpret_cast<const int4*>(labels);
+  const i32x4* lab4 = reinterpret_cast<const i32x4*>(labels);
   const size_t base = static_cast<size_t>(row) * neighbors;
+  const int group = lane / LANES, slot = lane % LANES;
+  auto count = [&](bool v) -> int {
+    const uint64_t m = __ballot(v);
+    if constexpr (LANES == 64) return __popcll(m);
+    else return __popc(static_cast<uint32_t>(group != 0 ? m >> 32 : m));
+  };
 
-  // Co-assignment counts: 4 runs per lane per chunk of 256 runs.
-  for (int j = 0; live && j < neighbors; ++j) {
-    const int stored = indices[base + j];
+  for (int j0 = 0; j0 < neighbors; j0 += kInFlight * kEdges) {
+    int nb[kInFlight], same[kInFlight], valid[kInFlight];
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) {
+      const int j = j0 + u * kEdges + group;
+      const int stored = j < neighbors ? indices[base + j] : -1;
+      nb[u] = stored >= 0 && input_one_based ? stored - 1 : stored;
+      same[u] = valid[u] = 0;
+    }
+    for (int q0 = 0; q0 < quads; q0 += LANES) {
+      const int q = q0 + slot;
+      const i32x4 zero = {0, 0, 0, 0};
+      const i32x4 a = q < quads ? lab4[static_cast<size_t>(row) * quads + q] : zero;
+      i32x4 b[kInFlight];
+#pragma unroll
+      for (int u = 0; u < kInFlight; ++u) {
+        b[u] = q < quads && nb[u] >= 0 && nb[u] < samples ? lab4[static_cast<size_t>(nb[u]) * quads + q] : zero;
+      }
+#pragma unroll
+      for (int u = 0; u < kInFlight; ++u) {
+        const bool v0 = a.x != 0 && b[u].x != 0, v1 = a.y != 0 && b[u].y != 0;
+        const bool v2 = a.z != 0 && b[u].z != 0, v3 = a.w != 0 && b[u].w != 0;
+        valid[u] += count(v0) + count(v1) + count(v2) + count(v3);
+        same[u] += count(v0 && a.x == b[u].x) + count(v1 && a.y == b[u].y) + count(v2 && a.z == b[u].z) +
+                   count(v3 && a.w == b[u].w);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kInFlight; ++u) {
+      const int j = j0 + u * kEdges + group;
+      if (slot == 0 && j < neighbors) {
+        keys[j] = static_cast<unsigned long long>(static_cast<uint32_t>(same[u])) << 32 | static_cast<uint32_t>(valid[u]);
+      }
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  for (int e = lane; e < neighbors; e += kWave) {
+    const int stored = indices[base + e];
     const int nb = stored >= 0 && input_one_based ? stored - 1 : stored;
-    float d = distances[base + j];
+    float d = distances[base + e];
     int out_id = stored;
     if (nb >= 0 && nb < samples && isfinite(d)) {
-      int same = 0, valid = 0;
-      for (int q0 = 0; q0 < quads; q0 += kWave) {
-        const int q = q0 + lane;
-        int4 a = make_int4(0, 0, 0, 0), b = make_int4(0, 0, 0, 0);
-        if (q < quads) {
-          a = lab4[static_cast<size_t>(row) * quads + q];
-          b = lab4[static_cast<size_t>(nb) * quads + q];
-        }
-        const bool v0 = a.x != 0 && b.x != 0, v1 = a.y != 0 && b.y != 0;
-        const bool v2 = a.z != 0 && b.z != 0, v3 = a.w != 0 && b.w != 0;
-        valid += __popcll(__ballot(v0)) + __popcll(__ballot(v1)) + __popcll(__ballot(v2)) + __popcll(__ballot(v3));
-        same += __popcll(__ballot(v0 && a.x == b.x)) + __popcll(__ballot(v1 && a.y == b.y)) +
-                __popcll(__ballot(v2 && a.z == b.z)) + __popcll(__ballot(v3 && a.w == b.w));
-      }
+      const int same = static_cast<int>(keys[e] >> 32), valid = static_cast<int>(static_cast<uint32_t>(keys[e]));
       if (same == 0 || valid == 0) {
         d = INFINITY;
       } else {
@@ -118,20 +157,20 @@ dissimilarity_kernel(int* __restrict__ indices, float* __restrict__ distances, i
     } else {
       d = INFINITY;
     }
-    if (lane == 0) {
-      keys[j] = (static_cast<unsigned long long>(ordered_bits(d)) << 32) |
-                static_cast<unsigned long long>(static_cast<uint32_t>(out_id) ^ 0x80000000u);
-      ids[j] = out_id;
-    }
+    keys[e] = (static_cast<unsigned long long>(ordered_bits(d)) << 32) |
+              static_cast<unsigned long long>(static_cast<uint32_t>(out_id) ^ 0x80000000u);
+    ids[e] = out_id;
   }
-  __syncthreads();  // orders lane 0's LDS writes before the other lanes' reads
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
   // Stable order by (distance, id): rank = smaller keys + equal keys earlier.
-  for (int e = lane; live && e < neighbors; e += kWave) {
+  for (int e = lane; e < neighbors; e += kWave) {
     const unsigned long long ke = keys[e];
     int rank = 0;
+#pragma unroll 8
     for (int f = 0; f < neighbors; ++f) {
       const unsigned long long kf = keys[f];
-      rank += (kf < ke || (kf == ke && f < e)) ? 1 : 0;
+      rank += (kf < ke ? 1 : 0) + (kf == ke && f < e ? 1 : 0);
     }
     const uint32_t bits = static_cast<uint32_t>(ke >> 32);
     const uint32_t fb = (bits & 0x80000000u) ? (bits & 0x7FFFFFFFu) : ~bits;
@@ -186,9 +225,15 @@ hipError_t launch_dissimilarity(int* indices, float* distances, int samples, int
   if (samples == 0 || neighbors == 0) return hipSuccess;
   if (stride % 4 != 0 || dissimilarity_lds_bytes(neighbors) > 64 * 1024) return hipErrorInvalidValue;
   const unsigned blocks = static_cast<unsigned>((samples + kRowsPerBlock - 1) / kRowsPerBlock);
-  hipLaunchKernelGGL(dissimilarity_kernel, dim3(blocks), dim3(kWave * kRowsPerBlock),
-                     dissimilarity_lds_bytes(neighbors), s, indices, distances, samples, neighbors, labels, stride,
-                     input_one_based ? 1 : 0, output_one_based ? 1 : 0);
+  if (stride <= 4 * 32) {
+    hipLaunchKernelGGL((dissimilarity_kernel<32>), dim3(blocks), dim3(kWave * kRowsPerBlock),
+                       dissimilarity_lds_bytes(neighbors), s, indices, distances, samples, neighbors, labels, stride,
+                       input_one_based ? 1 : 0, output_one_based ? 1 : 0);
+  } else {
+    hipLaunchKernelGGL((dissimilarity_kernel<64>), dim3(blocks), dim3(kWave * kRowsPerBlock),
+                       dissimilarity_lds_bytes(neighbors), s, indices, distances, samples, neighbors, labels, stride,
+                       input_one_based ? 1 : 0, output_one_based ? 1 : 0);
+  }
   return hipGetLastError();
 }
 
