@@ -21,8 +21,8 @@ inline int stream_width(int p, int parts, bool euclid) { return parts * p + (euc
 inline int stream_steps(int p, int parts, bool euclid) { return (stream_width(p, parts, euclid) + 31) / 32; }
 // Candidates kept per query and slice (list 8, k <= 32: 128; list 16: 256).
 inline int stream_capacity(int list) { return 16 * list; }
-// Queries per wave of the candidates: four 16-query tiles, two where the
-// operands are wide.
+// Queries per wave of the maxima and candidates: two 32-query tiles, one where
+// the operands are wide.
 inline int stream_queries_per_wave(int steps) { return steps <= 4 ? 64 : 32; }
 // Slices of the maxima at least: 2.1 k class maxima place the k-th largest of
 // them at about the 1.4 k-th largest score.
@@ -73,7 +73,9 @@ hipError_t launch_stream_norms(const float* x, int rows, int p, int stride, floa
                                hipStream_t s);
 inline int stream_row_stride(int p) { return (p + 3) / 4 * 4; }
 // Rows -> operand fragments of `steps` x 32 columns, rows padded with zeros to
-// pad_rows; either output may be null. norm2_max [2] scales them.
+// pad_rows; either output may be null. norm2_max [2] scales them. `tile` rows a
+// fragment: 32 (x 16 columns, v_mfma_f32_32x32x16_f16) or 16 (x 32 columns,
+// v_mfma_f32_16x16x32_f16).
 // For the padded table layout pass block_run / run_offsets / pad_offsets.
 struct StreamOperandJob {
   const float* x = nullptr;
@@ -81,7 +83,8 @@ struct StreamOperandJob {
   const float* norm2 = nullptr;
   const float* norm2_max = nullptr;
   int rows = 0, p = 0, parts = 1, euclid = 0;
-  int pad_rows = 0;                 // multiple of 16
+  int tile = 32;
+  int pad_rows = 0;                 // multiple of tile
   int group_rows = 0, group_pad = 0;  // equal groups of group_rows rows, padded to group_pad (0: one group)
   const int* block_run = nullptr;   // tables: run of each 256 padded rows
   const int* run_offsets = nullptr;

@@ -7,16 +7,18 @@
 // 2^14, rounded to FP16 (parts = 1) or split into two FP16 parts (parts = 3:
 // hi.hi + hi.lo + lo.hi along K), and the norm term rides in spare K columns
 // (2^13 on the query side, the FP16 parts of -|t|^2 / 2^14 on the train
-// side), so one v_mfma_f32_16x16x32_f16 chain gives s for 16 x 16 pairs. Each
+// side), so one v_mfma_f32_32x32x16_f16 chain gives s for 32 x 32 pairs. Each
 // s differs from the exact distance's by at most E (pair_error below).
 //
-// Three kernels stream the train rows (a wave owns 16 NQ queries as B operands
+// Three kernels stream the train rows (a wave owns 32 NQ queries as B operands
 // in registers; train rows go through LDS 64 at a time in the fragment order
 // of the A operand, so staging and reads are linear; output lane l holds query
-// l % 16 against train rows 4 (l / 16) + r):
+// l % 32 against train rows 8 (r / 4) + 4 (l / 32) + r % 4, r = 0..15). The
+// 32 x 32 products reach 1.8 PFLOP/s here on random operands (2.45 on zeros),
+// the 16 x 16 ones 1.25 (1.36), measured with operands held in registers.
 //
 // knn_maxima_kernel, over all rows or a sample of about 1000 k: each lane
-// keeps the largest score of each of its 8 row classes (half a three-way
+// keeps the largest score of each of its 16 row classes (half a three-way
 // maximum per pair, no branch). A query has 32 classes per slice of the
 // sample, at least 2.1 k in all.
 // knn_threshold_kernel: T = the k-th largest of a query's class maxima (all of
@@ -24,10 +26,17 @@
 // score), threshold T - 2E: the k-th best exact distance belongs to a
 // score >= T - E, so every row of the true k nearest scores >= T - 2E.
 // knn_candidates_kernel, over all rows: a pair below its query's threshold is
-// dropped with one maximum and one compare per four pairs; the others are
+// dropped with one maximum per two pairs and one compare per 16; the others are
 // appended to the query's candidate buffer. Where the sample was a part of the
 // rows the buffer may run full; the wave then tightens T from the buffer
 // itself (bisection over ballots) and drops what falls below.
+// At 1M rows the matrix cores are busy 47 % of the cycles at 1.9 GHz (the
+// maxima: 71 % at 1.5; the card holds 1.7 of its 2.4 GHz under bare products
+// of such operands, so power is the outer limit); the rest is a wave with
+// pairs to append, nearly every stage, holding the other three at its barrier.
+// 128 queries per wave, half the LDS traffic and half the waves: 161 ms
+// against 134. The pairs queued in LDS and drained 64 at a time: 507 ms (the
+// queue's code spills registers in the loop).
 // Two passes of MFMAs with 1.4 k appends per query cost less than one
 // pass with lists or a running threshold (k ln(n / k) appends): an append
 // takes as long as the MFMAs of some 1000 pairs.
@@ -45,12 +54,12 @@
 // Queries whose bound kept more than the buffer holds (many near-equal
 // distances) are flagged for another path.
 //
-// Measured on one MI355X: the self graph of 1M x 50, k = 30, maxima 3.5 ms,
-// candidates 130 ms (7.7e12 pairs/s, 0.98 PFLOP/s of FP16 with the padding to
+// Measured on one MI355X: the self graph of 1M x 50, k = 30, maxima 3.6 ms,
+// candidates 134 ms (7.5e12 pairs/s, 0.95 PFLOP/s of FP16 with the padding to
 // 64 columns), rerank 4.1 ms (5.4 with 4-byte loads, a bound for every query and
 // keys of two words); split-BF16 products with sorted lists per lane
-// column took 871 + 34 ms for the candidates. 100k x 50, k = 100: 1.0 + 2.8 +
-// 1.06 ms (1.5) against 26.6 + 18.9 (scan of the queries the lists could not
+// column took 871 + 34 ms for the candidates. 100k x 50, k = 100: 1.05 + 2.55
+// (3.0 with 16 x 16 products, which take as long at 1M rows) + 1.06 ms (1.5) against 26.6 + 18.9 (scan of the queries the lists could not
 // certify) + 1.3. 10007 x 30011 x 100, k = 30: 0.33 ms against 23.1 ms of the
 // register scan. A running threshold without the maxima appended 3.5 times as
 // much: 316 ms at 1M rows, 18.3 ms at 100k.
@@ -69,7 +78,10 @@ namespace kodama_hip {
 namespace {
 
 constexpr int kWave = 64;
+constexpr int kTile = 32;   // rows of an operand fragment and of an MFMA
 constexpr int kChunk = 64;  // train rows per LDS stage
+// Train row, in its tile of 32, of output register r in the wave's half h.
+constexpr int tile_row(int r) { return 8 * (r / 4) + r % 4; }  // + 4 h
 
 // A key that at least k of the wave's keys (R per lane, 0 = empty, at least k
 // non-empty) reach and at most k + 2 unless ties or `exact`: bisection on
@@ -131,17 +143,19 @@ __global__ void stream_norms_kernel(const float* __restrict__ x, int rows, int p
   if (threadIdx.x == 0 && s_max != 0u) atomicMax(reinterpret_cast<uint32_t*>(norm2_max), s_max);
 }
 
-// One thread per 16-byte fragment piece: piece ((tile * steps + step) * 64 +
-// lane) holds row tile * 16 + lane % 16, columns step * 32 + 8 (lane / 16)
-// .. + 7. Blocks cover 256 pieces; reads are 8 consecutive floats of 16 rows.
+// One thread per 16-byte fragment piece: with fragments of T rows (32 or 16)
+// and 512 / T columns, piece ((tile * (steps T / 16) + step) * 64 + lane)
+// holds row tile * T + lane % T, columns step * 512 / T + 8 (lane / T) .. + 7.
+// Blocks cover 256 pieces; reads are 8 consecutive floats a lane.
 __global__ void stream_operands_kernel(StreamOperandJob job, int steps) {
   const size_t e = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const size_t total = static_cast<size_t>(job.pad_rows) / 16 * steps * 64;
   if (e >= total) return;
   const int lane = static_cast<int>(e & 63);
+  const int tile = job.tile, fragments = steps * tile / 16;
   const size_t ts = e >> 6;
-  const int step = static_cast<int>(ts % steps);
-  const int prow = static_cast<int>(ts / steps) * 16 + (lane & 15);
+  const int step = static_cast<int>(ts % fragments);
+  const int prow = static_cast<int>(ts / fragments) * tile + (lane & (tile - 1));
   int row = prow;
   bool live = prow < job.rows;
   if (job.group_pad > 0) {
@@ -157,7 +171,7 @@ __global__ void stream_operands_kernel(StreamOperandJob job, int steps) {
   }
   const float scale = operand_scale(job.norm2_max);
   const int p = job.p;
-  const int c0 = step * 32 + 8 * (lane >> 4);
+  const int c0 = step * (512 / tile) + 8 * (lane / tile);
   _Float16 tv[8], qv[8];
   const float* src = job.x + static_cast<size_t>(live ? row : 0) * (job.stride != 0 ? job.stride : p);
   const float nt = live && job.euclid ? -(job.norm2[row] * scale) * scale * 0x1p-14f : 0.0f;
@@ -222,63 +236,78 @@ __device__ __forceinline__ StreamRange stream_range(const KnnStreamParams& prm, 
 // LDS staging of 64 train rows: the next chunk is loaded into registers while
 // this one is scored; two buffers, one barrier per chunk.
 constexpr int kThreads = 256;
-template <int KS>
+template <int KS, bool FOLDS>
 __device__ __forceinline__ void fetch_chunk(const KnnStreamParams& prm, const StreamRange& g, int c0, u32x4 (&pre)[KS],
                                             int& pre_grp) {
-  const u32x4* src = reinterpret_cast<const u32x4*>(prm.train_op) + static_cast<size_t>(c0 / 16) * (KS * 64);
+  const u32x4* src = reinterpret_cast<const u32x4*>(prm.train_op) + static_cast<size_t>(c0 / kTile) * (2 * KS * 64);
 #pragma unroll
   for (int i = 0; i < KS; ++i) pre[i] = src[static_cast<int>(threadIdx.x) + i * kThreads];
-  if (prm.folds != nullptr && threadIdx.x < kChunk) {
+  if (FOLDS && threadIdx.x < kChunk) {
     const int j = c0 + static_cast<int>(threadIdx.x);
     pre_grp = j < g.t_end ? prm.folds[j + g.delta] : -2;
   }
 }
-template <int KS>
+template <int KS, bool FOLDS>
 __device__ __forceinline__ void store_chunk(const KnnStreamParams& prm, const u32x4 (&pre)[KS], int pre_grp, u32x4* s_t,
                                             int* s_grp) {
 #pragma unroll
   for (int i = 0; i < KS; ++i) s_t[static_cast<int>(threadIdx.x) + i * kThreads] = pre[i];
-  if (prm.folds != nullptr && threadIdx.x < kChunk) s_grp[threadIdx.x] = pre_grp;
+  if (FOLDS && threadIdx.x < kChunk) s_grp[threadIdx.x] = pre_grp;
 }
 
 template <int KS, int NQ>
 __device__ __forceinline__ void load_queries(const KnnStreamParams& prm, int q_wave, int q_end, int lane,
-                                             f16x8 (&bq)[NQ][KS]) {
+                                             f16x8 (&bq)[NQ][2 * KS]) {
 #pragma unroll
   for (int t = 0; t < NQ; ++t) {
     // Operand tiles exist for the padded rows; a wave past them reads none.
     const u32x4* src =
-        reinterpret_cast<const u32x4*>(prm.query_op) + (static_cast<size_t>(q_wave / 16 + t) * KS) * 64 + lane;
-    const bool tile = q_wave + t * 16 < q_end;
+        reinterpret_cast<const u32x4*>(prm.query_op) + (static_cast<size_t>(q_wave / kTile + t) * (2 * KS)) * 64 + lane;
+    const bool tile = q_wave + t * kTile < q_end;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) bq[t][ks] = as_f16x8(tile ? src[ks * 64] : u32x4{0, 0, 0, 0});
+    for (int ks = 0; ks < 2 * KS; ++ks) bq[t][ks] = as_f16x8(tile ? src[ks * 64] : u32x4{0, 0, 0, 0});
   }
 }
 
-// KS: 32-deep steps. NQ: 16-query tiles per wave. blockIdx.x: query block,
+// Scores of one tile of train rows against the wave's queries.
+template <int KS, int NQ>
+__device__ __forceinline__ void score_tile(const u32x4* s_tile, int lane, const f16x8 (&bq)[NQ][2 * KS],
+                                           f32x16 (&acc)[NQ]) {
+  const f32x16 zero = {};
+#pragma unroll
+  for (int ks = 0; ks < 2 * KS; ++ks) {
+    const f16x8 a = as_f16x8(s_tile[ks * 64 + lane]);
+#pragma unroll
+    for (int t = 0; t < NQ; ++t) {
+      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, bq[t][ks], ks == 0 ? zero : acc[t], 0, 0, 0);
+    }
+  }
+}
+
+// KS: 32 columns of the operands each. NQ: 32-query tiles per wave. blockIdx.x: query block,
 // blockIdx.y: share of the sampled chunks.
 template <int KS, int NQ, bool FOLDS>
 __global__ void __launch_bounds__(256, KS <= 2 ? 3 : 2) knn_maxima_kernel(KnnStreamParams prm) {
-  constexpr int kWaveQueries = NQ * 16;
+  constexpr int kWaveQueries = NQ * kTile;
   __shared__ u32x4 s_t[2][KS * kThreads];  // 64 rows x KS x 64 bytes
   __shared__ int s_grp[2][FOLDS ? kChunk : 4];
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
-  const int grp = lane >> 4, col = lane & 15;
+  const int half = lane / kTile, col = lane % kTile;
   const int q_block = blockIdx.x * (4 * kWaveQueries);
   const StreamRange g = stream_range(prm, q_block);
   if (q_block >= g.q_end) return;
   const int q_wave = q_block + wave * kWaveQueries;
-  f16x8 bq[NQ][KS];
+  f16x8 bq[NQ][2 * KS];
   load_queries<KS, NQ>(prm, q_wave, g.q_end, lane, bq);
   int fold[NQ];
-  float top[NQ][8];  // class 2 sub + r / 2
+  float top[NQ][16];  // class 8 sub + r / 2
 #pragma unroll
   for (int t = 0; t < NQ; ++t) {
-    const int q = q_wave + t * 16 + col;
+    const int q = q_wave + t * kTile + col;
     fold[t] = FOLDS && q < g.q_end ? prm.folds[q + g.delta] : -1;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) top[t][i] = -INFINITY;
+    for (int i = 0; i < 16; ++i) top[t][i] = -INFINITY;
   }
   // Sampled chunks, evenly spread and distinct (a row counted in two classes
   // would spoil the threshold): chunk i of `picked` is floor(i chunks / picked).
@@ -293,66 +322,67 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 3 : 2) knn_maxima_kernel(KnnStr
   u32x4 pre[KS];
   int pre_grp = -2;
   if (i0 < i1) {
-    fetch_chunk<KS>(prm, g, chunk_row(i0), pre, pre_grp);
-    store_chunk<KS>(prm, pre, pre_grp, s_t[0], s_grp[0]);
+    fetch_chunk<KS, FOLDS>(prm, g, chunk_row(i0), pre, pre_grp);
+    store_chunk<KS, FOLDS>(prm, pre, pre_grp, s_t[0], s_grp[0]);
   }
   __builtin_amdgcn_s_waitcnt(0);  // the operands too: no wait for them (and the prefetch) in the loop
   __syncthreads();
   int buf = 0;
   for (int i = i0; i < i1; ++i, buf ^= 1) {
-    if (i + 1 < i1) fetch_chunk<KS>(prm, g, chunk_row(i + 1), pre, pre_grp);
+    if (i + 1 < i1) fetch_chunk<KS, FOLDS>(prm, g, chunk_row(i + 1), pre, pre_grp);
     const int c0 = chunk_row(i);
     // `cut`: rows past the end (the last chunk only) must not count.
     auto score = [&](auto cut) {
 #pragma unroll
-      for (int sub = 0; sub < kChunk / 16; ++sub) {
-        f32x4 acc[NQ];
-#pragma unroll
-        for (int t = 0; t < NQ; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          const f16x8 a = as_f16x8(s_t[buf][(sub * KS + ks) * 64 + lane]);
-#pragma unroll
-          for (int t = 0; t < NQ; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq[t][ks], acc[t], 0, 0, 0);
-        }
+      for (int sub = 0; sub < kChunk / kTile; ++sub) {
+        f32x16 acc[NQ];
+        score_tile<KS, NQ>(&s_t[buf][sub * 2 * KS * 64], lane, bq, acc);
         if constexpr (decltype(cut)::value) {
-          const int j0 = c0 + sub * 16 + 4 * grp;
+          const int j0 = c0 + sub * kTile + 4 * half;
 #pragma unroll
           for (int t = 0; t < NQ; ++t) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[t][r] = j0 + r < g.t_end ? acc[t][r] : -INFINITY;
+            for (int r = 0; r < 16; ++r) acc[t][r] = j0 + tile_row(r) < g.t_end ? acc[t][r] : -INFINITY;
           }
         }
         if constexpr (FOLDS) {
-          const int4 f = *reinterpret_cast<const int4*>(&s_grp[buf][sub * 16 + 4 * grp]);
 #pragma unroll
-          for (int t = 0; t < NQ; ++t) {
-            acc[t][0] = f.x != fold[t] ? acc[t][0] : -INFINITY;
-            acc[t][1] = f.y != fold[t] ? acc[t][1] : -INFINITY;
-            acc[t][2] = f.z != fold[t] ? acc[t][2] : -INFINITY;
-            acc[t][3] = f.w != fold[t] ? acc[t][3] : -INFINITY;
+          for (int b = 0; b < 4; ++b) {
+            const int4 f = *reinterpret_cast<const int4*>(&s_grp[buf][sub * kTile + 8 * b + 4 * half]);
+#pragma unroll
+            for (int t = 0; t < NQ; ++t) {
+              acc[t][4 * b] = f.x != fold[t] ? acc[t][4 * b] : -INFINITY;
+              acc[t][4 * b + 1] = f.y != fold[t] ? acc[t][4 * b + 1] : -INFINITY;
+              acc[t][4 * b + 2] = f.z != fold[t] ? acc[t][4 * b + 2] : -INFINITY;
+              acc[t][4 * b + 3] = f.w != fold[t] ? acc[t][4 * b + 3] : -INFINITY;
+            }
           }
         }
 #pragma unroll
         for (int t = 0; t < NQ; ++t) {
-          top[t][2 * sub] = fmaxf(fmaxf(top[t][2 * sub], acc[t][0]), acc[t][1]);
-          top[t][2 * sub + 1] = fmaxf(fmaxf(top[t][2 * sub + 1], acc[t][2]), acc[t][3]);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            float& c = top[t][8 * sub + i];
+            c = fmaxf(fmaxf(c, acc[t][2 * i]), acc[t][2 * i + 1]);
+          }
         }
       }
     };
     if (c0 + kChunk > g.t_end) score(std::true_type{});
     else score(std::false_type{});
-    if (i + 1 < i1) store_chunk<KS>(prm, pre, pre_grp, s_t[buf ^ 1], s_grp[buf ^ 1]);
+    if (i + 1 < i1) store_chunk<KS, FOLDS>(prm, pre, pre_grp, s_t[buf ^ 1], s_grp[buf ^ 1]);
     __syncthreads();
   }
 #pragma unroll
   for (int t = 0; t < NQ; ++t) {
-    const int q = q_wave + t * 16 + col;
+    const int q = q_wave + t * kTile + col;
     if (q < g.q_end) {
       float4* dst = reinterpret_cast<float4*>(prm.maxima + (static_cast<size_t>(q) * prm.max_slices + blockIdx.y) * 32 +
-                                              grp * 8);
-      dst[0] = make_float4(top[t][0], top[t][1], top[t][2], top[t][3]);
-      dst[1] = make_float4(top[t][4], top[t][5], top[t][6], top[t][7]);
+                                              half * 16);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dst[i] = make_float4(top[t][4 * i], top[t][4 * i + 1], top[t][4 * i + 2], top[t][4 * i + 3]);
+      }
     }
   }
 }
@@ -394,17 +424,20 @@ __global__ void __launch_bounds__(256) knn_threshold_kernel(KnnStreamParams prm,
 }
 
 // R: capacity / 64. blockIdx.x: query block, blockIdx.y: slice of the train rows.
-template <int KS, int NQ, int R>
+template <int KS, int NQ, int R, bool FOLDS>
 __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(KnnStreamParams prm) {
   constexpr int kCap = 64 * R;
-  constexpr int kWaveQueries = NQ * 16;
+  constexpr int kFull = kCap - kTile;      // a tile of train rows may add 32 to a query
+  constexpr int kCompact = kFull - 8;
+  constexpr int kWaveQueries = NQ * kTile;
   __shared__ u32x4 s_t[2][KS * kThreads];  // 64 rows x KS x 64 bytes
-  __shared__ int s_grp[2][kChunk];
+  __shared__ int s_grp[2][FOLDS ? kChunk : 4];
   __shared__ int s_cnt[4][kWaveQueries];
   __shared__ float s_th[4][kWaveQueries];
+  __shared__ int s_ex[4][kWaveQueries];
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
-  const int grp = lane >> 4, col = lane & 15;
+  const int half = lane / kTile, col = lane % kTile;
   const int q_block = blockIdx.x * (4 * kWaveQueries);
   StreamRange g = stream_range(prm, q_block);
   if (q_block >= g.q_end) return;
@@ -419,23 +452,23 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(Kn
   const size_t slot0 = static_cast<size_t>(q_wave) * prm.slices + blockIdx.y;  // query i: + i * slices
   const bool usable = norms_usable(prm.norm2_max);
 
-  f16x8 bq[NQ][KS];
+  f16x8 bq[NQ][2 * KS];
   load_queries<KS, NQ>(prm, q_wave, g.q_end, lane, bq);
   float th[NQ];
-  int ex[NQ];
 #pragma unroll
   for (int t = 0; t < NQ; ++t) {
-    const int q = q_wave + t * 16 + col;
+    const int q = q_wave + t * kTile + col;
     const bool live = q < g.q_end;
     th[t] = live ? prm.threshold[q] : INFINITY;
-    ex[t] = -1;
-    if (live) {
-      if (prm.folds != nullptr) ex[t] = prm.folds[q + g.delta];
-      else if (prm.exclude != nullptr) ex[t] = prm.exclude[q];
-    }
-    if (grp == 0) {
-      s_cnt[wave][t * 16 + col] = usable ? 0 : -1;
-      s_th[wave][t * 16 + col] = th[t];
+    if (half == 0) {
+      int ex = -1;  // the query's own fold or row
+      if (live) {
+        if (FOLDS) ex = prm.folds[q + g.delta];
+        else if (prm.exclude != nullptr) ex = prm.exclude[q];
+      }
+      s_ex[wave][t * kTile + col] = ex;
+      s_cnt[wave][t * kTile + col] = usable ? 0 : -1;
+      s_th[wave][t * kTile + col] = th[t];
     }
   }
 
@@ -473,7 +506,7 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(Kn
         if (keep) base[kept + __popcll(m & below)] = ent[i];
         kept += __popcll(m);
       }
-      const bool over = kept > kCap - 32;
+      const bool over = kept > kCompact;
       if (lane == 0) {
         s_cnt[wave][q] = over ? -1 : kept;
         s_th[wave][q] = over ? INFINITY : fmaxf(bound, s_th[wave][q]);
@@ -482,81 +515,74 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(Kn
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int t = 0; t < NQ; ++t) th[t] = s_th[wave][t * 16 + col];
+    for (int t = 0; t < NQ; ++t) th[t] = s_th[wave][t * kTile + col];
   };
 
   u32x4 pre[KS];
   int pre_grp = -2;
   if (g.t_begin < g.t_end) {
-    fetch_chunk<KS>(prm, g, g.t_begin, pre, pre_grp);
-    store_chunk<KS>(prm, pre, pre_grp, s_t[0], s_grp[0]);
+    fetch_chunk<KS, FOLDS>(prm, g, g.t_begin, pre, pre_grp);
+    store_chunk<KS, FOLDS>(prm, pre, pre_grp, s_t[0], s_grp[0]);
   }
   __builtin_amdgcn_s_waitcnt(0);  // the operands too: no wait for them (and the prefetch) in the loop
   __syncthreads();
   int buf = 0;
   for (int c0 = g.t_begin; c0 < g.t_end; c0 += kChunk, buf ^= 1) {
     const bool more = c0 + kChunk < g.t_end;
-    if (more) fetch_chunk<KS>(prm, g, c0 + kChunk, pre, pre_grp);  // in flight during the scoring
+    if (more) fetch_chunk<KS, FOLDS>(prm, g, c0 + kChunk, pre, pre_grp);  // in flight during the scoring
     const int limit = more ? c0 + kChunk : g.t_end;
 #pragma unroll 1
-    for (int sub = 0; sub < kChunk / 16; ++sub) {
-      f32x4 acc[NQ];
-#pragma unroll
-      for (int t = 0; t < NQ; ++t) acc[t] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const f16x8 a = as_f16x8(s_t[buf][(sub * KS + ks) * 64 + lane]);
-#pragma unroll
-        for (int t = 0; t < NQ; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq[t][ks], acc[t], 0, 0, 0);
-      }
+    for (int sub = 0; sub < kChunk / kTile; ++sub) {
+      f32x16 acc[NQ];
+      score_tile<KS, NQ>(&s_t[buf][sub * 2 * KS * 64], lane, bq, acc);
       uint64_t hit[NQ], any = 0ull;
 #pragma unroll
       for (int t = 0; t < NQ; ++t) {
-        // Strictly above (the bound has slack): two three-way maxima and a compare.
-        hit[t] = __ballot(fmaxf(fmaxf(fmaxf(fmaxf(th[t], acc[t][0]), acc[t][1]), acc[t][2]), acc[t][3]) > th[t]);
+        // Strictly above (the bound has slack): eight three-way maxima and a compare.
+        float top = th[t];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) top = fmaxf(fmaxf(top, acc[t][2 * i]), acc[t][2 * i + 1]);
+        hit[t] = __ballot(top > th[t]);
         any |= hit[t];
       }
       if (any != 0ull) {
-        const int j0 = c0 + sub * 16 + 4 * grp;
-        int4 gr = make_int4(j0, j0 + 1, j0 + 2, j0 + 3);
-        if (prm.folds != nullptr) gr = *reinterpret_cast<const int4*>(&s_grp[buf][sub * 16 + 4 * grp]);
-        const int row[4] = {gr.x, gr.y, gr.z, gr.w};
+        const int in_chunk = sub * kTile + 4 * half;
+        int c_of = col;  // opaque: no buffer addresses kept in registers over the loop
+        asm volatile("" : "+v"(c_of));
         bool full = false;
 #pragma unroll
         for (int t = 0; t < NQ; ++t) {
           if (hit[t] == 0ull) continue;
-          bool pass[4];
-          int c = 0;
+          const int qi = t * kTile + c_of;
+          const int ex = s_ex[wave][qi];
+          uint2* dst = prm.cand + (slot0 + static_cast<size_t>(qi) * prm.slices) * kCap;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            pass[r] = acc[t][r] > th[t] && row[r] != ex[t] && j0 + r < limit;
-            c += pass[r] ? 1 : 0;
-          }
-          if (c > 0) {
-            // The lane's next slots of its query (four lanes share one).
-            const int slot = atomicAdd(&s_cnt[wave][t * 16 + col], c);
-            uint2* dst = prm.cand + (slot0 + static_cast<size_t>(t * 16 + col) * prm.slices) * kCap + slot;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              if (pass[r]) *dst++ = make_uint2(__float_as_uint(acc[t][r]), static_cast<uint32_t>(j0 + r + g.delta));
+          for (int r = 0; r < 16; ++r) {
+            const bool above = acc[t][r] > th[t];
+            if (__ballot(above) == 0ull) continue;
+            const int j = c0 + in_chunk + tile_row(r);
+            const int group = FOLDS ? s_grp[buf][in_chunk + tile_row(r)] : j;
+            if (above && group != ex && j < limit) {
+              const int slot = atomicAdd(&s_cnt[wave][qi], 1);
+              dst[slot] = make_uint2(__float_as_uint(acc[t][r]), static_cast<uint32_t>(j + g.delta));
+              full = full || slot >= kFull;
             }
-            full = full || slot + c > kCap - 16;
           }
         }
-        if (__ballot(full) != 0ull) compact(kCap - 32);
+        if (__ballot(full) != 0ull) compact(kCompact);
       }
     }
-    if (more) store_chunk<KS>(prm, pre, pre_grp, s_t[buf ^ 1], s_grp[buf ^ 1]);
+    if (more) store_chunk<KS, FOLDS>(prm, pre, pre_grp, s_t[buf ^ 1], s_grp[buf ^ 1]);
     __syncthreads();
   }
   // Several slices: keep each list short enough for the rerank to hold all.
   if (prm.slices > 1) compact(max(prm.k + 8, 24));
 #pragma unroll
   for (int t = 0; t < NQ; ++t) {
-    const int q = q_wave + t * 16 + col;
-    if (grp == 0 && q < g.q_end) {
-      const size_t o = slot0 + static_cast<size_t>(t * 16 + col) * prm.slices;
-      prm.cand_count[o] = s_cnt[wave][t * 16 + col];
+    const int q = q_wave + t * kTile + col;
+    if (half == 0 && q < g.q_end) {
+      const size_t o = slot0 + static_cast<size_t>(t * kTile + col) * prm.slices;
+      prm.cand_count[o] = s_cnt[wave][t * kTile + col];
       prm.cand_bound[o] = th[t];
     }
   }
@@ -751,7 +777,7 @@ hipError_t launch_stream_norms(const float* x, int rows, int p, int stride, floa
 hipError_t launch_stream_operands(const StreamOperandJob& job, hipStream_t s) {
   if (job.pad_rows == 0) return hipSuccess;
   const int steps = stream_steps(job.p, job.parts, job.euclid != 0);
-  if (job.pad_rows % 16 != 0 || job.p < 1 || steps > kStreamMaxSteps ||
+  if ((job.tile != 16 && job.tile != 32) || job.pad_rows % job.tile != 0 || job.p < 1 || steps > kStreamMaxSteps ||
       (job.parts != 1 && job.parts != 3)) {
     return hipErrorInvalidValue;
   }
@@ -764,8 +790,8 @@ hipError_t launch_stream_operands(const StreamOperandJob& job, hipStream_t s) {
 template <int KS>
 static void launch_steps(const KnnStreamParams& prm, hipStream_t s) {
   const int rows = prm.block_run != nullptr ? prm.pad_rows : prm.query_rows;
-  constexpr int NQ = KS <= 4 ? 4 : 2;
-  const int qpb = 4 * NQ * 16;
+  constexpr int NQ = KS <= 4 ? 2 : 1;
+  const int qpb = 4 * NQ * kTile;
   const unsigned qblocks = static_cast<unsigned>((rows + qpb - 1) / qpb);
   const dim3 mgrid(qblocks, static_cast<unsigned>(prm.max_slices));
   if (prm.folds != nullptr) hipLaunchKernelGGL((knn_maxima_kernel<KS, NQ, true>), mgrid, dim3(256), 0, s, prm);
@@ -777,8 +803,13 @@ static void launch_steps(const KnnStreamParams& prm, hipStream_t s) {
   else if (per_query <= 256) hipLaunchKernelGGL((knn_threshold_kernel<4>), tgrid, dim3(256), 0, s, prm, rows, per_query);
   else hipLaunchKernelGGL((knn_threshold_kernel<8>), tgrid, dim3(256), 0, s, prm, rows, per_query);
   const dim3 grid(qblocks, static_cast<unsigned>(prm.slices));
-  if (prm.list == 8) hipLaunchKernelGGL((knn_candidates_kernel<KS, NQ, 2>), grid, dim3(256), 0, s, prm);
-  else hipLaunchKernelGGL((knn_candidates_kernel<KS, NQ, 4>), grid, dim3(256), 0, s, prm);
+  if (prm.folds != nullptr) {
+    if (prm.list == 8) hipLaunchKernelGGL((knn_candidates_kernel<KS, NQ, 2, true>), grid, dim3(256), 0, s, prm);
+    else hipLaunchKernelGGL((knn_candidates_kernel<KS, NQ, 4, true>), grid, dim3(256), 0, s, prm);
+  } else {
+    if (prm.list == 8) hipLaunchKernelGGL((knn_candidates_kernel<KS, NQ, 2, false>), grid, dim3(256), 0, s, prm);
+    else hipLaunchKernelGGL((knn_candidates_kernel<KS, NQ, 4, false>), grid, dim3(256), 0, s, prm);
+  }
 }
 
 hipError_t launch_knn_stream(const KnnStreamParams& prm, hipStream_t s) {

@@ -143,6 +143,7 @@ struct DeviceLloyd {
   }
   StreamOperandJob operand_job(const float* x, const float* norm2, int rows, int pad) const {
     StreamOperandJob op;
+    op.tile = 16;
     op.x = x;
     op.norm2 = norm2;
     op.norm2_max = norm2_max.get();
