@@ -663,6 +663,7 @@ void KnnBatch::allocate(const IVec& run_offsets) {
   h_counts_.resize(static_cast<size_t>(runs_) * classes_);
   h_firsts_.resize(static_cast<size_t>(runs_) * classes_);
   h_matches_.resize(static_cast<size_t>(runs_));
+  check(launch_vote_reset(d_counts_.get(), d_firsts_.get(), d_matches_.get(), runs_, classes_, s), "vote reset");
   // Device-evolution staging: 16-bit labels per padded row plus per-run words
   // (keys, widths, state, the elapsed ticks of up to eight workgroups), and
   // the accuracy history of up to 128 cycles.
@@ -764,15 +765,18 @@ KnnBatch::~KnnBatch() {
   if (graph_ != nullptr) (void)hipGraphDestroy(graph_);
 }
 
+// No copy where the kernels can do it: they write the predictions and the
+// reductions to pinned host memory, and labels of which all blocks together
+// read kDirectLabelBytes or less are staged from there as well (every block of
+// a run stages the whole run: 64 KiB for 2000 rows, 16 MB for 100 runs of
+// 3500, against 0.06 ms of the copy). The vote is bound by these round trips:
+// 2000 rows 40.2 -> 27.9 us a call, 55 -> 47 us a cycle of the plain
+// evolution, 14.4 -> 13.2 ms for 20 cycles of 100 runs.
 void KnnBatch::enqueue_vote(bool reduce, bool timed) {
   const hipStream_t s = stream_.get();
-  d_labels_.upload(h_labels_.get(), static_cast<size_t>(pad_total_), s);
-  if (reduce) check(launch_vote_reset(d_counts_.get(), d_firsts_.get(), d_matches_.get(), runs_, classes_, s), "vote reset");
-  if (timed) timer_.start(s);
   VoteParams prm;
   prm.neighbors = d_nbr_.get();
   prm.scores = d_score_.get();
-  prm.labels = d_labels_.get();
   prm.block_run = d_block_run_.get();
   prm.run_offsets = d_run_off_.get();
   prm.pad_offsets = d_pad_off_.get();
@@ -780,19 +784,25 @@ void KnnBatch::enqueue_vote(bool reduce, bool timed) {
   prm.k = k_;
   prm.max_rows = max_rows_;
   prm.classes = classes_;
-  prm.predictions = d_pred_.get();
+  constexpr size_t kDirectLabelBytes = 128 * 1024;
+  if (vote_stages_labels(prm) && sizeof(int) * blocks_ * static_cast<size_t>(max_rows_) <= kDirectLabelBytes) {
+    prm.labels = h_labels_.get();
+  } else {
+    d_labels_.upload(h_labels_.get(), static_cast<size_t>(pad_total_), s);
+    prm.labels = d_labels_.get();
+  }
+  prm.predictions = h_pred_.get();
   if (reduce) {
     prm.counts = d_counts_.get();
     prm.firsts = d_firsts_.get();
     prm.matches = d_matches_.get();
   }
+  if (timed) timer_.start(s);
   check(launch_vote(prm, blocks_, s), "vote launch");
   if (timed) timer_.stop(s);
-  d_pred_.download(h_pred_.get(), static_cast<size_t>(pad_total_), s);
   if (reduce) {
-    d_counts_.download(h_counts_.get(), static_cast<size_t>(runs_) * classes_, s);
-    d_firsts_.download(h_firsts_.get(), static_cast<size_t>(runs_) * classes_, s);
-    d_matches_.download(h_matches_.get(), static_cast<size_t>(runs_), s);
+    check(launch_vote_publish(d_counts_.get(), d_firsts_.get(), d_matches_.get(), runs_, classes_, h_counts_.get(),
+                              h_firsts_.get(), h_matches_.get(), s), "vote publish");
   }
 }
 
@@ -803,11 +813,12 @@ void KnnBatch::vote_all(bool reduce) {
     stream_.sync();
     return;
   }
-  enqueue_vote(reduce, true);
+  enqueue_vote(reduce, reduce);
   stream_.sync();
+  if (!reduce) return;
   vote_ms_ += timer_.ms();
   ++vote_calls_;
-  if (graph_on_ && reduce) {
+  if (graph_on_) {
     // Capture the same sequence (without the timer) for the later calls.
     check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     enqueue_vote(true, false);

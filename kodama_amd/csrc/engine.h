@@ -167,9 +167,10 @@ class KnnBatch {
   const int* firsts_host() const { return h_firsts_.get(); }
   const int* matches_host() const { return h_matches_.get(); }
 
-  // Upload labels_host(), vote all runs, download the results; blocks.
+  // Votes all runs on labels_host(), with the results in the pinned buffers;
+  // blocks.
   void vote_all(bool reduce = true);
-  // From the next vote_all(true) on, the upload, the vote and the downloads
+  // From the next vote_all(true) on, the upload (if any) and the two kernels
   // run as one captured graph (hipGraph), replayed once per call; the first
   // such call runs eagerly (timed) and captures. The staging buffers keep
   // their addresses, so every replay reads the labels of its call.

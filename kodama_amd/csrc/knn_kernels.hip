@@ -33,6 +33,7 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kWave = 64;
+using i32x4 = __attribute__((ext_vector_type(4))) int;
 
 // Candidate rows per LDS tile: 16 KiB of candidates for up to 64 dimensions,
 // 32 KiB beyond.
@@ -369,9 +370,23 @@ __global__ void __launch_bounds__(kBlock) vote_kernel(VoteParams prm) {
   if (STAGE) {
     // The run's labels, remapped. The remap is idempotent (targets map to
     // themselves), so a label another block already rewrote stages the same.
-    for (int i = threadIdx.x; i < L; i += kBlock) {
-      const int c = prm.labels[pad_base + i];
-      lab_s[i] = remapping && remap[c] >= 0 ? remap[c] : c;
+    // 16 bytes and four loads in flight a thread: they may come over the host
+    // link, a round trip of microseconds each (a run starts at a multiple of
+    // 256 labels and is padded to one).
+    const i32x4* src = reinterpret_cast<const i32x4*>(prm.labels + pad_base);
+    const int quads = (L + 3) / 4;
+    for (int i0 = threadIdx.x; i0 < quads; i0 += 4 * kBlock) {
+      i32x4 v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] = src[min(i0 + u * kBlock, quads - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int i = 4 * (i0 + u * kBlock) + e, c = v[u][e];
+          if (i < L) lab_s[i] = remapping && remap[c] >= 0 ? remap[c] : c;
+        }
+      }
     }
     __syncthreads();
   }
@@ -449,6 +464,23 @@ __global__ void vote_reset_kernel(int* counts, int* firsts, int* matches, int ru
     firsts[i] = INT_MAX;
   }
   if (i < runs) matches[i] = 0;
+}
+
+// A vote's reductions to (pinned host) memory, and cleared for the next vote.
+__global__ void vote_publish_kernel(int* counts, int* firsts, int* matches, int runs, int classes, int* out_counts,
+                                    int* out_firsts, int* out_matches) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int total = runs * classes;
+  if (i < total) {
+    out_counts[i] = counts[i];
+    out_firsts[i] = firsts[i];
+    counts[i] = 0;
+    firsts[i] = INT_MAX;
+  }
+  if (i < runs) {
+    out_matches[i] = matches[i];
+    matches[i] = 0;
+  }
 }
 
 // Merge of per-slice top-k lists, one wave per query: lane s holds the head of
@@ -594,18 +626,36 @@ hipError_t launch_knn_merge_slices(const int* idx, const float* dist, int slices
   return hipGetLastError();
 }
 
+static size_t vote_base_lds(const VoteParams& prm) {
+  return sizeof(int) * (3 * static_cast<size_t>(prm.classes) + 2 * kBlock + 2);
+}
+
+// The run's labels go to LDS when they fit (48 KiB of labels at most).
+bool vote_stages_labels(const VoteParams& prm) {
+  const size_t staged = vote_base_lds(prm) + sizeof(int) * static_cast<size_t>(prm.max_rows);
+  return prm.max_rows > 0 && staged <= 64 * 1024 && prm.max_rows <= 12288;
+}
+
 hipError_t launch_vote(const VoteParams& prm, int blocks, hipStream_t stream) {
   if (prm.k < 1 || prm.k > kMaxK) return hipErrorInvalidValue;
   if (blocks == 0) return hipSuccess;
-  const size_t base = sizeof(int) * (3 * static_cast<size_t>(prm.classes) + 2 * kBlock + 2);
+  const size_t base = vote_base_lds(prm);
   if (base > 64 * 1024) return hipErrorInvalidValue;
-  // Stage the run's labels in LDS when they fit (48 KiB of labels at most).
-  const size_t staged = base + sizeof(int) * static_cast<size_t>(prm.max_rows);
-  if (prm.max_rows > 0 && staged <= 64 * 1024 && prm.max_rows <= 12288) {
-    launch_vote_k<true>(prm, dim3(blocks), staged, stream);
+  if (vote_stages_labels(prm)) {
+    launch_vote_k<true>(prm, dim3(blocks), base + sizeof(int) * static_cast<size_t>(prm.max_rows), stream);
   } else {
     launch_vote_k<false>(prm, dim3(blocks), base, stream);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_vote_publish(int* counts, int* firsts, int* matches, int runs, int classes, int* out_counts,
+                               int* out_firsts, int* out_matches, hipStream_t stream) {
+  const int total = runs * classes > runs ? runs * classes : runs;
+  const int blocks = (total + kBlock - 1) / kBlock;
+  if (blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(vote_publish_kernel, dim3(blocks), dim3(kBlock), 0, stream, counts, firsts, matches, runs, classes,
+                     out_counts, out_firsts, out_matches);
   return hipGetLastError();
 }
 

@@ -83,6 +83,9 @@ hipError_t launch_knn_topk(const KnnTopkParams& prm, int mode, bool euclid, int 
 hipError_t launch_knn_merge_slices(const int* idx, const float* dist, int slices, int query_rows, int k,
                                    int* out_index, float* out_dist, hipStream_t stream);
 hipError_t launch_vote(const VoteParams& prm, int blocks, hipStream_t stream);
+bool vote_stages_labels(const VoteParams& prm);
+hipError_t launch_vote_publish(int* counts, int* firsts, int* matches, int runs, int classes, int* out_counts,
+                               int* out_firsts, int* out_matches, hipStream_t stream);
 hipError_t launch_vote_reset(int* counts, int* firsts, int* matches, int runs, int classes,
                              hipStream_t stream);
 
