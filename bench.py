@@ -212,7 +212,7 @@ def copy_probe() -> int:
 
 def graph_bench(rows: int, k: int, lists_ab: bool = False) -> int:
     """Exact self-kNN graph of the 20-cluster mixture (config-4 generator,
-    p = 50) through the split-BF16 MFMA path; one JSON line. With lists_ab,
+    p = 50) through the matrix-core path; one JSON line. With lists_ab,
     the graph is built with packed candidate lists, separate ones and packed
     again (one line each, and whether the graphs are identical)."""
     import kodama_amd as K
@@ -277,12 +277,12 @@ def matrix_bench(rows: int, runs: int, cycles: int, k: int, forms) -> int:
 
 
 def tables_bench(runs: int, n: int, k: int) -> int:
-    """Per-fold kNN tables of the batched-runs workload built by every schedule
-    the tuner chooses from (register scan; split-BF16 MFMA + exact rerank with
-    8 or 16 candidates per lane column and 4 or 8 waves per workgroup, the
-    lists as packed keys or as separate values and indices), twice each, then
-    the tuned build; one JSON line per build with its wall time, the rows the
-    MFMA path rescanned, and whether the tables equal the scan's."""
+    """Per-fold kNN tables of the batched-runs workload built under every
+    schedule setting (register scan; matrix-core candidates + exact rerank with
+    buffers of 128 or 256 rows per query, the wave and list-form settings as
+    they are kept), twice each, then the build the rule chooses; one JSON line
+    per build with its wall time, the rows the matrix-core path flagged, and
+    whether the tables equal the scan's."""
     import kodama_amd as K
     x, rows, fids, _ = make_workload(runs, n, 50, k)
     ref = None

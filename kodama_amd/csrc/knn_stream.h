@@ -1,4 +1,4 @@
-// Exact kNN through FP16 matrix-core candidates with a running threshold
+// Exact kNN through FP16 matrix-core candidates with a threshold from class maxima
 // (knn_stream.hip): parameter blocks and launchers.
 #pragma once
 

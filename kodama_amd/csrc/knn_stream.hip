@@ -1,4 +1,4 @@
-// Exact kNN through FP16 matrix-core candidates with a running threshold, and
+// Exact kNN through FP16 matrix-core candidates with a threshold from class maxima, and
 // an exact FP32 rerank.
 //
 // Score of a (query, train row) pair: s = q.t - |t|^2 / 2 (Euclidean) or q.t
