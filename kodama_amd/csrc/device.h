@@ -28,14 +28,17 @@ inline void check(hipError_t e, const char* what) {
 // some thousand blocks. A block freed under a stream may still be read or
 // written by work queued there, so it goes only to allocations under the same
 // stream until that stream has been settled (its work done); then to any.
-// At most kPoolBytes per device stay in the pool, the rest is freed, and a
-// failed allocation empties it first.
+// At most kPoolBytes per device stay in the pool: a block that comes back to a
+// full pool takes the place of the settled blocks unused the longest, so what
+// stays follows the sizes that calls ask for now; where those do not make room
+// it is freed. A failed allocation empties the pool first.
 constexpr size_t kPoolBytes = size_t(2) << 30;
 struct PoolBlock {
   void* p = nullptr;
   size_t bytes = 0;         // of the block
   int device = -1;
   hipStream_t tag = nullptr;  // null: not from the pool
+  uint64_t given = 0;         // order of return, of kept blocks
 };
 PoolBlock pool_take(size_t bytes, int device, hipStream_t tag);
 void pool_give(const PoolBlock& block);

@@ -17,6 +17,7 @@ struct Pool {
   struct PerDevice {
     std::multimap<size_t, PoolBlock> blocks;  // by size; tag null once settled
     size_t bytes = 0;
+    uint64_t returns = 0;
   };
   std::map<int, PerDevice> devices;
 };
@@ -82,16 +83,36 @@ PoolBlock pool_take(size_t bytes, int device, hipStream_t tag) {
 
 void pool_give(const PoolBlock& block) {
   Pool& pl = pool();
+  std::vector<void*> out;  // freed without the lock: hipFree waits for the device
   {
     std::lock_guard<std::mutex> lock(pl.mutex);
     Pool::PerDevice& d = pl.devices[block.device];
-    if (d.bytes + block.bytes <= kPoolBytes) {
-      d.blocks.emplace(block.bytes, block);
-      d.bytes += block.bytes;
-      return;
+    bool keep = true;
+    if (d.bytes + block.bytes > kPoolBytes) {
+      size_t settled = 0;
+      for (const auto& kv : d.blocks) settled += kv.second.tag == nullptr ? kv.first : 0;
+      keep = d.bytes - settled + block.bytes <= kPoolBytes;
+    }
+    while (keep && d.bytes + block.bytes > kPoolBytes) {
+      auto oldest = d.blocks.end();
+      for (auto it = d.blocks.begin(); it != d.blocks.end(); ++it) {
+        if (it->second.tag != nullptr) continue;
+        if (oldest == d.blocks.end() || it->second.given < oldest->second.given) oldest = it;
+      }
+      out.push_back(oldest->second.p);
+      d.bytes -= oldest->first;
+      d.blocks.erase(oldest);
+    }
+    if (keep) {
+      PoolBlock kept = block;
+      kept.given = ++d.returns;
+      d.blocks.emplace(kept.bytes, kept);
+      d.bytes += kept.bytes;
+    } else {
+      out.push_back(block.p);
     }
   }
-  (void)hipFree(block.p);
+  for (void* p : out) (void)hipFree(p);
 }
 
 void pool_settle(int device, hipStream_t tag) {
