@@ -40,13 +40,16 @@ struct PoolBlock {
   hipStream_t tag = nullptr;  // null: not from the pool
   uint64_t given = 0;         // order of return, of kept blocks
 };
+// hipMalloc on the current device (`device`); on failure the pool of that
+// device is emptied and the request repeated. Throws DeviceError.
+void* device_alloc(size_t bytes, int device);
 PoolBlock pool_take(size_t bytes, int device, hipStream_t tag);
 void pool_give(const PoolBlock& block);
 void pool_settle(int device, hipStream_t tag);  // every block of this tag is idle
 void pool_drop(int device, hipStream_t tag);    // free them instead (their work is unknown)
 
 // The stream under which the calling thread's DeviceBuffers allocate; scopes
-// nest. Without one they use hipMalloc and hipFree.
+// nest. Without one they use device_alloc and hipFree.
 class Stream;
 class StreamScope {
  public:
@@ -88,7 +91,9 @@ class DeviceBuffer {
       if (StreamScope::current() != nullptr) {
         block_ = pool_take(n * sizeof(T), StreamScope::current_device(), StreamScope::current());
       } else {
-        check(hipMalloc(&block_.p, n * sizeof(T)), "hipMalloc");
+        int device = 0;
+        check(hipGetDevice(&device), "hipGetDevice");
+        block_.p = device_alloc(n * sizeof(T), device);
       }
     }
     n_ = n;

@@ -43,6 +43,27 @@ StreamScope::~StreamScope() {
 hipStream_t StreamScope::current() { return g_scope; }
 int StreamScope::current_device() { return g_scope_device; }
 
+void* device_alloc(size_t bytes, int device) {
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  // Out of memory: give back what is kept and try once more.
+  Pool& pl = pool();
+  std::vector<void*> kept;
+  {
+    std::lock_guard<std::mutex> lock(pl.mutex);
+    Pool::PerDevice& d = pl.devices[device];
+    for (auto& kv : d.blocks) kept.push_back(kv.second.p);
+    d.blocks.clear();
+    d.bytes = 0;
+  }
+  for (void* k : kept) (void)hipFree(k);  // hipFree waits for their work
+  const hipError_t e = hipMalloc(&p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();  // not to be found by the next launch
+  check(e, "hipMalloc");
+  return p;
+}
+
 PoolBlock pool_take(size_t bytes, int device, hipStream_t tag) {
   const size_t need = (bytes + kGrain - 1) / kGrain * kGrain;
   Pool& pl = pool();
@@ -65,19 +86,7 @@ PoolBlock pool_take(size_t bytes, int device, hipStream_t tag) {
   b.bytes = need;
   b.device = device;
   b.tag = tag;
-  if (hipMalloc(&b.p, need) == hipSuccess) return b;
-  (void)hipGetLastError();
-  // Out of memory: give back what is kept and try once more.
-  std::vector<PoolBlock> kept;
-  {
-    std::lock_guard<std::mutex> lock(pl.mutex);
-    Pool::PerDevice& d = pl.devices[device];
-    for (auto& kv : d.blocks) kept.push_back(kv.second);
-    d.blocks.clear();
-    d.bytes = 0;
-  }
-  for (const PoolBlock& k : kept) (void)hipFree(k.p);  // hipFree waits for their work
-  check(hipMalloc(&b.p, need), "hipMalloc");
+  b.p = device_alloc(need, device);
   return b;
 }
 

@@ -128,3 +128,21 @@ def test_a_block_larger_than_the_pool_evicts_nothing(run):
     pool_give(huge);
     EXPECT(g_live.count(keep.p) == 1 && g_live.count(huge.p) == 0);
     """)
+
+
+def test_an_allocation_outside_a_call_gets_the_kept_memory(run):
+    """A buffer without a stream scope (the arrays of a resident graph) on a
+    device whose free memory is what the pool keeps."""
+    run(r"""
+    g_room = 1024 * MiB;
+    PoolBlock b = pool_take(800 * MiB, 0, tag(0));
+    pool_give(b);
+    pool_settle(0, tag(0));
+    DeviceBuffer<float> plain(600 * MiB / sizeof(float));
+    EXPECT(plain.get() != nullptr && g_live.size() == 1 && g_used == 600 * MiB);
+    plain.release();
+    EXPECT(g_used == 0);
+    bool threw = false;
+    try { DeviceBuffer<float> much(1025 * MiB / sizeof(float)); } catch (const DeviceError&) { threw = true; }
+    EXPECT(threw);
+    """)
