@@ -101,6 +101,11 @@ typedef struct kodama_hip_core_result {
 const char* kodama_hip_last_error(void);
 /* Number of visible gfx950 devices (hipGetDeviceCount + arch check). */
 int kodama_hip_device_count(int32_t* count);
+/* Device memory is kept between calls, at most 2 GiB per device, and given back
+ * when an allocation of the library fails. This gives all of it back at once,
+ * for other users of the device in the process; memory of calls in progress and
+ * of resident handles is not touched. */
+int kodama_hip_release_memory(int32_t device);
 /* Library version string, e.g. "kodama_hip 0.1.0 gfx950". */
 const char* kodama_hip_version(void);
 

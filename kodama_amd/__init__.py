@@ -20,7 +20,7 @@ from ._native import (CoreOptions, InvalidArgument, KodamaHipError, NoDevice,  #
 __all__ = [
     "KNNCV", "PLSLDACV", "CoreKNN", "CorePLSLDA", "CoreKNNGraph", "KODAMA_knn_graph",
     "KODAMA_dissimilarity", "core_knn", "core_plslda", "core_knn_batch", "exact_knn_search",
-    "KnnVoteGraph", "core_options", "device_count", "version",
+    "KnnVoteGraph", "core_options", "device_count", "version", "release_memory",
     "set_evolution_split", "last_evolution_workgroups", "set_cooperative_launch", "set_lds_flow_table",
     "last_evolution_lds_flows",
 ]
@@ -28,6 +28,12 @@ __all__ = [
 
 def version() -> str:
     return N.lib().kodama_hip_version().decode()
+
+
+def release_memory(gpu_device=0):
+    """Gives the device memory kept between calls (up to 2 GiB) back to other
+    users of the device; calls in progress and resident handles keep theirs."""
+    N.call("kodama_hip_release_memory", C.c_int32(int(gpu_device)))
 
 
 def _metric(metric) -> int:

@@ -93,6 +93,13 @@ const char* kodama_hip_version(void) { return "kodama_hip 0.1.0 gfx950"; }
 
 int kodama_hip_last_knn_fallbacks(void) { return kodama_hip::g_knn_fallbacks; }
 
+int kodama_hip_release_memory(int32_t device) {
+  return kodama_hip::guarded([&] {
+    kodama_hip::select_device(device);
+    kodama_hip::pool_empty(device);
+  });
+}
+
 int kodama_hip_device_count(int32_t* count) {
   return kodama_hip::guarded([&] {
     int n = 0;

@@ -45,6 +45,7 @@ struct PoolBlock {
 void* device_alloc(size_t bytes, int device);
 PoolBlock pool_take(size_t bytes, int device, hipStream_t tag);
 void pool_give(const PoolBlock& block);
+void pool_empty(int device);  // frees everything kept (hipFree waits for its work)
 void pool_settle(int device, hipStream_t tag);  // every block of this tag is idle
 void pool_drop(int device, hipStream_t tag);    // free them instead (their work is unknown)
 

@@ -43,11 +43,7 @@ StreamScope::~StreamScope() {
 hipStream_t StreamScope::current() { return g_scope; }
 int StreamScope::current_device() { return g_scope_device; }
 
-void* device_alloc(size_t bytes, int device) {
-  void* p = nullptr;
-  if (hipMalloc(&p, bytes) == hipSuccess) return p;
-  (void)hipGetLastError();
-  // Out of memory: give back what is kept and try once more.
+void pool_empty(int device) {
   Pool& pl = pool();
   std::vector<void*> kept;
   {
@@ -57,7 +53,14 @@ void* device_alloc(size_t bytes, int device) {
     d.blocks.clear();
     d.bytes = 0;
   }
-  for (void* k : kept) (void)hipFree(k);  // hipFree waits for their work
+  for (void* p : kept) (void)hipFree(p);
+}
+
+void* device_alloc(size_t bytes, int device) {
+  void* p = nullptr;
+  if (hipMalloc(&p, bytes) == hipSuccess) return p;
+  (void)hipGetLastError();
+  pool_empty(device);
   const hipError_t e = hipMalloc(&p, bytes);
   if (e != hipSuccess) (void)hipGetLastError();  // not to be found by the next launch
   check(e, "hipMalloc");

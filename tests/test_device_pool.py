@@ -146,3 +146,18 @@ def test_an_allocation_outside_a_call_gets_the_kept_memory(run):
     try { DeviceBuffer<float> much(1025 * MiB / sizeof(float)); } catch (const DeviceError&) { threw = true; }
     EXPECT(threw);
     """)
+
+
+def test_everything_kept_can_be_given_back(run):
+    """Settled blocks and those of unfinished work (hipFree waits for it), on
+    one device only; blocks in use stay."""
+    run(r"""
+    PoolBlock a = pool_take(10 * MiB, 0, tag(0)), b = pool_take(20 * MiB, 0, tag(1)), c = pool_take(30 * MiB, 0, tag(1));
+    PoolBlock other = pool_take(40 * MiB, 1, tag(2));
+    pool_give(a); pool_give(b); pool_give(other);
+    pool_settle(0, tag(0));
+    pool_empty(0);
+    EXPECT(g_live.size() == 2 && g_live.count(c.p) && g_live.count(other.p));
+    pool_give(c);
+    EXPECT(pool_take(30 * MiB, 0, tag(1)).p == c.p);
+    """)

@@ -1,5 +1,6 @@
 """Host side of the calls: memory and streams kept between calls (several
 threads, sizes that shrink and grow), and label encoding by table or by sort."""
+import ctypes
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -61,3 +62,36 @@ def test_label_values_do_not_matter(spread):
     out = K.KNNCV(x, lab, k=7, metric="euclidean", folds=5)
     assert np.array_equal(out["predicted_labels"], (base["predicted_labels"] - 9) * spread)
     assert np.array_equal(out["fold_assignments"], base["fold_assignments"])
+
+
+def _free_bytes():
+    """Free device memory, from the HIP runtime that the library is linked to."""
+    K.version()
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL("libamdhip64.so.7").hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_released_memory_is_free_for_others():
+    """What a call leaves in the pool comes back with release_memory; a resident
+    handle keeps its own, and later calls allocate again."""
+    rng = np.random.default_rng(5)
+    nbr = rng.integers(0, 3000, (3000, 12), dtype=np.int32)
+    score = -np.sort(rng.random((3000, 12), dtype=np.float32), axis=1)
+    codes = rng.integers(0, 9, 3000, dtype=np.int32)
+    x, _ = D.config3(n=60000, p=50, seed=3)
+    graph = K.KnnVoteGraph(nbr, score)
+    votes = graph.predict(codes)
+    K.release_memory()
+    before = _free_bytes()
+    want = K.KODAMA_knn_graph(x, k=20)
+    kept = before - _free_bytes()
+    K.release_memory()
+    assert kept > 30 << 20
+    assert before - _free_bytes() <= kept // 8
+    assert np.array_equal(graph.predict(codes), votes)
+    graph.close()
+    again = K.KODAMA_knn_graph(x, k=20)
+    assert np.array_equal(again["indices"], want["indices"])
+    with pytest.raises(K.NoDevice):
+        K.release_memory(gpu_device=99)
