@@ -67,7 +67,8 @@ typedef struct kodama_hip_core_options {
   int32_t scale;
   int32_t pls_fold_cache;         /* 1 = data_epoch != 0 (folds cached per run) */
   int32_t device;                 /* KNNOptions::gpu_device / PLSOptions::gpu_device */
-  int32_t n_threads;              /* host threads for the batched engine (0 = auto) */
+  int32_t n_threads;              /* host threads for the batched engine (0 = the processors
+                                     the process may run on) */
 } kodama_hip_core_options;
 
 /* Outputs of one label-evolution run (kodama::CoreResult, kodama.hpp:316-349).
@@ -417,7 +418,7 @@ typedef struct kodama_hip_matrix_options {
   int32_t form;             /* 0 = plain (reference streams per run), 1 = device-resident,
                                2 = device-resident with the learned proposal (kNN only) */
   int32_t device;
-  int32_t n_threads;        /* host threads of the plain form (0 = automatic) */
+  int32_t n_threads;        /* host threads of the plain form (0 as above) */
   const float* mlp_params;  /* form 2: the network, fp32 [10400] (kodama_hip_mlp_train) */
   float mlp_fallback;       /* form 2: share of cycles on the uniform proposal */
   int32_t classifier;       /* KODAMAMatrixOptions::classifier: 1 = KNN, 0 = PLS_LDA

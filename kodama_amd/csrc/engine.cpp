@@ -7,6 +7,7 @@
 #include <limits>
 #include <map>
 #include <numeric>
+#include <thread>
 #include <unordered_map>
 
 #include <omp.h>
@@ -845,9 +846,9 @@ void KnnBatch::download_tables(int r, int* nbr, float* score) {
 }
 
 int resolve_threads(int requested, int runs) {
-  // Automatic: what OpenMP would use, which follows the process's share of the
-  // host (affinity, OMP_NUM_THREADS).
-  int t = requested > 0 ? requested : omp_get_max_threads();
+  // Automatic: the processors this process may run on. Not OpenMP's count:
+  // launchers of one process per GPU set OMP_NUM_THREADS to 1.
+  int t = requested > 0 ? requested : static_cast<int>(std::thread::hardware_concurrency());
   if (t < 1) t = 1;
   return std::max(1, std::min(t, runs));
 }

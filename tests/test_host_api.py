@@ -94,3 +94,22 @@ def test_mlp_init_is_he_normal_and_deterministic():
     assert np.all(a[MO.B1:MO.W2] == 0) and np.all(a[MO.B2:MO.W3] == 0) and np.all(a[MO.B3:] == 0)
     w1 = a[MO.W1:MO.B1]
     assert abs(w1.std() - math.sqrt(2 / 64)) < 0.01 and abs(w1.mean()) < 0.01
+
+
+def test_automatic_threads_do_not_follow_openmp_settings():
+    """n_threads = 0 takes the processors the process may run on, at most one
+    per run, whatever OMP_NUM_THREADS says: launchers of one process per GPU
+    set it to 1, which is no wish for a serial evolution."""
+    import os
+    import subprocess
+    import sys
+    if not N.lib_available():
+        pytest.skip("libkodama_hip.so is not built")
+    code = ("import ctypes, os\n"
+            f"f = ctypes.CDLL({N.LIB_PATH!r})._ZN10kodama_hip15resolve_threadsEii\n"
+            "n = len(os.sched_getaffinity(0))\n"
+            "print(f(0, 1000) == n, f(0, 1) == 1, f(3, 1000) == 3, f(5, 2) == 2)")
+    for value in ("1", "2"):
+        out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, OMP_NUM_THREADS=value), check=True,
+                             capture_output=True, text=True, timeout=60).stdout
+        assert out.split() == ["True"] * 4, (value, out)
