@@ -19,6 +19,7 @@
 #include "host_pages.h"
 #include "knn_search.h"
 #include "launch.h"
+#include "loop_errors.h"
 #include "mlp.h"
 
 using namespace kodama_hip;
@@ -85,10 +86,9 @@ void run_knn_batch(const BatchRequest& q, int mode, const float* mlp_params, flo
     codes(static_cast<size_t>(runs)), cons(static_cast<size_t>(runs)), fixed(static_cast<size_t>(runs));
   IVec fold_concat(static_cast<size_t>(total));
   int classes = 1;
-  bool one_fold = false, bad_folds = !q.fold_ids && options->folds < 2;
-#pragma omp parallel for schedule(dynamic, 4) reduction(max : classes) reduction(|| : one_fold) if (total > (1 << 14) && !bad_folds)
-  for (int r = 0; r < runs; ++r) {
-    if (bad_folds) continue;  // refused below
+  bool one_fold = false;
+  LoopErrors errors;
+  auto prepare_run = [&](int r, int& most, bool& single) {
     const int L = offsets[r + 1] - offsets[r];
     const int* lab = q.initial_labels + offsets[r];
     if (q.constrain) cons[r].assign(q.constrain + offsets[r], q.constrain + offsets[r + 1]);
@@ -99,12 +99,14 @@ void run_knn_batch(const BatchRequest& q, int mode, const float* mlp_params, flo
     // Two folds or more: every row then has training rows, so the exact
     // search gives it at least one neighbour.
     const auto mm = std::minmax_element(folds[r].begin(), folds[r].end());
-    one_fold = one_fold || *mm.first == *mm.second;
+    single = single || *mm.first == *mm.second;
     encode_labels(lab, L, values[r], codes[r]);
-    classes = std::max(classes, static_cast<int>(values[r].size()));
+    most = std::max(most, static_cast<int>(values[r].size()));
     std::copy(folds[r].begin(), folds[r].end(), fold_concat.begin() + offsets[r]);
-  }
-  require(!bad_folds, "Number of folds must be at least 2.");
+  };
+#pragma omp parallel for schedule(dynamic, 4) reduction(max : classes) reduction(|| : one_fold) if (total > (1 << 14))
+  for (int r = 0; r < runs; ++r) errors.run([&] { prepare_run(r, classes, one_fold); });
+  errors.rethrow();
   require(!one_fold, "every run needs at least two distinct folds.");
   std::unique_ptr<KnnBatch> owned;
   if (tables) {

@@ -9,6 +9,7 @@
 #include "../../include/kodama_hip.h"
 #include "capi_common.h"
 #include "engine.h"
+#include "loop_errors.h"
 #include "pls_engine.h"
 #include "batch_api.h"
 
@@ -193,13 +194,16 @@ void run_plslda_batch(const BatchRequest& q, int32_t* clbest, double* accbest, d
   std::vector<IVec> values(static_cast<size_t>(runs)), codes(static_cast<size_t>(runs)),
     cons(static_cast<size_t>(runs)), fixed(static_cast<size_t>(runs));
   int classes = 1;
-#pragma omp parallel for schedule(dynamic, 4) reduction(max : classes) if (total > (1 << 14))
-  for (int r = 0; r < runs; ++r) {
+  LoopErrors errors;
+  auto prepare_run = [&](int r, int& most) {
     encode_labels(q.initial_labels + offsets[r], offsets[r + 1] - offsets[r], values[r], codes[r]);
-    classes = std::max(classes, static_cast<int>(values[r].size()));
+    most = std::max(most, static_cast<int>(values[r].size()));
     if (q.constrain) cons[r].assign(q.constrain + offsets[r], q.constrain + offsets[r + 1]);
     if (q.fixed) fixed[r].assign(q.fixed + offsets[r], q.fixed + offsets[r + 1]);
-  }
+  };
+#pragma omp parallel for schedule(dynamic, 4) reduction(max : classes) if (total > (1 << 14))
+  for (int r = 0; r < runs; ++r) errors.run([&] { prepare_run(r, classes); });
+  errors.rethrow();
   const int F = options->folds;
   const bool cache = options->stratified == 0;
   auto run_folds = [&](int r, const IVec& labs) {

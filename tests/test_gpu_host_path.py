@@ -95,3 +95,13 @@ def test_released_memory_is_free_for_others():
     assert np.array_equal(again["indices"], want["indices"])
     with pytest.raises(K.NoDevice):
         K.release_memory(gpu_device=99)
+
+
+def test_an_error_in_a_parallel_loop_is_an_error_of_the_call():
+    """20 runs, enough rows for the parallel preparation, and a fold count that
+    the fold dealer refuses inside it."""
+    x, comp = D.config3(n=3000, p=8, seed=2)
+    rows = [np.arange(r, 1000 + r, dtype=np.int32) for r in range(20)]
+    o = K.core_options(cycles=1, k=5, folds=1, stratified=0, evolutionary_search=1, guarded_diversity=1)
+    with pytest.raises(ValueError, match="Number of folds must be at least 2"):
+        K.core_knn_batch(x, rows, [comp[r] for r in rows], o)
