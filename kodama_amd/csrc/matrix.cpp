@@ -118,13 +118,13 @@ struct DeviceLloyd {
   int runs, n, p, k, parts, steps, pad_n, pad_k;
   hipStream_t s;
   DeviceBuffer<float> xn, cent, cn, sizes, norm2_max;
-  DeviceBuffer<int> asg, changed, offsets, members;
+  DeviceBuffer<int> asg, changed, offsets, members;  // changed: per run, then the largest centroid norm
   DeviceBuffer<unsigned char> row_op, cent_op;
 
   DeviceLloyd(const float* x, int runs_, int n_, int p_, int k_, hipStream_t stream)
       : d_x(x), runs(runs_), n(n_), p(p_), k(k_), s(stream), xn(static_cast<size_t>(runs) * n),
         cent(static_cast<size_t>(runs) * k * p), cn(static_cast<size_t>(runs) * k), sizes(cn.size()), norm2_max(2),
-        asg(xn.size()), changed(static_cast<size_t>(runs)),
+        asg(xn.size()), changed(static_cast<size_t>(runs) + 1),
         offsets(static_cast<size_t>(runs) * k * kmeans_segments(n)), members(xn.size()) {
     // Three FP16 parts where they are as wide as one.
     parts = stream_steps(p, 3, true) == stream_steps(p, 1, true) ? 3 : 1;
@@ -133,10 +133,9 @@ struct DeviceLloyd {
     pad_k = (k + 63) / 64 * 64;
     row_op.resize(stream_operand_bytes(static_cast<size_t>(runs) * pad_n, steps));
     cent_op.resize(stream_operand_bytes(static_cast<size_t>(runs) * pad_k, steps));
-    check(launch_sse_norms(d_x, runs * n, p, xn.get(), s), "sse_norms launch");
     check(hipMemsetAsync(asg.get(), 0xFF, sizeof(int) * asg.size(), s), "memset");  // -1: unassigned
     check(hipMemsetAsync(norm2_max.get(), 0, 2 * sizeof(float), s), "memset");
-    check(launch_norms_max(xn.get(), xn.size(), norm2_max.get(), s), "norms_max launch");
+    check(launch_sse_norms(d_x, runs * n, p, xn.get(), norm2_max.get(), s), "sse_norms launch");
     StreamOperandJob op = operand_job(d_x, xn.get(), n, pad_n);
     op.query_op = row_op.get();
     check(launch_stream_operands(op, s), "stream_operands launch");
@@ -157,11 +156,12 @@ struct DeviceLloyd {
   }
   // Assignment to the centroids in `cent`; counts the changes.
   void assign(const int* active) {
-    check(launch_sse_norms(cent.get(), runs * k, p, cn.get(), s), "sse_norms launch");
+    check(hipMemsetAsync(changed.get(), 0, sizeof(int) * changed.size(), s), "memset");
+    float* const cn_max = reinterpret_cast<float*>(changed.get() + runs);
+    check(launch_sse_norms(cent.get(), runs * k, p, cn.get(), cn_max, s), "sse_norms launch");
     StreamOperandJob op = operand_job(cent.get(), cn.get(), k, pad_k);
     op.train_op = cent_op.get();
     check(launch_stream_operands(op, s), "stream_operands launch");
-    check(hipMemsetAsync(changed.get(), 0, sizeof(int) * changed.size(), s), "memset");
     KmeansAssignParams a;
     a.x = d_x;
     a.n = n;
@@ -176,6 +176,7 @@ struct DeviceLloyd {
     a.row_op = row_op.get();
     a.centroid_op = cent_op.get();
     a.norm2_max = norm2_max.get();
+    a.c_norm_max = cn_max;
     a.parts = parts;
     a.pad_n = pad_n;
     a.pad_k = pad_k;

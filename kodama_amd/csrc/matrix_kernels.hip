@@ -67,13 +67,8 @@ __device__ __forceinline__ float sse_dot_rows(const float* __restrict__ a, const
   return sum;
 }
 
-}  // namespace
-
-__global__ void __launch_bounds__(kBlock) sse_norms_kernel(const float* __restrict__ x, int rows, int p,
-                                                            float* __restrict__ out) {
-  const int r = blockIdx.x * kBlock + threadIdx.x;
-  if (r >= rows) return;
-  const float* a = x + static_cast<size_t>(r) * p;
+// Reference-order squared norm of a row.
+__device__ __forceinline__ float sse_norm(const float* __restrict__ a, int p) {
   float s[16];
 #pragma unroll
   for (int j = 0; j < 16; ++j) s[j] = 0.0f;
@@ -87,23 +82,28 @@ __global__ void __launch_bounds__(kBlock) sse_norms_kernel(const float* __restri
   for (int l = 0; l < 4; ++l) lane[l] = __fadd_rn(__fadd_rn(s[l], s[4 + l]), __fadd_rn(s[8 + l], s[12 + l]));
   float sum = __fadd_rn(__fadd_rn(__fadd_rn(lane[0], lane[1]), lane[2]), lane[3]);
   for (; i < p; ++i) sum = __fadd_rn(sum, __fmul_rn(a[i], a[i]));
-  out[r] = sum;
+  return sum;
 }
 
-// Largest of the norms (>= 0, so their bits order as integers; NaN excluded).
-__global__ void __launch_bounds__(kBlock) norms_max_kernel(const float* __restrict__ norms, size_t count,
-                                                            float* __restrict__ out) {
+}  // namespace
+
+// norm_max (may be null): raised to the block's largest norm (>= 0, so their
+// bits order as integers; NaN excluded).
+__global__ void __launch_bounds__(kBlock) sse_norms_kernel(const float* __restrict__ x, int rows, int p,
+                                                            float* __restrict__ out, float* __restrict__ norm_max) {
   __shared__ uint32_t s_max;
   if (threadIdx.x == 0) s_max = 0u;
   __syncthreads();
-  uint32_t best = 0u;
-  for (size_t i = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x; i < count;
-       i += static_cast<size_t>(gridDim.x) * kBlock) {
-    if (norms[i] >= 0.0f) best = max(best, __float_as_uint(norms[i]));
+  const int r = blockIdx.x * kBlock + threadIdx.x;
+  if (r < rows) {
+    const float sum = sse_norm(x + static_cast<size_t>(r) * p, p);
+    out[r] = sum;
+    if (sum > 0.0f) atomicMax(&s_max, __float_as_uint(sum));
   }
-  if (best != 0u) atomicMax(&s_max, best);
   __syncthreads();
-  if (threadIdx.x == 0 && s_max != 0u) atomicMax(reinterpret_cast<uint32_t*>(out), s_max);
+  if (threadIdx.x == 0 && norm_max != nullptr && s_max != 0u) {
+    atomicMax(reinterpret_cast<uint32_t*>(norm_max), s_max);
+  }
 }
 
 // Roundings of the reference's (|x|^2 + |c|^2) - 2 x.c in units of its norms: 16
@@ -245,9 +245,11 @@ __global__ void __launch_bounds__(kBlock, KS <= 8 ? 2 : 1) kmeans_assign_kernel(
   };
   stream(std::integral_constant<int, 0>{});
   const float scale = operand_scale(prm.norm2_max);
-  const bool usable = norms_usable(prm.norm2_max);
-  // Centroids are means of rows (and splits of 1 / 1024): within 1.003 of the largest row.
-  const float cmax = sqrtf(prm.norm2_max[0]) * scale * 1.003f;
+  // The largest centroid of this assignment: repeated splits of one donor and
+  // long float sums take centroids past the largest row. The scale is the
+  // rows', and FP16 holds the norm column up to 2^15.
+  const float cmax = sqrtf(*prm.c_norm_max) * scale * 1.0001f;
+  const bool usable = norms_usable(prm.norm2_max) && cmax < 30000.0f;
 #pragma unroll
   for (int t = 0; t < NQ; ++t) {
     float m = th[t];
@@ -476,16 +478,10 @@ __global__ void __launch_bounds__(kBlock) project_kernel(ProjectParams prm) {
 
 // ---- launchers --------------------------------------------------------------
 
-hipError_t launch_sse_norms(const float* x, int rows, int p, float* out, hipStream_t s) {
+hipError_t launch_sse_norms(const float* x, int rows, int p, float* out, float* norm_max, hipStream_t s) {
   if (rows == 0) return hipSuccess;
-  hipLaunchKernelGGL(sse_norms_kernel, dim3((rows + kBlock - 1) / kBlock), dim3(kBlock), 0, s, x, rows, p, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_norms_max(const float* norms, size_t count, float* out, hipStream_t s) {
-  if (count == 0) return hipSuccess;
-  const unsigned blocks = static_cast<unsigned>(std::min<size_t>((count + kBlock - 1) / kBlock, 1024));
-  hipLaunchKernelGGL(norms_max_kernel, dim3(blocks), dim3(kBlock), 0, s, norms, count, out);
+  hipLaunchKernelGGL(sse_norms_kernel, dim3((rows + kBlock - 1) / kBlock), dim3(kBlock), 0, s, x, rows, p, out,
+                     norm_max);
   return hipGetLastError();
 }
 
@@ -499,7 +495,7 @@ static void launch_assign_steps(const KmeansAssignParams& prm, int runs, hipStre
 hipError_t launch_kmeans_assign(const KmeansAssignParams& prm, hipStream_t s, int runs) {
   const int steps = stream_steps(prm.p, prm.parts, true);
   if (prm.p < 1 || prm.p > 256 || prm.k < 1 || prm.k > (1 << 25) || runs < 1 || runs > 65535 || steps < 1 || steps > 9 ||
-      prm.pad_n % 16 != 0 || prm.pad_n < prm.n || prm.pad_k % 64 != 0 || prm.pad_k < prm.k) {
+      prm.pad_n % 16 != 0 || prm.pad_n < prm.n || prm.pad_k % 64 != 0 || prm.pad_k < prm.k || prm.c_norm_max == nullptr) {
     return hipErrorInvalidValue;
   }
   if (prm.n == 0) return hipSuccess;

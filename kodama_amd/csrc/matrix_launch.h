@@ -9,11 +9,9 @@
 
 namespace kodama_hip {
 
-// out[r] = dot(x_r, x_r) in the reference's float order (see matrix_kernels.hip).
-hipError_t launch_sse_norms(const float* x, int rows, int p, float* out, hipStream_t s);
-
-// *out = max(*out, the largest of the norms); the caller cleared *out.
-hipError_t launch_norms_max(const float* norms, size_t count, float* out, hipStream_t s);
+// out[r] = dot(x_r, x_r) in the reference's float order (see matrix_kernels.hip);
+// *norm_max (may be null; the caller cleared it) = their largest.
+hipError_t launch_sse_norms(const float* x, int rows, int p, float* out, float* norm_max, hipStream_t s);
 
 // Nearest centroid of every row (smallest (|x|^2 + |c|^2) - 2 x.c, first
 // cluster on ties); rows whose assignment changes are counted in *changed.
@@ -36,6 +34,7 @@ struct KmeansAssignParams {
   const void* row_op = nullptr;
   const void* centroid_op = nullptr;
   const float* norm2_max = nullptr;  // [2]: the largest row norm, 0
+  const float* c_norm_max = nullptr; // largest of c_norm over all problems
   int parts = 1, pad_n = 0, pad_k = 0;
 };
 hipError_t launch_kmeans_assign(const KmeansAssignParams& prm, hipStream_t s, int runs = 1);

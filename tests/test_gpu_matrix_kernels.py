@@ -51,6 +51,18 @@ def test_rows_without_spread(oracle):
     _check(oracle, x, landmarks=150, splitting=70)
 
 
+@pytest.mark.parametrize("value", [7.0, 1e-3])
+def test_many_splits_of_one_donor(oracle, value):
+    """Nearly all rows equal and far more clusters than distinct rows: each
+    round splits the same donors over and over, which scales centroids by
+    (1 + 1 / 1024) each time, past every row's norm; the bound of the scores
+    follows them. One column, so that every product is rounded alone."""
+    rng = np.random.default_rng(3)
+    x = np.full((3000, 1), value, np.float32)
+    x[::100] += rng.normal(0.0, value / 100, (30, 1)).astype(np.float32)
+    _check(oracle, x, landmarks=1500, splitting=200)
+
+
 @pytest.mark.parametrize("scale", [1e-18, 1e18])
 def test_scales_outside_the_scores(oracle, scale):
     """Norms the FP16 scores do not serve: every pair is evaluated exactly."""
