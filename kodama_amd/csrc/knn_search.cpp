@@ -23,36 +23,6 @@ constexpr int kSliceAlign = 64;          // LDS tile rows of the scan
 constexpr int kTableTargetBlocks = 2048; // sliced rescans of flagged table rows
 constexpr int kStreamMinTrain = 4096;     // smaller train sets use the register scan
 constexpr int kStreamWideQueries = 1024;  // queries beyond 64 dimensions for the matrix cores
-constexpr int kStreamTargetBlocks = 2048; // eight workgroups per CU
-constexpr int kStreamSliceRows = 256;     // train rows per slice at least
-constexpr size_t kStreamCandBytes = size_t(1) << 30;  // candidate buffers per launch
-
-// How one pass is cut: slices of the candidates and of the maxima that bring
-// about eight workgroups per CU, each with at least kStreamSliceRows train
-// rows, the candidate buffers within kStreamCandBytes where slices allow it.
-struct StreamPlan {
-  int slices, max_slices, list, k;
-  size_t query_bytes;  // buffer of one query: its candidates, before them its maxima
-  StreamPlan(int query_rows, int train_rows, int k_, int list_, int steps) : list(list_), k(k_) {
-    const int per_block = 4 * stream_queries_per_wave(steps);
-    const int blocks = (query_rows + per_block - 1) / per_block;
-    const int want = std::min((kStreamTargetBlocks + blocks - 1) / blocks,
-                              std::min(kStreamMaxSlices, std::max(1, train_rows / kStreamSliceRows)));
-    const size_t list_bytes = static_cast<size_t>(stream_capacity(list)) * sizeof(uint2);
-    const size_t fit = kStreamCandBytes / (list_bytes * blocks * per_block);
-    slices = std::max(1, std::min(want, static_cast<int>(std::min<size_t>(fit, kStreamMaxSlices))));
-    max_slices = std::min(kStreamMaxSlices, std::max(stream_min_max_slices(k), want));
-    query_bytes = std::max(list_bytes * slices, static_cast<size_t>(max_slices) * 32 * sizeof(float));
-  }
-  void apply(KnnStreamParams& m, unsigned char* buffer) const {
-    m.slices = slices;
-    m.list = list;
-    m.sample_chunks = stream_sample_chunks(k);
-    m.max_slices = max_slices;
-    m.maxima = reinterpret_cast<float*>(buffer);  // read before the candidates are written
-    m.cand = reinterpret_cast<uint2*>(buffer);
-  }
-};
 
 }  // namespace
 
@@ -147,10 +117,8 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
       check(launch_stream_operands(op, s), "stream_operands launch");
     }
     const StreamPlan plan(rows, train_rows, k, list, steps);
-    const size_t query_bytes = plan.query_bytes;
-    const size_t fit = kStreamCandBytes / query_bytes;
-    const int batch = std::min(q_pad, static_cast<int>(std::max<size_t>(1, fit / kStreamBlockRows) * kStreamBlockRows));
-    DeviceBuffer<unsigned char> cand(static_cast<size_t>(batch) * query_bytes);
+    const int batch = std::min(q_pad, plan.batch());
+    DeviceBuffer<unsigned char> cand(static_cast<size_t>(batch) * plan.query_bytes);
     DeviceBuffer<float> threshold(static_cast<size_t>(batch));
     DeviceBuffer<int> count(static_cast<size_t>(batch) * plan.slices), flags(static_cast<size_t>(rows));
     DeviceBuffer<float> bound(count.size());
@@ -307,9 +275,10 @@ int device_fold_tables(const FoldTableJob& job, hipStream_t s) {
     op.query_op = q_op.get();
     check(launch_stream_operands(op, s), "stream_operands launch");
     const StreamPlan plan(job.pad_total, job.max_rows, job.k, list, steps);
-    DeviceBuffer<unsigned char> cand(static_cast<size_t>(job.pad_total) * plan.query_bytes);
-    DeviceBuffer<int> count(static_cast<size_t>(job.pad_total) * plan.slices);
-    DeviceBuffer<float> bound(count.size()), threshold(static_cast<size_t>(job.pad_total));
+    const int batch = std::min(job.pad_total, plan.batch());
+    DeviceBuffer<unsigned char> cand(static_cast<size_t>(batch) * plan.query_bytes);
+    DeviceBuffer<int> count(static_cast<size_t>(batch) * plan.slices);
+    DeviceBuffer<float> bound(count.size()), threshold(static_cast<size_t>(batch));
     KnnStreamParams m;
     m.train = m.query = xc.get();
     m.train_stride = m.query_stride = stride;
@@ -317,7 +286,7 @@ int device_fold_tables(const FoldTableJob& job, hipStream_t s) {
     m.query_op = q_op.get();
     m.query_norm2 = n2.get();
     m.norm2_max = n2_max.get();
-    m.train_rows = m.query_rows = total;
+    m.train_rows = total;
     m.dims = job.p;
     m.k = job.k;
     m.parts = parts;
@@ -334,7 +303,10 @@ int device_fold_tables(const FoldTableJob& job, hipStream_t s) {
     m.flags = flags.get();
     m.out_index = job.d_nbr;
     m.out_dist = job.d_score;
-    check(launch_knn_stream(m, s), "knn_stream launch");
+    for (m.query_begin = 0; m.query_begin < job.pad_total; m.query_begin += batch) {
+      m.query_rows = std::min(batch, job.pad_total - m.query_begin);
+      check(launch_knn_stream(m, s), "knn_stream launch");
+    }
     flags.download(h_flags.data(), h_flags.size(), s);
     check(hipStreamSynchronize(s), "fold tables sync");
   };

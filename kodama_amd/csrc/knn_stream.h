@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cstddef>
 
 namespace kodama_hip {
@@ -52,19 +53,58 @@ struct KnnStreamParams {
   const int* pad_offsets = nullptr;
   const int* folds = nullptr;       // [rows], concatenated
   int pad_rows = 0;
+  // For tables query_rows padded rows from query_begin on (a multiple of 256),
+  // and the buffers below start at query_begin; otherwise 0.
+  int query_begin = 0;
   // Class maxima: sampled 64-row chunks (all rows when at least as many),
   // dealt to max_slices workgroups per query block; 32 values per query and slice.
   int sample_chunks = 1, max_slices = 1;
-  float* maxima = nullptr;          // [query rows (padded for tables)][max_slices][32]; may share cand
+  float* maxima = nullptr;          // [query rows][max_slices][32]; may share cand
   float* threshold = nullptr;       // [query rows]
   int slices = 1;                   // the candidates' train rows are cut into this many ranges
   int list = 8;                     // capacity / 16
-  uint2* cand = nullptr;            // [query rows (padded for tables)][slices][capacity] (score bits, row)
+  uint2* cand = nullptr;            // [query rows][slices][capacity] (score bits, row)
   int* cand_count = nullptr;        // [query rows][slices], -1 = overflowed
   float* cand_bound = nullptr;      // [query rows][slices] scores below it were dropped
-  int* flags = nullptr;             // [query rows] 1 = needs another path
+  int* flags = nullptr;             // [query rows] 1 = needs another path; tables: [rows], concatenated
   int* out_index = nullptr;         // [query rows x k]; tables: the vote layout [k x pad_rows]
   float* out_dist = nullptr;        // internal distances; tables: scores (minus the distance)
+};
+
+// How one pass is cut: slices of the candidates and of the maxima towards eight
+// workgroups per CU, at most kStreamMaxSlices of at least kStreamSliceRows
+// train rows each (so a few hundred queries leave most CUs idle), and launches
+// of batch() queries whose candidate buffers stay within kStreamCandBytes.
+constexpr int kStreamTargetBlocks = 2048;
+constexpr int kStreamSliceRows = 256;
+constexpr size_t kStreamCandBytes = size_t(1) << 30;
+struct StreamPlan {
+  int slices, max_slices, list, k;
+  size_t query_bytes;  // buffer of one query: its candidates, before them its maxima
+  StreamPlan(int query_rows, int train_rows, int k_, int list_, int steps) : list(list_), k(k_) {
+    const int per_block = 4 * stream_queries_per_wave(steps);
+    const int blocks = (query_rows + per_block - 1) / per_block;
+    const int want = std::min((kStreamTargetBlocks + blocks - 1) / blocks,
+                              std::min(kStreamMaxSlices, std::max(1, train_rows / kStreamSliceRows)));
+    const size_t list_bytes = static_cast<size_t>(stream_capacity(list)) * sizeof(uint2);
+    const size_t fit = kStreamCandBytes / (list_bytes * blocks * per_block);
+    slices = std::max(1, std::min(want, static_cast<int>(std::min<size_t>(fit, kStreamMaxSlices))));
+    max_slices = std::min(kStreamMaxSlices, std::max(stream_min_max_slices(k), want));
+    query_bytes = std::max(list_bytes * slices, static_cast<size_t>(max_slices) * 32 * sizeof(float));
+  }
+  // Query rows per launch, whole blocks of kStreamBlockRows.
+  int batch() const {
+    const size_t blocks = std::max<size_t>(1, kStreamCandBytes / query_bytes / kStreamBlockRows);
+    return static_cast<int>(std::min<size_t>(blocks, (1 << 30) / kStreamBlockRows)) * kStreamBlockRows;
+  }
+  void apply(KnnStreamParams& m, unsigned char* buffer) const {
+    m.slices = slices;
+    m.list = list;
+    m.sample_chunks = stream_sample_chunks(k);
+    m.max_slices = max_slices;
+    m.maxima = reinterpret_cast<float*>(buffer);  // read before the candidates are written
+    m.cand = reinterpret_cast<uint2*>(buffer);
+  }
 };
 
 // Squared norms [rows] (rows `stride` floats apart) and their maximum (into

@@ -294,7 +294,7 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 3 : 2) knn_maxima_kernel(KnnStr
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   const int half = lane / kTile, col = lane % kTile;
-  const int q_block = blockIdx.x * (4 * kWaveQueries);
+  const int q_block = prm.query_begin + static_cast<int>(blockIdx.x) * (4 * kWaveQueries);
   const StreamRange g = stream_range(prm, q_block);
   if (q_block >= g.q_end) return;
   const int q_wave = q_block + wave * kWaveQueries;
@@ -377,8 +377,8 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 3 : 2) knn_maxima_kernel(KnnStr
   for (int t = 0; t < NQ; ++t) {
     const int q = q_wave + t * kTile + col;
     if (q < g.q_end) {
-      float4* dst = reinterpret_cast<float4*>(prm.maxima + (static_cast<size_t>(q) * prm.max_slices + blockIdx.y) * 32 +
-                                              half * 16);
+      float4* dst = reinterpret_cast<float4*>(
+        prm.maxima + (static_cast<size_t>(q - prm.query_begin) * prm.max_slices + blockIdx.y) * 32 + half * 16);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         dst[i] = make_float4(top[t][4 * i], top[t][4 * i + 1], top[t][4 * i + 2], top[t][4 * i + 3]);
@@ -389,17 +389,19 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 3 : 2) knn_maxima_kernel(KnnStr
 
 // One wave per operand row; REGS x 64 class maxima (empty ones -inf).
 template <int REGS>
-__global__ void __launch_bounds__(256) knn_threshold_kernel(KnnStreamParams prm, int rows, int per_query) {
-  const int q = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x / kWave));
+__global__ void __launch_bounds__(256) knn_threshold_kernel(KnnStreamParams prm, int per_query) {
+  // Row of the buffers, and operand row.
+  const int local = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + static_cast<int>(threadIdx.x / kWave));
+  const int q = prm.query_begin + local;
   const int lane = threadIdx.x & (kWave - 1);
-  if (q >= rows) return;
+  if (local >= prm.query_rows) return;
   int delta = 0;
   if (prm.block_run != nullptr) {
     const StreamRange g = stream_range(prm, q);
     if (q >= g.q_end) return;
     delta = g.delta;
   }
-  const float* src = prm.maxima + static_cast<size_t>(q) * per_query;
+  const float* src = prm.maxima + static_cast<size_t>(local) * per_query;
   uint32_t key[REGS];
   int valid = 0;
 #pragma unroll
@@ -420,7 +422,7 @@ __global__ void __launch_bounds__(256) knn_threshold_kernel(KnnStreamParams prm,
     bound = drop_bound(key_value(kth_largest<REGS>(key, REGS, want)),
                        2.0f * pair_error(qn, tmax, prm.dims, prm.parts, width));
   }
-  if (lane == 0) prm.threshold[q] = bound;
+  if (lane == 0) prm.threshold[local] = bound;
 }
 
 // R: capacity / 64. blockIdx.x: query block, blockIdx.y: slice of the train rows.
@@ -438,7 +440,7 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(Kn
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   const int half = lane / kTile, col = lane % kTile;
-  const int q_block = blockIdx.x * (4 * kWaveQueries);
+  const int q_block = prm.query_begin + static_cast<int>(blockIdx.x) * (4 * kWaveQueries);
   StreamRange g = stream_range(prm, q_block);
   if (q_block >= g.q_end) return;
   // This slice's rows (a multiple of 64 except at the end; may be empty).
@@ -449,7 +451,7 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(Kn
     g.t_end = min(g.t_end, g.t_begin + per);
   }
   const int q_wave = q_block + wave * kWaveQueries;
-  const size_t slot0 = static_cast<size_t>(q_wave) * prm.slices + blockIdx.y;  // query i: + i * slices
+  const size_t slot0 = static_cast<size_t>(q_wave - prm.query_begin) * prm.slices + blockIdx.y;  // query i: + i * slices
   const bool usable = norms_usable(prm.norm2_max);
 
   f16x8 bq[NQ][2 * KS];
@@ -459,7 +461,7 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(Kn
   for (int t = 0; t < NQ; ++t) {
     const int q = q_wave + t * kTile + col;
     const bool live = q < g.q_end;
-    th[t] = live ? prm.threshold[q] : INFINITY;
+    th[t] = live ? prm.threshold[q - prm.query_begin] : INFINITY;
     if (half == 0) {
       int ex = -1;  // the query's own fold or row
       if (live) {
@@ -657,10 +659,11 @@ __global__ void __launch_bounds__(256, 4) knn_stream_rerank_kernel(KnnStreamPara
   __shared__ float s_dist[4][kStreamMerge];
   const int wave = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
-  const int op_row = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + wave);
+  const int local = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * 4 + wave);  // row of the buffers
+  const int op_row = prm.query_begin + local;
   const int k = prm.k, p = prm.dims, cap = 16 * prm.list;
   const bool tables = prm.block_run != nullptr;
-  if (op_row >= (tables ? prm.pad_rows : prm.query_rows)) return;  // whole waves; no block barrier below
+  if (local >= prm.query_rows) return;  // whole waves; no block barrier below
   const StreamRange g = stream_range(prm, op_row);
   if (op_row >= g.q_end) return;
   const int q = op_row + g.delta;
@@ -670,13 +673,13 @@ __global__ void __launch_bounds__(256, 4) knn_stream_rerank_kernel(KnnStreamPara
   bool bad = false;
   float bound = -INFINITY;
   for (int sl = 0; sl < prm.slices; ++sl) {
-    const size_t o = static_cast<size_t>(op_row) * prm.slices + sl;
+    const size_t o = static_cast<size_t>(local) * prm.slices + sl;
     bad = bad || prm.cand_count[o] < 0;
     bound = fmaxf(bound, prm.cand_bound[o]);
   }
   int n = 0;
   for (int sl = 0; sl < prm.slices && !bad; ++sl) {
-    const size_t o = static_cast<size_t>(op_row) * prm.slices + sl;
+    const size_t o = static_cast<size_t>(local) * prm.slices + sl;
     const int c = prm.cand_count[o];
     for (int e0 = 0; e0 < c; e0 += kWave) {
       const int e = e0 + lane;
@@ -789,7 +792,7 @@ hipError_t launch_stream_operands(const StreamOperandJob& job, hipStream_t s) {
 
 template <int KS>
 static void launch_steps(const KnnStreamParams& prm, hipStream_t s) {
-  const int rows = prm.block_run != nullptr ? prm.pad_rows : prm.query_rows;
+  const int rows = prm.query_rows;
   constexpr int NQ = KS <= 4 ? 2 : 1;
   const int qpb = 4 * NQ * kTile;
   const unsigned qblocks = static_cast<unsigned>((rows + qpb - 1) / qpb);
@@ -798,10 +801,10 @@ static void launch_steps(const KnnStreamParams& prm, hipStream_t s) {
   else hipLaunchKernelGGL((knn_maxima_kernel<KS, NQ, false>), mgrid, dim3(256), 0, s, prm);
   const int per_query = prm.max_slices * 32;
   const dim3 tgrid(static_cast<unsigned>((rows + 3) / 4));
-  if (per_query <= 64) hipLaunchKernelGGL((knn_threshold_kernel<1>), tgrid, dim3(256), 0, s, prm, rows, per_query);
-  else if (per_query <= 128) hipLaunchKernelGGL((knn_threshold_kernel<2>), tgrid, dim3(256), 0, s, prm, rows, per_query);
-  else if (per_query <= 256) hipLaunchKernelGGL((knn_threshold_kernel<4>), tgrid, dim3(256), 0, s, prm, rows, per_query);
-  else hipLaunchKernelGGL((knn_threshold_kernel<8>), tgrid, dim3(256), 0, s, prm, rows, per_query);
+  if (per_query <= 64) hipLaunchKernelGGL((knn_threshold_kernel<1>), tgrid, dim3(256), 0, s, prm, per_query);
+  else if (per_query <= 128) hipLaunchKernelGGL((knn_threshold_kernel<2>), tgrid, dim3(256), 0, s, prm, per_query);
+  else if (per_query <= 256) hipLaunchKernelGGL((knn_threshold_kernel<4>), tgrid, dim3(256), 0, s, prm, per_query);
+  else hipLaunchKernelGGL((knn_threshold_kernel<8>), tgrid, dim3(256), 0, s, prm, per_query);
   const dim3 grid(qblocks, static_cast<unsigned>(prm.slices));
   if (prm.folds != nullptr) {
     if (prm.list == 8) hipLaunchKernelGGL((knn_candidates_kernel<KS, NQ, 2, true>), grid, dim3(256), 0, s, prm);
@@ -816,8 +819,17 @@ hipError_t launch_knn_stream(const KnnStreamParams& prm, hipStream_t s) {
   if (prm.query_rows == 0) return hipSuccess;
   const int steps = stream_steps(prm.dims, prm.parts, prm.euclid != 0);
   if (prm.dims < 1 || steps > kStreamMaxSteps || prm.k < 1 || prm.k > kStreamMaxK || prm.train_rows < 1 ||
-      prm.train_stride % 4 != 0 || prm.train_stride < prm.dims || prm.query_stride < prm.dims || prm.slices < 1 || prm.max_slices < 1 || prm.max_slices > kStreamMaxSlices || prm.sample_chunks < 1 || (prm.list != 8 && prm.list != 16) || (prm.list == 8 && prm.k > 32) ||
-      (prm.block_run != nullptr) != (prm.folds != nullptr) || prm.pad_rows % kStreamBlockRows != 0) {
+      prm.train_stride % 4 != 0 || prm.train_stride < prm.dims || prm.query_stride < prm.dims) {
+    return hipErrorInvalidValue;
+  }
+  if (prm.slices < 1 || prm.slices > kStreamMaxSlices || prm.max_slices < 1 || prm.max_slices > kStreamMaxSlices ||
+      prm.sample_chunks < 1 || (prm.list != 8 && prm.list != 16) || (prm.list == 8 && prm.k > 32)) {
+    return hipErrorInvalidValue;
+  }
+  const bool tables = prm.block_run != nullptr;
+  if (tables != (prm.folds != nullptr) || prm.query_begin % kStreamBlockRows != 0 ||
+      (tables ? prm.pad_rows % kStreamBlockRows != 0 || prm.query_rows > prm.pad_rows - prm.query_begin
+              : prm.query_begin != 0)) {
     return hipErrorInvalidValue;
   }
   switch (steps) {
@@ -831,7 +843,7 @@ hipError_t launch_knn_stream(const KnnStreamParams& prm, hipStream_t s) {
     case 8: launch_steps<8>(prm, s); break;
     default: launch_steps<9>(prm, s); break;
   }
-  const unsigned rblocks = static_cast<unsigned>(((prm.block_run != nullptr ? prm.pad_rows : prm.query_rows) + 3) / 4);
+  const unsigned rblocks = static_cast<unsigned>((prm.query_rows + 3) / 4);
   if (prm.euclid) hipLaunchKernelGGL((knn_stream_rerank_kernel<true>), dim3(rblocks), dim3(256), 0, s, prm);
   else hipLaunchKernelGGL((knn_stream_rerank_kernel<false>), dim3(rblocks), dim3(256), 0, s, prm);
   return hipGetLastError();

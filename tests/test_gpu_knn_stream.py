@@ -2,6 +2,9 @@
 candidates, exact rerank): neighbours and distances bit-identical to the
 oracle's exhaustive search where the operand width, the number of parts, the
 sample, the slices and the candidate buffers change."""
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 
@@ -131,3 +134,50 @@ def test_fold_tables_of_equal_rows(oracle):
         assert (K.last_knn_fallbacks() == 0) == (copies == 40)
         wn, ws = oracle.precompute_knn_cv(x, fids[0], 20, 2)
         assert np.array_equal(nbr[0], wn) and np.array_equal(score[0], ws)
+
+
+def test_fold_tables_of_many_runs_in_several_launches(oracle):
+    """1.07M padded rows with the larger buffers (2 KiB a row): three launches of
+    524288 rows at most, the last of a part, on 1 GiB of candidates. Equal to
+    the scan everywhere, and to the oracle in the runs around the seams."""
+    x, _ = D.config3(n=6000, p=4, seed=9)
+    rng = np.random.default_rng(1)
+    rows = [np.sort(rng.choice(6000, 5000, replace=False)).astype(np.int32) for _ in range(210)]
+    fids = [rng.integers(0, 7, 5000).astype(np.int32) for _ in rows]
+    K.release_memory()
+    least = _least_free()
+    with least:
+        nbr, score, used = K.knn_fold_tables(x, rows, fids, 40, "euclidean", path="mfma")
+    assert used == "mfma" and least.used < 2_000_000_000, least.used
+    sn, ss, used = K.knn_fold_tables(x, rows, fids, 40, "euclidean", path="scan")
+    assert used == "scan"
+    for r in range(210):
+        assert np.array_equal(nbr[r], sn[r]) and np.array_equal(score[r], ss[r]), r
+    for r in (0, 102, 204, 209):
+        wn, ws = oracle.precompute_knn_cv(x[rows[r]], fids[r], 40, 2)
+        assert np.array_equal(nbr[r], wn) and np.array_equal(score[r], ws), r
+
+
+class _least_free:
+    """The most device memory in use above the start while the block runs, as
+    the HIP runtime that the library is linked to reports it."""
+
+    def _free(self):
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert self._hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    def __enter__(self):
+        self._hip, self.used, self._stop = ctypes.CDLL("libamdhip64.so.7"), 0, threading.Event()
+        start = self._free()
+
+        def watch():
+            while not self._stop.is_set():
+                self.used = max(self.used, start - self._free())
+
+        self._thread = threading.Thread(target=watch)
+        self._thread.start()
+
+    def __exit__(self, *_):
+        self._stop.set()
+        self._thread.join()
