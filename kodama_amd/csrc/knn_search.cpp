@@ -73,9 +73,21 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
   // the buffer the width of k needs; the queries it cannot certify take three
   // parts and the larger buffer, and only what is left the scan.
   const bool same = d_query == d_train;
-  DeviceBuffer<float> t_n2(static_cast<size_t>(train_rows)), n2_max(2);
-  check(hipMemsetAsync(n2_max.get(), 0, 2 * sizeof(float), s), "memset");
-  check(launch_stream_norms(d_train, train_rows, dims, dims, t_n2.get(), n2_max.get(), s), "stream_norms launch");
+  // Norms: Euclidean, of the centred rows on both sides; inner product, the
+  // train rows' centred and as given, the queries' as given.
+  DeviceBuffer<float> center(static_cast<size_t>(dims)), t_n2(static_cast<size_t>(train_rows)), n2_max(3);
+  check(launch_stream_center(d_train, train_rows, dims, dims, center.get(), s), "stream_center launch");
+  check(hipMemsetAsync(n2_max.get(), 0, 3 * sizeof(float), s), "memset");
+  const float* const query_center = euclid ? center.get() : nullptr;
+  StreamNormsJob tn;
+  tn.x = d_train;
+  tn.rows = train_rows;
+  tn.p = tn.stride = dims;
+  tn.center = center.get();
+  tn.norm2_max = n2_max.get();
+  (euclid ? tn.norm2 : tn.given_norm2) = t_n2.get();
+  if (!euclid) tn.given_norm2_max = n2_max.get() + (same ? 1 : 2);
+  check(launch_stream_norms(tn, s), "stream_norms launch");
   // The rerank's 16-byte loads need rows of whole ones: a padded copy where
   // the columns are not a multiple of four (0.1 ms per million rows of 50).
   const int stride = stream_row_stride(dims);
@@ -93,10 +105,19 @@ void device_exact_knn(const float* d_train, int train_rows, const float* d_query
     DeviceBuffer<float> q_n2;
     if (!self) {
       q_n2.resize(static_cast<size_t>(rows));
-      check(launch_stream_norms(q, rows, dims, dims, q_n2.get(), n2_max.get() + 1, s), "stream_norms launch");
+      StreamNormsJob qn;
+      qn.x = q;
+      qn.rows = rows;
+      qn.p = qn.stride = dims;
+      qn.center = query_center;
+      qn.norm2 = q_n2.get();
+      qn.norm2_max = n2_max.get() + 1;
+      check(launch_stream_norms(qn, s), "stream_norms launch");
     }
     StreamOperandJob op;
     op.x = d_train;
+    op.train_center = center.get();
+    op.query_center = query_center;
     op.norm2 = t_n2.get();
     op.norm2_max = n2_max.get();
     op.rows = train_rows;
@@ -249,11 +270,23 @@ int device_fold_tables(const FoldTableJob& job, hipStream_t s) {
   }
 
   const int stride = stream_row_stride(job.p);
-  DeviceBuffer<float> xc(static_cast<size_t>(total) * stride), n2(static_cast<size_t>(total)), n2_max(2);
+  DeviceBuffer<float> xc(static_cast<size_t>(total) * stride), center(static_cast<size_t>(job.p)),
+    n2(static_cast<size_t>(total)), n2_max(3);
   DeviceBuffer<int> flags(static_cast<size_t>(total));
   check(launch_gather_rows(job.d_x, job.d_rows, total, job.p, xc.get(), s, stride), "gather_rows launch");
-  check(hipMemsetAsync(n2_max.get(), 0, 2 * sizeof(float), s), "memset");
-  check(launch_stream_norms(xc.get(), total, job.p, stride, n2.get(), n2_max.get(), s), "stream_norms launch");
+  // Norms and centre as in device_exact_knn for a set searched in itself.
+  check(launch_stream_center(xc.get(), total, job.p, stride, center.get(), s), "stream_center launch");
+  check(hipMemsetAsync(n2_max.get(), 0, 3 * sizeof(float), s), "memset");
+  StreamNormsJob norms;
+  norms.x = xc.get();
+  norms.rows = total;
+  norms.p = job.p;
+  norms.stride = stride;
+  norms.center = center.get();
+  norms.norm2_max = n2_max.get();
+  (euclid ? norms.norm2 : norms.given_norm2) = n2.get();
+  if (!euclid) norms.given_norm2_max = n2_max.get() + 1;
+  check(launch_stream_norms(norms, s), "stream_norms launch");
   std::vector<int> h_flags(static_cast<size_t>(total));
   auto pass = [&](int parts, int list) {
     const int steps = stream_steps(job.p, parts, euclid);
@@ -261,6 +294,8 @@ int device_fold_tables(const FoldTableJob& job, hipStream_t s) {
     StreamOperandJob op;
     op.x = xc.get();
     op.stride = stride;
+    op.train_center = center.get();
+    op.query_center = euclid ? center.get() : nullptr;
     op.norm2 = n2.get();
     op.norm2_max = n2_max.get();
     op.rows = total;

@@ -42,7 +42,7 @@ struct KnnStreamParams {
   const void* train_op = nullptr;   // operand fragments (launch_stream_operands)
   const void* query_op = nullptr;
   const float* query_norm2 = nullptr;  // [query rows]
-  const float* norm2_max = nullptr;    // [2] largest squared norm of the train rows, of the queries
+  const float* norm2_max = nullptr;    // [3], see StreamNormsJob
   int train_rows = 0, query_rows = 0, dims = 0, k = 0;
   int parts = 1, euclid = 0;
   const int* exclude = nullptr;     // [query rows] train row to skip, may be null
@@ -107,20 +107,42 @@ struct StreamPlan {
   }
 };
 
-// Squared norms [rows] (rows `stride` floats apart) and their maximum (into
-// *norm2_max, which the caller cleared to 0).
-hipError_t launch_stream_norms(const float* x, int rows, int p, int stride, float* norm2, float* norm2_max,
-                               hipStream_t s);
+// The operands are the rows less a centre: the error of a score grows with the
+// norms, and data away from the origin would otherwise be certified by little
+// but its offset. Euclidean distances do not change when every row is moved;
+// inner products change by q.centre, the same for all of a query's train rows,
+// when the train rows alone are. centre [p]: the mean of up to kStreamCenterRows
+// rows spread evenly (any centre gives the same results), finite values only, 0
+// where there is none.
+constexpr int kStreamCenterRows = 1024;
+hipError_t launch_stream_center(const float* x, int rows, int p, int stride, float* center, hipStream_t s);
+// Squared norms [rows] of the rows less the centre and of the rows as given
+// (either may be null), and their maxima. norm2_max of the searches is three
+// floats that the caller clears to 0: the largest of the train rows as their
+// operands have them, of the queries likewise, and (inner product) of the train
+// rows as given, unless the queries are the same rows.
+struct StreamNormsJob {
+  const float* x = nullptr;
+  int rows = 0, p = 0, stride = 0;
+  const float* center = nullptr;    // [p] (null: 0)
+  float* norm2 = nullptr;
+  float* norm2_max = nullptr;
+  float* given_norm2 = nullptr;
+  float* given_norm2_max = nullptr; // may be null
+};
+hipError_t launch_stream_norms(const StreamNormsJob& job, hipStream_t s);
 inline int stream_row_stride(int p) { return (p + 3) / 4 * 4; }
 // Rows -> operand fragments of `steps` x 32 columns, rows padded with zeros to
-// pad_rows; either output may be null. norm2_max [2] scales them. `tile` rows a
+// pad_rows; either output may be null. norm2_max scales them. `tile` rows a
 // fragment: 32 (x 16 columns, v_mfma_f32_32x32x16_f16) or 16 (x 32 columns,
 // v_mfma_f32_16x16x32_f16).
 // For the padded table layout pass block_run / run_offsets / pad_offsets.
 struct StreamOperandJob {
   const float* x = nullptr;
   int stride = 0;                   // floats between rows (0: p)
-  const float* norm2 = nullptr;
+  const float* train_center = nullptr;  // [p], of the rows as train rows / as queries (null: 0)
+  const float* query_center = nullptr;
+  const float* norm2 = nullptr;     // Euclidean train rows: of the centred rows
   const float* norm2_max = nullptr;
   int rows = 0, p = 0, parts = 1, euclid = 0;
   int tile = 32;

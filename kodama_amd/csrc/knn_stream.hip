@@ -2,12 +2,16 @@
 // an exact FP32 rerank.
 //
 // Score of a (query, train row) pair: s = q.t - |t|^2 / 2 (Euclidean) or q.t
-// (inner product, cosine rows); the nearest rows have the largest scores. All
-// rows are scaled by one power of two that brings the largest norm to at most
-// 2^14, rounded to FP16 (parts = 1) or split into two FP16 parts (parts = 3:
-// hi.hi + hi.lo + lo.hi along K), and the norm term rides in spare K columns
-// (2^13 on the query side, the FP16 parts of -|t|^2 / 2^14 on the train
-// side), so one v_mfma_f32_32x32x16_f16 chain gives s for 32 x 32 pairs. Each
+// (inner product, cosine rows); the nearest rows have the largest scores. The
+// train rows, and for Euclidean distances the queries, are taken less a sample's
+// mean, which moves no distance (or all of a query's inner products alike): the
+// error below follows the spread of the data and not their offset (50k x 128,
+// k = 30, at a mean of 10 standard deviations: 3.9 ms; without, every row was
+// flagged twice and scanned, 193 ms). All rows are scaled by one power of two
+// that brings the largest norm to at most 2^14, rounded to FP16 (parts = 1) or
+// split into two FP16 parts (parts = 3: hi.hi + hi.lo + lo.hi along K), and the
+// norm term rides in spare K columns (2^13 on the query side, the FP16 parts of
+// -|t|^2 / 2^14 on the train side), so one v_mfma_f32_32x32x16_f16 chain gives s for 32 x 32 pairs. Each
 // s differs from the exact distance's by at most E (pair_error below).
 //
 // Three kernels stream the train rows (a wave owns 32 NQ queries as B operands
@@ -117,30 +121,78 @@ __device__ __forceinline__ uint32_t kth_largest(const uint32_t (&key)[R], int us
 
 }  // namespace
 
-// 16 lanes per row; block maximum, one atomic per block (norms are >= 0, so
+// Mean of a sample of the rows. 16 columns a block, 64 threads a column with all
+// their loads in flight: one round trip to memory (four times as many in turn
+// added some 15 us to a call).
+__global__ void __launch_bounds__(1024) stream_center_kernel(const float* __restrict__ x, int rows, int p, int stride,
+                                                             float* __restrict__ center) {
+  constexpr int kParts = 64, kLoads = kStreamCenterRows / kParts;
+  __shared__ float s_sum[kParts][17];
+  __shared__ int s_count[kParts][17];
+  const int sub = threadIdx.x & 15, part = threadIdx.x >> 4;
+  const int c = static_cast<int>(blockIdx.x) * 16 + sub;
+  float v[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int e = part + i * kParts;
+    const size_t row = rows > kStreamCenterRows ? static_cast<size_t>(e) * static_cast<size_t>(rows) / kStreamCenterRows
+                                                : static_cast<size_t>(e);
+    v[i] = c < p && row < static_cast<size_t>(rows) ? x[row * stride + c] : INFINITY;
+  }
+  float sum = 0.0f;
+  int count = 0;
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const bool use = isfinite(v[i]);
+    sum += use ? v[i] : 0.0f;
+    count += use ? 1 : 0;
+  }
+  s_sum[part][sub] = sum;
+  s_count[part][sub] = count;
+  __syncthreads();
+  if (part != 0 || c >= p) return;
+#pragma unroll 8
+  for (int i = 1; i < kParts; ++i) {
+    sum += s_sum[i][sub];
+    count += s_count[i][sub];
+  }
+  const float mean = sum / static_cast<float>(max(count, 1));
+  center[c] = isfinite(mean) ? mean : 0.0f;
+}
+
+// 16 lanes per row; block maxima, one atomic each per block (norms are >= 0, so
 // their bits order as integers; a NaN norm does not enter).
-__global__ void stream_norms_kernel(const float* __restrict__ x, int rows, int p, int stride, float* __restrict__ norm2,
-                                    float* __restrict__ norm2_max) {
-  __shared__ uint32_t s_max;
-  if (threadIdx.x == 0) s_max = 0u;
+__global__ void stream_norms_kernel(StreamNormsJob job) {
+  __shared__ uint32_t s_max[2];
+  if (threadIdx.x < 2) s_max[threadIdx.x] = 0u;
   __syncthreads();
   const int sub = threadIdx.x & 15;
-  for (size_t r = static_cast<size_t>(blockIdx.x) * 16 + (threadIdx.x >> 4); r < static_cast<size_t>(rows);
+  for (size_t r = static_cast<size_t>(blockIdx.x) * 16 + (threadIdx.x >> 4); r < static_cast<size_t>(job.rows);
        r += static_cast<size_t>(gridDim.x) * 16) {
-    const float* src = x + r * stride;
-    float s = 0.0f;
-    for (int d = sub; d < p; d += 16) s = fmaf(src[d], src[d], s);
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    s += __shfl_xor(s, 4);
-    s += __shfl_xor(s, 8);
+    const float* src = job.x + r * job.stride;
+    float s = 0.0f, given = 0.0f;
+    for (int d = sub; d < job.p; d += 16) {
+      const float g = src[d], v = g - (job.center != nullptr ? job.center[d] : 0.0f);
+      s = fmaf(v, v, s);
+      given = fmaf(g, g, given);
+    }
+#pragma unroll
+    for (int m = 1; m < 16; m <<= 1) {
+      s += __shfl_xor(s, m);
+      given += __shfl_xor(given, m);
+    }
     if (sub == 0) {
-      norm2[r] = s;
-      if (s >= 0.0f) atomicMax(&s_max, __float_as_uint(s));
+      if (job.norm2 != nullptr) job.norm2[r] = s;
+      if (s >= 0.0f) atomicMax(&s_max[0], __float_as_uint(s));
+      if (job.given_norm2 != nullptr) job.given_norm2[r] = given;
+      if (given >= 0.0f) atomicMax(&s_max[1], __float_as_uint(given));
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0 && s_max != 0u) atomicMax(reinterpret_cast<uint32_t*>(norm2_max), s_max);
+  if (threadIdx.x == 0 && s_max[0] != 0u) atomicMax(reinterpret_cast<uint32_t*>(job.norm2_max), s_max[0]);
+  if (threadIdx.x == 1 && s_max[1] != 0u && job.given_norm2_max != nullptr) {
+    atomicMax(reinterpret_cast<uint32_t*>(job.given_norm2_max), s_max[1]);
+  }
 }
 
 // One thread per 16-byte fragment piece: with fragments of T rows (32 or 16)
@@ -182,11 +234,12 @@ __global__ void stream_operands_kernel(StreamOperandJob job, int steps) {
     if (live) {
       if (c < job.parts * p) {
         const int seg = c / p, d = c - seg * p;
-        const float v = src[d] * scale;
-        const _Float16 h = static_cast<_Float16>(v);
-        const _Float16 l = static_cast<_Float16>(v - static_cast<float>(h));
-        a = seg == 1 ? l : h;  // train: hi, lo, hi
-        b = seg == 2 ? l : h;  // query: hi, hi, lo
+        const float v = src[d];
+        const float t = (v - (job.train_center != nullptr ? job.train_center[d] : 0.0f)) * scale;
+        const float q = (v - (job.query_center != nullptr ? job.query_center[d] : 0.0f)) * scale;
+        const _Float16 th = static_cast<_Float16>(t), qh = static_cast<_Float16>(q);
+        a = seg == 1 ? static_cast<_Float16>(t - static_cast<float>(th)) : th;  // train: hi, lo, hi
+        b = seg == 2 ? static_cast<_Float16>(q - static_cast<float>(qh)) : qh;  // query: hi, hi, lo
       } else if (job.euclid) {
         const int j = c - job.parts * p;
         const _Float16 h = static_cast<_Float16>(nt);
@@ -231,6 +284,24 @@ __device__ __forceinline__ StreamRange stream_range(const KnnStreamParams& prm, 
     g.delta = prm.run_offsets[run] - g.t_begin;
   }
   return g;
+}
+
+// Roundings of the kNN distances (p <= 256: at most 8 block sums, the lane tree
+// of 5 and 31 tail terms in sequence, one rounding each: 50) and of a centred
+// row (2^-24 of it, which moves half a squared distance by at most
+// 2^-23 (q^2 + t^2)).
+constexpr float kDistanceRoundings = 52.0f;
+
+// 2E for a query of squared norm norm2, scaled. A Euclidean value is computed
+// from differences, which the centre does not enter; an inner product from the
+// rows as given.
+__device__ __forceinline__ float drop_error(const KnnStreamParams& prm, float norm2) {
+  const float scale = operand_scale(prm.norm2_max) * 1.0001f;
+  const float q = sqrtf(norm2) * scale;
+  const float t = sqrtf(prm.norm2_max[0]) * scale;
+  const float given = prm.euclid ? t : sqrtf(fmaxf(prm.norm2_max[1], prm.norm2_max[2])) * scale;
+  const int width = prm.parts * prm.dims + (prm.euclid ? 3 : 0);
+  return 2.0f * pair_error(q, t, prm.dims, prm.parts, width, q * q + given * given, kDistanceRoundings);
 }
 
 // LDS staging of 64 train rows: the next chunk is loaded into registers while
@@ -415,12 +486,7 @@ __global__ void __launch_bounds__(256) knn_threshold_kernel(KnnStreamParams prm,
   const int want = prm.k + (prm.exclude != nullptr ? 1 : 0);
   float bound = norms_usable(prm.norm2_max) ? -INFINITY : INFINITY;
   if (valid >= want && bound < 0.0f) {
-    const float scale = operand_scale(prm.norm2_max);
-    const float tmax = sqrtf(prm.norm2_max[0]) * scale * 1.0001f;
-    const float qn = sqrtf(prm.query_norm2[q + delta]) * scale * 1.0001f;
-    const int width = prm.parts * prm.dims + (prm.euclid ? 3 : 0);
-    bound = drop_bound(key_value(kth_largest<REGS>(key, REGS, want)),
-                       2.0f * pair_error(qn, tmax, prm.dims, prm.parts, width));
+    bound = drop_bound(key_value(kth_largest<REGS>(key, REGS, want)), drop_error(prm, prm.query_norm2[q + delta]));
   }
   if (lane == 0) prm.threshold[local] = bound;
 }
@@ -480,9 +546,6 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(Kn
     __builtin_amdgcn_wave_barrier();
     const int mine = lane < kWaveQueries ? s_cnt[wave][lane] : 0;
     uint64_t todo = __ballot(mine > limit);
-    const float scale = operand_scale(prm.norm2_max);
-    const float tmax = sqrtf(prm.norm2_max[0]) * scale * 1.0001f;
-    const int width = prm.parts * prm.dims + (prm.euclid ? 3 : 0);
     while (todo != 0ull) {
       const int q = __builtin_ctzll(todo);
       todo &= todo - 1ull;
@@ -496,9 +559,8 @@ __global__ void __launch_bounds__(256, KS <= 2 ? 4 : 2) knn_candidates_kernel(Kn
         ent[i] = e < n ? base[e] : make_uint2(0xFF800000u, 0u);  // -inf
         key[i] = e < n ? order_key(__uint_as_float(ent[i].x)) : 0u;
       }
-      const float qn = sqrtf(prm.query_norm2[q_wave + q + g.delta]) * scale * 1.0001f;
       const float bound = drop_bound(key_value(kth_largest<R>(key, R, prm.k)),
-                                     2.0f * pair_error(qn, tmax, prm.dims, prm.parts, width));
+                                     drop_error(prm, prm.query_norm2[q_wave + q + g.delta]));
       int kept = 0;
       const uint64_t below = (1ull << lane) - 1ull;
 #pragma unroll
@@ -704,14 +766,10 @@ __global__ void __launch_bounds__(256, 4) knn_stream_rerank_kernel(KnnStreamPara
   __builtin_amdgcn_wave_barrier();
   // A tighter bound only where it can save a round of 64 exact distances.
   if ((n + kWave - 1) / kWave > (k + kWave - 1) / kWave) {
-    const float scale = operand_scale(prm.norm2_max);
-    const float tmax = sqrtf(prm.norm2_max[0]) * scale * 1.0001f;
-    const float qn = sqrtf(prm.query_norm2[q]) * scale * 1.0001f;
-    const int width = prm.parts * p + (prm.euclid ? 3 : 0);
     const uint32_t kth = n <= 2 * kWave   ? kth_of_entries<2>(ent, n, k, lane)
                          : n <= 4 * kWave ? kth_of_entries<4>(ent, n, k, lane)
                                           : kth_of_entries<kStreamMerge / kWave>(ent, n, k, lane);
-    bound = drop_bound(key_value(kth), 2.0f * pair_error(qn, tmax, p, prm.parts, width));
+    bound = drop_bound(key_value(kth), drop_error(prm, prm.query_norm2[q]));
     // In-place compaction: a register's entries go to slots at or before
     // their own, and each is read before a later register's is written.
     int kept = 0;
@@ -768,12 +826,19 @@ __global__ void __launch_bounds__(256, 4) knn_stream_rerank_kernel(KnnStreamPara
   }
 }
 
-hipError_t launch_stream_norms(const float* x, int rows, int p, int stride, float* norm2, float* norm2_max,
-                               hipStream_t s) {
-  if (rows == 0) return hipSuccess;
-  const int blocks = (rows + 15) / 16;
-  hipLaunchKernelGGL(stream_norms_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s, x,
-                     rows, p, stride, norm2, norm2_max);
+hipError_t launch_stream_center(const float* x, int rows, int p, int stride, float* center, hipStream_t s) {
+  if (rows < 1 || p < 1 || stride < p) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(stream_center_kernel, dim3(static_cast<unsigned>((p + 15) / 16)), dim3(1024), 0, s, x, rows,
+                     p, stride, center);
+  return hipGetLastError();
+}
+
+hipError_t launch_stream_norms(const StreamNormsJob& job, hipStream_t s) {
+  if (job.rows == 0) return hipSuccess;
+  if (job.p < 1 || job.stride < job.p || job.norm2_max == nullptr) return hipErrorInvalidValue;
+  const int blocks = (job.rows + 15) / 16;
+  hipLaunchKernelGGL(stream_norms_kernel, dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, s,
+                     job);
   return hipGetLastError();
 }
 

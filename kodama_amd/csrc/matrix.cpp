@@ -123,7 +123,7 @@ struct DeviceLloyd {
 
   DeviceLloyd(const float* x, int runs_, int n_, int p_, int k_, hipStream_t stream)
       : d_x(x), runs(runs_), n(n_), p(p_), k(k_), s(stream), xn(static_cast<size_t>(runs) * n),
-        cent(static_cast<size_t>(runs) * k * p), cn(static_cast<size_t>(runs) * k), sizes(cn.size()), norm2_max(2),
+        cent(static_cast<size_t>(runs) * k * p), cn(static_cast<size_t>(runs) * k), sizes(cn.size()), norm2_max(3),
         asg(xn.size()), changed(static_cast<size_t>(runs) + 1),
         offsets(static_cast<size_t>(runs) * k * kmeans_segments(n)), members(xn.size()) {
     // Three FP16 parts where they are as wide as one.
@@ -134,7 +134,7 @@ struct DeviceLloyd {
     row_op.resize(stream_operand_bytes(static_cast<size_t>(runs) * pad_n, steps));
     cent_op.resize(stream_operand_bytes(static_cast<size_t>(runs) * pad_k, steps));
     check(hipMemsetAsync(asg.get(), 0xFF, sizeof(int) * asg.size(), s), "memset");  // -1: unassigned
-    check(hipMemsetAsync(norm2_max.get(), 0, 2 * sizeof(float), s), "memset");
+    check(hipMemsetAsync(norm2_max.get(), 0, 3 * sizeof(float), s), "memset");
     check(launch_sse_norms(d_x, runs * n, p, xn.get(), norm2_max.get(), s), "sse_norms launch");
     StreamOperandJob op = operand_job(d_x, xn.get(), n, pad_n);
     op.query_op = row_op.get();

@@ -257,7 +257,7 @@ __global__ void __launch_bounds__(kBlock, KS <= 8 ? 2 : 1) kmeans_assign_kernel(
     m = fmaxf(m, __shfl_xor(m, 32));
     const int row = row0 + t * 16 + col;
     const float qn = row < n ? sqrtf(x_norm[row]) * scale * 1.0001f : 0.0f;
-    const float err = pair_error(qn, cmax, p, prm.parts, prm.parts * p + 3, kAssignRoundings);
+    const float err = pair_error(qn, cmax, p, prm.parts, prm.parts * p + 3, qn * qn + cmax * cmax, kAssignRoundings);
     th[t] = usable ? drop_bound(m, 2.0f * err) : -INFINITY;
   }
   stream(std::integral_constant<int, 1>{});

@@ -33,7 +33,7 @@ struct KmeansAssignParams {
   const int* active = nullptr;
   const void* row_op = nullptr;
   const void* centroid_op = nullptr;
-  const float* norm2_max = nullptr;  // [2]: the largest row norm, 0
+  const float* norm2_max = nullptr;  // [3]: the largest row norm, 0, 0
   const float* c_norm_max = nullptr; // largest of c_norm over all problems
   int parts = 1, pad_n = 0, pad_k = 0;
 };

@@ -36,7 +36,7 @@ __device__ __forceinline__ float operand_scale(const float* __restrict__ norm2_m
 // underflow) are not served: every query is flagged.
 __device__ __forceinline__ bool norms_usable(const float* __restrict__ norm2_max) {
   const float m = fmaxf(norm2_max[0], norm2_max[1]);
-  return m < 1e37f && (m == 0.0f || m > 1e-30f);
+  return m < 1e37f && norm2_max[2] < 1e37f && (m == 0.0f || m > 1e-30f);
 }
 
 // Bound of |s - exact score| in scaled units, for a query of scaled norm q and
@@ -46,17 +46,14 @@ __device__ __forceinline__ bool norms_usable(const float* __restrict__ norm2_max
 //   flushed operands          2.1 2^-14 sqrt(p) (q + t) + 1,
 //   FP32 accumulation         K 2^-23 (q t + t^2 / 2), any order,
 //   the norm column           2^-22 t^2 / 2, and its FP32 sum (p + 2) 2^-25 t^2,
-//   the reference's own FP32 value  ref 2^-24 (q^2 + t^2).
-// ref = 50 for the kNN distances (p <= 256: at most 8 block sums, the lane tree
-// of 5 and 31 tail terms in sequence, one rounding each).
-constexpr float kDistanceRoundings = 50.0f;
-__device__ __forceinline__ float pair_error(float q, float t, int p, int parts, int width,
-                                            float ref = kDistanceRoundings) {
+//   the reference's own FP32 value  ref 2^-24 values2, values2 the sum of the
+//   squared (scaled) norms that this value is computed from.
+__device__ __forceinline__ float pair_error(float q, float t, int p, int parts, int width, float values2, float ref) {
   const float u = 0x1p-11f;
   const float c1 = (parts == 1 ? 2.0f * u + u * u : 3.1f * u * u) + width * 0x1.04p-23f;
-  const float c2 = 0x1p-23f + (p + 2) * 0x1p-25f + ref * 0x1p-24f + width * 0x1p-24f;
+  const float c2 = 0x1p-23f + (p + 2) * 0x1p-25f + width * 0x1p-24f;
   const float c3 = 2.1f * 0x1p-14f * sqrtf(static_cast<float>(p));
-  return 1.05f * (c1 * q * t + c2 * (q * q + t * t) + c3 * (q + t) + 1.0f);
+  return 1.05f * (c1 * q * t + c2 * (q * q + t * t) + ref * 0x1p-24f * values2 + c3 * (q + t) + 1.0f);
 }
 
 // Wave maximum / minimum by DPP (gfx9 row shifts and row broadcasts), uniform.

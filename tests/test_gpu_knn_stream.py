@@ -181,3 +181,77 @@ class _least_free:
     def __exit__(self, *_):
         self._stop.set()
         self._thread.join()
+
+
+# Rows far from the origin against their spread, on both sides of the width
+# where the second pass can take three parts (95 / 96 columns).
+@pytest.mark.parametrize("p", [50, 95, 96, 128, 256])
+@pytest.mark.parametrize("offset", [10.0, 1000.0])
+def test_rows_away_from_the_origin(oracle, p, offset):
+    rng = np.random.default_rng(p)
+    x = (rng.standard_normal((6100, p), dtype=np.float32) + np.float32(offset)).astype(np.float32)
+    x[:, 0] -= np.float32(2 * offset)  # columns of both signs
+    ex = (np.arange(1100, dtype=np.int32) * 37) % 5000
+    _check(oracle, x[:5000], x[5000:], 30, "euclidean", exclude=ex)
+    _check(oracle, x[:5000], x[5000:], 30, "inner_product")
+    g = K.KODAMA_knn_graph(x[:5000], k=30)
+    assert K.last_knn_fallbacks() == 0
+    idx, dist = oracle.knn_graph(x[:5000], 30, 2)
+    assert np.array_equal(g["indices"], idx) and np.array_equal(g["distances"], dist)
+
+
+def test_cosine_rows_around_one_direction(oracle):
+    rng = np.random.default_rng(2)
+    x = (rng.standard_normal((6000, 110), dtype=np.float32) + np.float32(10)).astype(np.float32)
+    g = K.KODAMA_knn_graph(x, k=20, metric="cosine")
+    assert K.last_knn_fallbacks() == 0
+    idx, dist = oracle.knn_graph(x, 20, 0)
+    assert np.array_equal(g["indices"], idx) and np.array_equal(g["distances"], dist)
+
+
+@pytest.mark.parametrize("name", ["euclidean", "cosine", "inner_product"])
+def test_fold_tables_away_from_the_origin(oracle, name):
+    rng = np.random.default_rng(4)
+    x = (rng.standard_normal((3000, 150), dtype=np.float32) + np.float32(20)).astype(np.float32)
+    rows, fids = _uneven(x, [900, 257, 1500], folds=5, seed=8)
+    nbr, score, used = K.knn_fold_tables(x, rows, fids, 20, name, path="mfma")
+    assert used == "mfma" and K.last_knn_fallbacks() == 0
+    for r, (rw, f) in enumerate(zip(rows, fids)):
+        wn, ws = oracle.precompute_knn_cv(x[rw], f, 20, K._metric(name))
+        assert np.array_equal(nbr[r], wn) and np.array_equal(score[r], ws), r
+
+
+@pytest.mark.parametrize("name", ["euclidean", "inner_product"])
+@pytest.mark.parametrize("what", ["huge_row", "nan_column", "equal_rows", "overflow"])
+def test_centres_that_help_nothing(oracle, name, what):
+    """A sample whose mean is useless or undefined changes no result: one row
+    that outweighs all others, a column without a finite value in the sample
+    (its rows are nobody's neighbours), rows that are all the same away from
+    the origin, and sums past the largest float."""
+    x, _ = D.config3(n=5200, p=40, seed=6)
+    train, query = x[:5000].copy(), x[5000:].copy()
+    if what == "huge_row":
+        train[0] = 1e15
+    elif what == "nan_column":
+        train[:, 3] = np.nan
+    elif what == "equal_rows":
+        train[:] = query[0] + np.float32(30)
+    else:
+        train[:, 5] = 3e38
+        query[:, 5] = 3e38
+    idx, dist = K.exact_knn_search(train, query, 6, name)
+    if what == "nan_column":
+        assert (idx == -1).all() and np.isinf(dist).all()
+        return
+    want = oracle.exact_knn(train, query, 6, K._metric(name))
+    assert np.array_equal(idx, want[0]) and np.array_equal(dist, want[1])
+
+
+def test_inner_product_rows_larger_than_what_is_left_of_them(oracle):
+    """Train rows whose offset is 30000 times their spread: the products' own
+    rounding hides their order from the scores, and the scan answers."""
+    rng = np.random.default_rng(9)
+    x = (rng.standard_normal((5200, 100), dtype=np.float32) + np.float32(30000)).astype(np.float32)
+    idx, dist = K.exact_knn_search(x[:4100], x[4100:], 12, "inner_product")
+    want = oracle.exact_knn(x[:4100], x[4100:], 12, 1)
+    assert np.array_equal(idx, want[0]) and np.array_equal(dist, want[1])
