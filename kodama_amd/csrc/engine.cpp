@@ -655,7 +655,6 @@ void KnnBatch::allocate(const IVec& run_offsets) {
   d_nbr_.resize(static_cast<size_t>(k_) * pad_total_);
   d_score_.resize(static_cast<size_t>(k_) * pad_total_);
   d_labels_.resize(static_cast<size_t>(pad_total_));
-  d_pred_.resize(static_cast<size_t>(pad_total_));
   d_counts_.resize(static_cast<size_t>(runs_) * classes_);
   d_firsts_.resize(static_cast<size_t>(runs_) * classes_);
   d_matches_.resize(static_cast<size_t>(runs_));

@@ -184,8 +184,6 @@ class KnnBatch {
 
   DeviceBuffer<int>& d_neighbors() { return d_nbr_; }
   DeviceBuffer<float>& d_scores() { return d_score_; }
-  DeviceBuffer<int>& d_labels() { return d_labels_; }
-  DeviceBuffer<int>& d_pred() { return d_pred_; }
   DeviceBuffer<int>& d_block_run() { return d_block_run_; }
   DeviceBuffer<int>& d_run_offsets() { return d_run_off_; }
   DeviceBuffer<int>& d_pad_offsets() { return d_pad_off_; }
@@ -199,7 +197,7 @@ class KnnBatch {
   Stream stream_;
   int runs_ = 0, k_ = 0, pad_total_ = 0, classes_ = 0, blocks_ = 0, max_rows_ = 0;
   IVec run_offsets_, pad_offsets_;
-  DeviceBuffer<int> d_nbr_, d_labels_, d_pred_, d_block_run_, d_run_off_, d_pad_off_;
+  DeviceBuffer<int> d_nbr_, d_labels_, d_block_run_, d_run_off_, d_pad_off_;
   DeviceBuffer<float> d_score_;
   DeviceBuffer<int> d_counts_, d_firsts_, d_matches_;
   PinnedBuffer<int> h_labels_, h_pred_, h_counts_, h_firsts_, h_matches_;
