@@ -1,7 +1,7 @@
 """Per-fold kNN tables of a batch of runs (precompute_knn_cv, core.cpp:694-782):
-the register scan and the split-BF16 MFMA candidates with the exact rerank
-must both give the oracle's tables bit-exactly (run-local ids in (distance,
-id) order, float32 scores), and the tuned choice must not change results."""
+the register scan and the matrix-core candidates with the exact rerank must
+both give the oracle's tables bit-exactly (run-local ids in (distance, id)
+order, float32 scores), and the rule that chooses must not change results."""
 import numpy as np
 import pytest
 
@@ -57,7 +57,7 @@ def test_fold_tables_ties_and_short_runs(oracle):
 
 def test_fold_tables_c3_shape(oracle):
     """Runs of 1000-5000 landmark rows on the 100k mixture with 10 uneven folds:
-    the shape of the batched evolution, where the MFMA path is meant to win."""
+    the shape of the batched evolution, where the matrix-core path serves."""
     x, _ = D.config3(n=100_000, p=50)
     rng = np.random.default_rng(6)
     sizes = rng.integers(1000, 5001, size=3)
@@ -65,12 +65,12 @@ def test_fold_tables_c3_shape(oracle):
     _check(oracle, x, rows, fids, 30, "euclidean")
 
 
-def test_tuned_path_is_stable_and_exact(oracle):
+def test_path_by_rule_is_stable_and_exact(oracle):
     x, _ = D.config3(n=5000, p=50, seed=4)
     rows, fids = _runs(x, [1500, 2500], folds=10, seed=3)
     first = K.knn_fold_tables(x, rows, fids, 30, "euclidean", path="tuned")
     second = K.knn_fold_tables(x, rows, fids, 30, "euclidean", path="tuned")
-    assert first[2] == second[2]  # the bucket's choice is cached
+    assert first[2] == second[2] == "mfma"
     for a, b in zip(first[0], second[0]):
         assert np.array_equal(a, b)
     _check(oracle, x, rows, fids, 30, "euclidean", paths=("tuned",))
@@ -96,17 +96,16 @@ def test_batch_evolution_identical_under_both_paths():
     assert np.array_equal(out["scan"]["vect_acc"], out["mfma"]["vect_acc"])
 
 
-@pytest.mark.parametrize("list_,waves", [(8, 4), (8, 8), (16, 4), (16, 8)])
+@pytest.mark.parametrize("list_", [8, 16])
 @pytest.mark.parametrize("k", [12, 30, 40])
-def test_fold_table_schedules_match_oracle(oracle, list_, waves, k):
-    """Every MFMA schedule the tuner chooses from (candidates per lane column,
-    waves per workgroup) gives the oracle's tables; a list of 8 cannot serve
-    k > 32, which then takes the scan."""
+def test_fold_table_schedules_match_oracle(oracle, list_, k):
+    """Both buffer sizes (16 x list rows per query and slice) give the oracle's
+    tables; a list of 8 cannot serve k > 32, which then takes the scan."""
     x, _ = D.config3(n=5000, p=50, seed=21)
-    rows, fids = _runs(x, [1500, 2400, 300], folds=10, seed=k + list_ + waves)
+    rows, fids = _runs(x, [1500, 2400, 300], folds=10, seed=k + list_)
     want = [oracle.precompute_knn_cv(x[rw], f, k, K._metric("euclidean")) for rw, f in zip(rows, fids)]
     try:
-        K.set_fold_table_schedule("tuned", list_, waves)
+        K.set_fold_table_schedule("tuned", list_, 0)
         nbr, score, used = K.knn_fold_tables(x, rows, fids, k, "euclidean", path="mfma")
         sched = K.last_fold_table_schedule()
     finally:
@@ -114,44 +113,37 @@ def test_fold_table_schedules_match_oracle(oracle, list_, waves, k):
     if list_ == 8 and k > 32:
         assert used == "scan" and sched["path"] == "scan"
     else:
-        assert used == "mfma" and sched == dict(path="mfma", list=list_, waves=waves)
+        assert used == "mfma" and (sched["path"], sched["list"]) == ("mfma", list_)
     for r, (wn, ws) in enumerate(want):
         assert np.array_equal(nbr[r], wn), r
         assert np.array_equal(score[r], ws), r
 
 
-def test_tuner_times_schedules_and_keeps_its_choice(oracle):
-    """With everything tuned, the first table of a shape bucket times the scan
-    and the four MFMA schedules; the choice is kept for the bucket and the
-    tables are the oracle's either way."""
-    x, _ = D.config3(n=6000, p=40, seed=33)
-    rows, fids = _runs(x, [1800, 2200], folds=8, seed=4)
-    K.set_fold_table_schedule("tuned", 0, 0)
-    first = K.knn_fold_tables(x, rows, fids, 20, "euclidean", path="tuned")
-    s1 = K.last_fold_table_schedule()
-    second = K.knn_fold_tables(x, rows, fids, 20, "euclidean", path="tuned")
-    s2 = K.last_fold_table_schedule()
-    assert s1 == s2 and s1["path"] in ("scan", "mfma")
-    if s1["path"] == "mfma":
-        assert s1["list"] in (8, 16) and s1["waves"] in (4, 8)
-    want = [oracle.precompute_knn_cv(x[rw], f, 20, K._metric("euclidean")) for rw, f in zip(rows, fids)]
-    for out in (first, second):
-        for r, (wn, ws) in enumerate(want):
-            assert np.array_equal(out[0][r], wn) and np.array_equal(out[1][r], ws)
+def test_wave_setting_is_kept_and_reported():
+    """waves chooses nothing any more: callers that set it read it back, and
+    other values are refused."""
+    x, _ = D.config3(n=800, p=10, seed=2)
+    rows, fids = _runs(x, [500], folds=4, seed=1)
+    try:
+        for waves, reported in ((0, 4), (4, 4), (8, 8)):
+            K.set_fold_table_schedule("tuned", 0, waves)
+            K.knn_fold_tables(x, rows, fids, 10, "euclidean", path="mfma")
+            assert K.last_fold_table_schedule() == dict(path="mfma", list=8, waves=reported)
+        with pytest.raises(ValueError):
+            K.set_fold_table_schedule("tuned", 0, 5)
+    finally:
+        K.set_fold_table_schedule("tuned", 0, 0)
 
 
-def test_tuned_choice_is_kept_per_k_bucket(oracle):
-    """A schedule tuned for k <= 32 (possibly 8 candidates per lane column) is
-    not reused for a k above 32 on the same shape: each k bucket is tuned on
-    its own and both tables are the oracle's."""
+def test_list_by_rule_follows_k(oracle):
+    """Without a setting the buffers are the smaller ones up to 32 neighbours
+    and the larger ones beyond, build after build."""
     x, _ = D.config3(n=6000, p=50, seed=47)
     rows, fids = _runs(x, [2600, 3100], folds=10, seed=9)
     K.set_fold_table_schedule("tuned", 0, 0)
-    for k in (30, 40):
+    for k, list_ in ((32, 8), (33, 16), (20, 8)):
         nbr, score, used = K.knn_fold_tables(x, rows, fids, k, "euclidean", path="tuned")
-        sched = K.last_fold_table_schedule()
-        if sched["path"] == "mfma" and k > 32:
-            assert sched["list"] == 16
+        assert used == "mfma" and K.last_fold_table_schedule()["list"] == list_
         want = [oracle.precompute_knn_cv(x[rw], f, k, K._metric("euclidean")) for rw, f in zip(rows, fids)]
         for r, (wn, ws) in enumerate(want):
             assert np.array_equal(nbr[r], wn) and np.array_equal(score[r], ws), (k, r)

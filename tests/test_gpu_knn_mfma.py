@@ -1,6 +1,6 @@
-"""Split-BF16 MFMA candidates + exact FP32 rerank: neighbour ids and distances
+"""Matrix-core candidates + exact FP32 rerank: neighbour ids and distances
 bit-identical to the exact scan (the oracle restates the reference's order),
-including the queries the candidate lists cannot certify (exact fallback)."""
+including the queries the candidate buffers cannot certify (exact fallback)."""
 import numpy as np
 import pytest
 
@@ -23,8 +23,8 @@ def test_graph_via_mfma_matches_oracle(oracle, metric, name):
 
 @pytest.mark.parametrize("k,metric,name", [(33, 2, "euclidean"), (100, 2, "euclidean"), (100, 0, "cosine")])
 def test_wide_graph_via_mfma_matches_oracle(oracle, k, metric, name):
-    """More than 32 neighbours: 16-entry candidate lists per lane column (256
-    candidates per query), the same certification and exact rerank."""
+    """More than 32 neighbours: buffers of 256 candidates per query and slice,
+    the same certification and exact rerank."""
     x, _ = D.config3(n=6000, p=50, seed=k)
     g = K.KODAMA_knn_graph(x, k=k, metric=name)
     fb = K.last_knn_fallbacks()
@@ -47,9 +47,9 @@ def test_search_with_exclusion_and_dimension_tail(oracle):
 
 
 def test_duplicate_rows_take_the_exact_fallback(oracle):
-    """1000 copies of each of 5 rows: every column list fills with (near-)zero
-    candidate values inside the bound, so no query can be certified and the
-    exact scan answers them all (ties resolved by index)."""
+    """1000 copies of each of 5 rows: more candidates inside the bound than the
+    buffers hold, so no query can be certified and the exact scan answers them
+    all (ties resolved by index)."""
     base, _, _ = D.config1(n=5, seed=9)
     x = np.repeat(base, 1000, axis=0)
     g = K.KODAMA_knn_graph(x, k=24)
