@@ -210,37 +210,20 @@ def copy_probe() -> int:
     return 0
 
 
-def graph_bench(rows: int, k: int, lists_ab: bool = False) -> int:
+def graph_bench(rows: int, k: int) -> int:
     """Exact self-kNN graph of the 20-cluster mixture (config-4 generator,
-    p = 50) through the matrix-core path; one JSON line. With lists_ab,
-    the graph is built with packed candidate lists, separate ones and packed
-    again (one line each, and whether the graphs are identical)."""
+    p = 50) through the matrix-core path; one JSON line. The rate counts two
+    operations per column of each pair over the whole call."""
     import kodama_amd as K
     from kodama_amd import datasets as D
     x, _ = D.config4(n=rows)
     K.KODAMA_knn_graph(x[:8192], k=k)  # warm-up (code objects, allocator)
-    forms = (True, False, True) if lists_ab else (True,)
-    first = None
-    try:
-        for packed in forms:
-            K.set_mfma_packed_lists(packed)
-            t0 = time.perf_counter()
-            g = K.KODAMA_knn_graph(x, k=k)
-            wall = time.perf_counter() - t0
-            fb = K.last_knn_fallbacks()
-            flops = 2.0 * rows * rows * 50 * 3  # three bf16 products per MAC (hi.hi, hi.lo, lo.hi)
-            line = {"graph_rows": rows, "k": k, "p": 50, "seconds": wall, "fallback_queries": fb,
-                    "candidate_bf16_tflops_per_s": flops / wall / 1e12, "neighbors": int(g["neighbors"])}
-            if lists_ab:
-                line["packed_lists"] = packed
-                if first is None:
-                    first = (g["indices"], g["distances"])
-                else:
-                    line["identical"] = bool(np.array_equal(first[0], g["indices"]) and
-                                             np.array_equal(first[1], g["distances"]))
-            print(json.dumps(line), flush=True)
-    finally:
-        K.set_mfma_packed_lists(True)
+    t0 = time.perf_counter()
+    g = K.KODAMA_knn_graph(x, k=k)
+    wall = time.perf_counter() - t0
+    print(json.dumps({"graph_rows": rows, "k": k, "p": 50, "seconds": wall, "fallback_queries": K.last_knn_fallbacks(),
+                      "pair_tflops_per_s": 2.0 * rows * rows * 50 / wall / 1e12, "neighbors": int(g["neighbors"])}),
+          flush=True)
     return 0
 
 
@@ -277,21 +260,18 @@ def matrix_bench(rows: int, runs: int, cycles: int, k: int, forms) -> int:
 
 
 def tables_bench(runs: int, n: int, k: int) -> int:
-    """Per-fold kNN tables of the batched-runs workload built under every
-    schedule setting (register scan; matrix-core candidates + exact rerank with
-    buffers of 128 or 256 rows per query, the wave and list-form settings as
-    they are kept), twice each, then the build the rule chooses; one JSON line
-    per build with its wall time, the rows the matrix-core path flagged, and
-    whether the tables equal the scan's."""
+    """Per-fold kNN tables of the batched-runs workload built by the register
+    scan and by matrix-core candidates + exact rerank with buffers of 128 (k <=
+    32) and 256 rows per query, twice each, then the build the rule chooses; one
+    JSON line per build with its wall time, the rows the matrix-core path
+    flagged, and whether the tables equal the scan's."""
     import kodama_amd as K
     x, rows, fids, _ = make_workload(runs, n, 50, k)
     ref = None
-    builds = [("scan", 0, 0, True)] + [("mfma", l, w, pk) for l in (8, 16) if l == 16 or k <= 32 for w in (8, 4)
-                                       for pk in (True, False)]
+    builds = [("scan", 0)] + [("mfma", lst) for lst in (8, 16) if lst == 16 or k <= 32]
     try:
-        for path, lst, waves, packed in builds * 2 + [("tuned", 0, 0, True)]:
-            K.set_fold_table_schedule("tuned", lst, waves)
-            K.set_mfma_packed_lists(packed)
+        for path, lst in builds * 2 + [("tuned", 0)]:
+            K.set_fold_table_schedule("tuned", lst, 0)
             t0 = time.perf_counter()
             nbr, score, used = K.knn_fold_tables(x, rows, fids, k, "euclidean", path=path)
             wall = time.perf_counter() - t0
@@ -301,12 +281,12 @@ def tables_bench(runs: int, n: int, k: int) -> int:
             else:
                 same = all(np.array_equal(a, b) for a, b in zip(nbr, ref[0])) and \
                     all(np.array_equal(a, b) for a, b in zip(score, ref[1]))
-            print(json.dumps({"tables": path, "schedule": K.last_fold_table_schedule(), "packed_lists": packed,
-                              "runs": runs, "n": n, "k": k, "seconds": wall,
-                              "mfma_fallback_rows": K.last_knn_fallbacks(), "equal_to_scan": same}), flush=True)
+            sched = K.last_fold_table_schedule()
+            print(json.dumps({"tables": path, "used": sched["path"], "list": sched["list"], "runs": runs, "n": n, "k": k,
+                              "seconds": wall, "mfma_fallback_rows": K.last_knn_fallbacks(), "equal_to_scan": same}),
+                  flush=True)
     finally:
         K.set_fold_table_schedule("tuned", 0, 0)
-        K.set_mfma_packed_lists(True)
     return 0
 
 
@@ -460,8 +440,6 @@ def main() -> int:
                     help="launch split evolution runs as an ordinary grid instead of cooperatively "
                          "(rocprofv3 ends with a fault after tracing cooperative launches and writes nothing)")
     ap.add_argument("--graph-rows", type=int, default=0, help="time the exact k-NN graph of this many rows and exit")
-    ap.add_argument("--lists-ab", action="store_true",
-                    help="with --graph-rows: build the graph with packed and with separate candidate lists")
     ap.add_argument("--learned-curve", action="store_true",
                     help="accuracy against wall time of the uniform and learned proposals on the 200k"
                          " label-noise configuration (--steps cycles, default 100 here) and exit")
@@ -475,7 +453,7 @@ def main() -> int:
     if args.copy_probe:
         return copy_probe()
     if args.graph_rows > 0:
-        return graph_bench(args.graph_rows, args.k, args.lists_ab)
+        return graph_bench(args.graph_rows, args.k)
     if args.tables:
         return tables_bench(args.runs, args.n, args.k)
     if args.learned_curve:
