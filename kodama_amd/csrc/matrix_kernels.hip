@@ -30,6 +30,11 @@
 // to 64 landmark neighbours sit in the lane's LDS slice, the results leave
 // through LDS as whole lines. A thread per (row, run) read the graph row once
 // per run, uncoalesced: 8.2 ms for 100k rows, 100 neighbours and 100 runs.
+// project_few_kernel: up to 32 runs the table has as many entries a row as the
+// next power of two, and as many lanes work on a row. 64 lanes and 128 bytes a
+// row for one run cost 1M rows 11 ms (and 128 MB) that the call's projection
+// does not take now (74.6 -> 63.4 ms, most of it the caller's graph; 32 runs
+// 77.8 -> 74.1).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -407,66 +412,67 @@ __global__ void __launch_bounds__(kBlock) local_scatter_kernel(ProjectParams prm
   static_cast<T*>(prm.local)[static_cast<size_t>(prm.landmarks[begin + j]) * prm.run_stride + r] = static_cast<T>(j);
 }
 
+// The result of row i in a run: `local` is the run's column of the table, `row`
+// the graph row, `votes` this lane's LDS slice (an entry per 64 lanes). Whole
+// waves; `mine` is false in lanes without a row or run.
+template <class T>
+__device__ __forceinline__ int project_row(const ProjectParams& prm, const int* row, const T* local, int i,
+                                           const int* lab, bool mine, int* votes) {
+  constexpr T kNone = static_cast<T>(-1);
+  const T self = mine ? local[static_cast<size_t>(i) * prm.run_stride] : kNone;
+  int nv = 0;
+  bool open = mine && self == kNone;  // still collects votes
+  for (int j0 = 0; j0 < prm.neighbors && __ballot(open) != 0ull; j0 += 8) {
+    // Eight neighbours' table rows in flight.
+    T pos[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int g = j0 + u < prm.neighbors ? row[j0 + u] : -1;
+      pos[u] = g >= 0 && g < prm.n ? local[static_cast<size_t>(g) * prm.run_stride] : kNone;
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (open && pos[u] != kNone) {
+        votes[nv * 64] = static_cast<int>(pos[u]);
+        open = ++nv < prm.votes;
+      }
+    }
+  }
+  if (!mine) return 0;
+  if (self != kNone) return lab[self];
+  if (nv == 0) return lab[0];
+  // Labels only now: their loads wait once, not per neighbour.
+  for (int a = 0; a < nv; ++a) votes[a * 64] = lab[votes[a * 64]];
+  int best = 0, best_count = 0;
+  for (int a = 0; a < nv; ++a) {
+    const int va = votes[a * 64];
+    int cnt = 0;
+    for (int b = 0; b < nv; ++b) cnt += votes[b * 64] == va ? 1 : 0;
+    if (cnt > best_count || (cnt == best_count && va < best)) {
+      best = va;
+      best_count = cnt;
+    }
+  }
+  return best;
+}
+
 // blockIdx.x: 64 rows, sixteen per wave; blockIdx.y: 64 runs, one per lane.
 template <class T>
 __global__ void __launch_bounds__(kBlock) project_kernel(ProjectParams prm) {
-  constexpr T kNone = static_cast<T>(-1);
   __shared__ int s_out[64][65];               // [run][row]
   extern __shared__ int votes_lds[];          // [4 waves][votes][64 lanes]
   // The wave is uniform: its graph rows come through scalar loads.
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6), lane = threadIdx.x & 63;
   const int r = static_cast<int>(blockIdx.y) * 64 + lane;
   const bool mine = r < prm.runs;
-  const int begin = mine ? prm.run_offsets[r] : 0;
-  const int* lab = prm.clbest + begin;
+  const int* lab = prm.clbest + (mine ? prm.run_offsets[r] : 0);
   const T* local = static_cast<const T*>(prm.local) + static_cast<size_t>(blockIdx.y) * 64 + lane;
   int* votes = votes_lds + wave * prm.votes * 64 + lane;
   for (int q = 0; q < 16; ++q) {
     const int i = static_cast<int>(blockIdx.x) * 64 + wave * 16 + q;
     if (i >= prm.n) break;
-    const T self = local[static_cast<size_t>(i) * prm.run_stride];
-    int nv = 0;
-    bool open = mine && self == kNone;  // still collects votes
     const int* row = prm.graph + static_cast<size_t>(i) * prm.neighbors;
-    for (int j0 = 0; j0 < prm.neighbors && __ballot(open) != 0ull; j0 += 8) {
-      // Eight neighbours' table rows in flight.
-      T pos[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int g = j0 + u < prm.neighbors ? row[j0 + u] : -1;
-        pos[u] = g >= 0 && g < prm.n ? local[static_cast<size_t>(g) * prm.run_stride] : kNone;
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        if (open && pos[u] != kNone) {
-          votes[nv * 64] = static_cast<int>(pos[u]);
-          open = ++nv < prm.votes;
-        }
-      }
-    }
-    int out = 0;
-    if (mine) {
-      if (self != kNone) {
-        out = lab[self];
-      } else if (nv == 0) {
-        out = lab[0];
-      } else {
-        // Labels only now: their loads wait once, not per neighbour.
-        for (int a = 0; a < nv; ++a) votes[a * 64] = lab[votes[a * 64]];
-        int best = 0, best_count = 0;
-        for (int a = 0; a < nv; ++a) {
-          const int va = votes[a * 64];
-          int cnt = 0;
-          for (int b = 0; b < nv; ++b) cnt += votes[b * 64] == va ? 1 : 0;
-          if (cnt > best_count || (cnt == best_count && va < best)) {
-            best = va;
-            best_count = cnt;
-          }
-        }
-        out = best;
-      }
-    }
-    s_out[lane][wave * 16 + q] = out;
+    s_out[lane][wave * 16 + q] = project_row<T>(prm, row, local, i, lab, mine, votes);
   }
   __syncthreads();
   const int i = static_cast<int>(blockIdx.x) * 64 + lane;
@@ -474,6 +480,24 @@ __global__ void __launch_bounds__(kBlock) project_kernel(ProjectParams prm) {
     const int run = static_cast<int>(blockIdx.y) * 64 + u;
     if (run < prm.runs && i < prm.n) prm.res[static_cast<size_t>(run) * prm.n + i] = s_out[u][lane];
   }
+}
+
+// Up to 32 runs: run_stride (a power of two) lanes per row, 64 / run_stride
+// rows a wave.
+template <class T>
+__global__ void __launch_bounds__(kBlock) project_few_kernel(ProjectParams prm) {
+  extern __shared__ int votes_lds[];          // [4 waves][votes][64 lanes]
+  const size_t t = static_cast<size_t>(blockIdx.x) * kBlock + threadIdx.x;
+  const size_t at = t / static_cast<unsigned>(prm.run_stride);
+  const int r = static_cast<int>(t & static_cast<unsigned>(prm.run_stride - 1));
+  const bool mine = at < static_cast<size_t>(prm.n) && r < prm.runs;
+  const int i = mine ? static_cast<int>(at) : 0;
+  const int* lab = prm.clbest + (mine ? prm.run_offsets[r] : 0);
+  const T* local = static_cast<const T*>(prm.local) + (mine ? r : 0);
+  int* votes = votes_lds + (threadIdx.x >> 6) * prm.votes * 64 + (threadIdx.x & 63);
+  const int out =
+      project_row<T>(prm, prm.graph + static_cast<size_t>(i) * prm.neighbors, local, i, lab, mine, votes);
+  if (mine) prm.res[static_cast<size_t>(r) * prm.n + i] = out;
 }
 
 // ---- launchers --------------------------------------------------------------
@@ -533,22 +557,33 @@ hipError_t launch_kmeans_update(const float* x, int n, int p, const int* assign,
 
 template <class T>
 static hipError_t launch_project_t(const ProjectParams& prm, hipStream_t s) {
+  const bool few = prm.run_stride < 64;
   const size_t votes = 4 * 64 * sizeof(int) * static_cast<size_t>(prm.votes);
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&project_kernel<T>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(votes));
+  const hipError_t e = hipFuncSetAttribute(
+      few ? reinterpret_cast<const void*>(&project_few_kernel<T>) : reinterpret_cast<const void*>(&project_kernel<T>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(votes));
   if (e != hipSuccess) return e;
-  const size_t words = static_cast<size_t>(prm.n) * prm.run_stride * sizeof(T) / sizeof(uint32_t);
+  const size_t words = project_local_bytes(prm.n, prm.runs, prm.max_landmarks) / sizeof(uint32_t);
   const size_t fill_blocks = std::min<size_t>((words + kBlock - 1) / kBlock, 8192);
   hipLaunchKernelGGL(local_fill_kernel, dim3(static_cast<unsigned>(fill_blocks)), dim3(kBlock), 0, s,
                      static_cast<uint32_t*>(prm.local), words);
   hipLaunchKernelGGL((local_scatter_kernel<T>), dim3((prm.max_landmarks + kBlock - 1) / kBlock, prm.runs),
                      dim3(kBlock), 0, s, prm);
-  hipLaunchKernelGGL((project_kernel<T>), dim3((prm.n + 63) / 64, (prm.runs + 63) / 64), dim3(kBlock), votes, s, prm);
+  if (few) {
+    const size_t threads = static_cast<size_t>(prm.n) * prm.run_stride;
+    hipLaunchKernelGGL((project_few_kernel<T>), dim3(static_cast<unsigned>((threads + kBlock - 1) / kBlock)),
+                       dim3(kBlock), votes, s, prm);
+  } else {
+    hipLaunchKernelGGL((project_kernel<T>), dim3((prm.n + 63) / 64, (prm.runs + 63) / 64), dim3(kBlock), votes, s, prm);
+  }
   return hipGetLastError();
 }
 
+// Whole words.
 size_t project_local_bytes(int n, int runs, int max_landmarks) {
-  return static_cast<size_t>(n) * project_run_stride(runs) * (max_landmarks <= kProjectNarrow ? 2 : 4);
+  const size_t bytes =
+      static_cast<size_t>(n) * project_run_stride(runs) * (max_landmarks <= kProjectNarrow ? 2 : 4);
+  return (bytes + 3) / 4 * 4;
 }
 
 hipError_t launch_project(const ProjectParams& prm, hipStream_t s) {

@@ -48,9 +48,14 @@ hipError_t launch_kmeans_update(const float* x, int n, int p, const int* assign,
                                 float* centroids, float* sizes, hipStream_t s, int runs = 1,
                                 const int* active = nullptr);
 
-// Runs per row of the projection's table (whole 64-lane groups) and the most
-// landmarks whose positions fit 16 bits.
-inline int project_run_stride(int runs) { return (runs + 63) / 64 * 64; }
+// Entries per row of the projection's table: a power of two up to 32 runs, whole
+// 64-lane groups beyond. And the most landmarks whose positions fit 16 bits.
+inline int project_run_stride(int runs) {
+  if (runs > 32) return (runs + 63) / 64 * 64;
+  int stride = 1;
+  while (stride < runs) stride *= 2;
+  return stride;
+}
 constexpr int kProjectNarrow = 65535;
 size_t project_local_bytes(int n, int runs, int max_landmarks);
 

@@ -70,8 +70,10 @@ def test_scales_outside_the_scores(oracle, scale):
     _check(oracle, (x * np.float32(scale)).astype(np.float32), landmarks=200, splitting=30)
 
 
-# One lane per run in groups of 64; votes at both ends.
-@pytest.mark.parametrize("runs,k", [(1, 1), (63, 64), (64, 30), (65, 5), (130, 20)])
+# 1 to 32 lanes a row, then one lane per run in groups of 64; votes at both ends;
+# an odd number of rows (16-bit entries in whole words).
+@pytest.mark.parametrize("runs,k", [(1, 1), (1, 64), (2, 30), (3, 7), (5, 64), (16, 9), (17, 30), (32, 64), (33, 12),
+                                    (63, 64), (64, 30), (65, 5), (130, 20)])
 def test_projection_runs_and_votes(oracle, runs, k):
-    x, _ = D.gaussian_mixture(500, 6, 4, seed=runs)
+    x, _ = D.gaussian_mixture(501, 6, 4, seed=runs)
     _check(oracle, x, runs=runs, cycles=1, landmarks=150, splitting=10, k=k, graph_neighbors=100)
