@@ -5,9 +5,12 @@
 // (kodama_matrix.cpp:91-124): 16 running partials over blocks of 16 dimensions
 // (each product rounded, then added), the lane sums (s[l] + s[4+l]) +
 // (s[8+l] + s[12+l]), then ((l0 + l1) + l2) + l3, then the remaining
-// dimensions one product at a time. The kernels spell every operation with
-// __fmul_rn / __fadd_rn so nothing is contracted into an FMA, and the
-// assignments, centroid sums and norms come out bit-identical to that build.
+// dimensions one product at a time. The kernels keep that order. A product and
+// its sum round once here, though: __fmul_rn and __fadd_rn are plain operators
+// in HIP's headers, where contraction is on, and the compiler makes FMAs of
+// them. So norms and distances can differ from that build in the last bit, and
+// an assignment where two distances are that close; the centroid sums have no
+// products and are bit-identical.
 //
 // kmeans_assign_kernel: the nearest centroid is the largest score q.c - |c|^2 /
 // 2 up to the bound of score_device.h, so FP16 matrix-core scores pick the
